@@ -1697,6 +1697,53 @@ __global__ void k_vtab(cpx<float> *VN, const cpx<double> *W, int N, int R) {
 // Then every thread accumulates its own output points (k/256 of the 2112)
 // over the round's four contributions, with coalesced weight reads, in FP64.
 // ---------------------------------------------------------------------------
+// Spectra of one group's Nyquist sums, one plane per half-wave: hw = 0 the
+// packed Z = s_K + i s_J, hw = 1 s_I.  Lane c ends with z[p] = spectrum(p, q = c);
+// L is the half-wave's own transpose buffer (N rows of N + 1).
+__device__ __forceinline__ void nyq_spectrum(const float *nb, cpx<float> *L, cpx<float> *z, int hw, int c) {
+    constexpr int N = 32, ROW = N + 1;
+    // lane c takes index c of the first axis and w runs over the second,
+    // so every load reads one contiguous row segment across the lanes:
+    // Z(vx = c, w) = s_K(vx, vy = w) + i s_J(vx, vz = w), or s_I(vy = c, vz = w)
+    if (hw == 0) {
+#pragma unroll
+        for (int w = 0; w < N; ++w) {
+            // non-temporal: the sums are read once (10% faster)
+            const float sk = (__builtin_nontemporal_load(nb + w * N + c) +
+                              __builtin_nontemporal_load(nb + N * N + w * N + c)) +
+                             (__builtin_nontemporal_load(nb + 2 * N * N + w * N + c) +
+                              __builtin_nontemporal_load(nb + 3 * N * N + w * N + c));
+            z[w] = {sk, __builtin_nontemporal_load(nb + 4 * N * N + w * N + c)};
+        }
+    } else {
+#pragma unroll
+        for (int w = 0; w < N; ++w) z[w] = {__builtin_nontemporal_load(nb + 5 * N * N + w * N + c), 0.f};
+    }
+    fq::LFFT<N, -1>::run(z);                       // along w: z[q]
+    plane_sync<32>();
+#pragma unroll
+    for (int q = 0; q < N; ++q) L[c * ROW + q] = z[q];
+    plane_sync<32>();
+#pragma unroll
+    for (int i = 0; i < N; ++i) z[i] = L[i * ROW + c];
+    fq::LFFT<N, -1>::run(z);                       // along the first axis
+}
+
+// B_g at point pt of the kCPer32 Nyquist points from the two spectra, rows of
+// ROW values.
+template <int ROW> __device__ __forceinline__ cpx<double> nyq_point(const cpx<float> *Z0, const cpx<float> *Z1, int pt) {
+    constexpr int N = 32, R = kHRows32;
+    if (pt < 2 * R * N) {
+        const int i2 = pt < R * N ? pt : pt - R * N;
+        const int p = i2 / N, q = i2 % N;
+        const cpx<float> z = Z0[p * ROW + q], zp = Z0[((N - p) % N) * ROW + (N - q) % N];
+        return pt < R * N ? cpx<double>{0.5 * (double(z.x) + zp.x), 0.5 * (double(z.y) - zp.y)}
+                          : cpx<double>{0.5 * (double(z.y) + zp.y), -0.5 * (double(z.x) - zp.x)};
+    }
+    const int i3 = pt - 2 * R * N;
+    return cvt<double>(Z1[(i3 / N) * ROW + i3 % N]);
+}
+
 __global__ __launch_bounds__(256) void k_nyqb(const float *__restrict__ NB, const cpx<float> *__restrict__ VN,
                                               const int *__restrict__ c_group, const int *__restrict__ t_c0,
                                               const int *__restrict__ t_cn, cpx<double> *__restrict__ C,
@@ -1715,33 +1762,8 @@ __global__ __launch_bounds__(256) void k_nyqb(const float *__restrict__ NB, cons
     for (int j = 0; j < PPT; ++j) acc[j] = {0, 0};
     for (int base = 0; base < cn; base += 4) {
         if (base + wave < cn) {                            // wave-uniform
-            const float *nb = NB + (int64_t(slot) * ngroups + c_group[c0 + base + wave]) * kNbPer32;
-            // lane c takes index c of the first axis and w runs over the second,
-            // so every load reads one contiguous row segment across the lanes:
-            // Z(vx = c, w) = s_K(vx, vy = w) + i s_J(vx, vz = w), or s_I(vy = c, vz = w)
             cpx<float> z[N];
-            if (hw == 0) {
-#pragma unroll
-                for (int w = 0; w < N; ++w) {
-                    // non-temporal: the sums are read once (10% faster)
-                    const float sk = (__builtin_nontemporal_load(nb + w * N + c) +
-                                      __builtin_nontemporal_load(nb + N * N + w * N + c)) +
-                                     (__builtin_nontemporal_load(nb + 2 * N * N + w * N + c) +
-                                      __builtin_nontemporal_load(nb + 3 * N * N + w * N + c));
-                    z[w] = {sk, __builtin_nontemporal_load(nb + 4 * N * N + w * N + c)};
-                }
-            } else {
-#pragma unroll
-                for (int w = 0; w < N; ++w) z[w] = {__builtin_nontemporal_load(nb + 5 * N * N + w * N + c), 0.f};
-            }
-            fq::LFFT<N, -1>::run(z);                       // along w: z[q]
-            plane_sync<32>();
-#pragma unroll
-            for (int q = 0; q < N; ++q) L[c * ROW + q] = z[q];
-            plane_sync<32>();
-#pragma unroll
-            for (int i = 0; i < N; ++i) z[i] = L[i * ROW + c];
-            fq::LFFT<N, -1>::run(z);                       // along the first axis: z[p] = spectrum(p, q = c)
+            nyq_spectrum(NB + (int64_t(slot) * ngroups + c_group[c0 + base + wave]) * kNbPer32, L, z, hw, c);
             plane_sync<32>();
 #pragma unroll
             for (int p = 0; p < N; ++p) L[p * ROW + c] = z[p];     // [p][q]
@@ -1754,18 +1776,7 @@ __global__ __launch_bounds__(256) void k_nyqb(const float *__restrict__ NB, cons
             for (int j = 0; j < PPT; ++j) {
                 const int pt = tid + 256 * j;
                 if (pt < NPT) {
-                    cpx<double> bv;
-                    if (pt < 2 * R * N) {
-                        const int i2 = pt < R * N ? pt : pt - R * N;
-                        const int p = i2 / N, q = i2 % N;
-                        const cpx<float> z = Z0[p * ROW + q], zp = Z0[((N - p) % N) * ROW + (N - q) % N];
-                        bv = pt < R * N ? cpx<double>{0.5 * (double(z.x) + zp.x), 0.5 * (double(z.y) - zp.y)}
-                                        : cpx<double>{0.5 * (double(z.y) + zp.y), -0.5 * (double(z.x) - zp.x)};
-                    } else {
-                        const int i3 = pt - 2 * R * N;
-                        bv = cvt<double>(Z1[(i3 / N) * ROW + i3 % N]);
-                    }
-                    fq::cmac(acc[j], cvt<double>(v[pt]), bv);
+                    fq::cmac(acc[j], cvt<double>(v[pt]), nyq_point<ROW>(Z0, Z1, pt));
                 }
             }
         }
@@ -1776,6 +1787,125 @@ __global__ __launch_bounds__(256) void k_nyqb(const float *__restrict__ NB, cons
     for (int j = 0; j < PPT; ++j) {
         const int pt = tid + 256 * j;
         if (pt < NPT) cc[pt] = acc[j];
+    }
+}
+
+// The same in two kernels for batches of few DOFs, where one workgroup per
+// (slot, target) leaves the device idle behind a serial chain of rounds
+// (271 us for one DOF): k_nyqt transforms every group's sums, one wave per
+// (slot, group), and leaves the spectra [Z, s_I][p][q] in the place of the
+// sums; k_nyqc accumulates one Nyquist point per thread over the target's
+// contributions, in k_nyqb's order, so the results are the same bits.
+__global__ __launch_bounds__(256) void k_nyqt(float *NB, int64_t nunits) {
+    constexpr int N = 32, ROW = N + 1;
+    __shared__ cpx<float> lds[4][2][N * ROW];
+    const int tid = int(threadIdx.x);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int hw = (tid / 32) & 1, c = tid % 32;
+    const int64_t unit = int64_t(blockIdx.x) * 4 + wave;
+    if (unit >= nunits) return;                            // whole waves, no workgroup barrier
+    float *nb = NB + unit * kNbPer32;
+    cpx<float> z[N];
+    nyq_spectrum(nb, lds[wave][hw], z, hw, c);
+    cpx<float> *out = reinterpret_cast<cpx<float> *>(nb) + hw * N * N;
+#pragma unroll
+    for (int p = 0; p < N; ++p) out[p * N + c] = z[p];
+}
+
+__global__ __launch_bounds__(64) void k_nyqc(const float *__restrict__ NB, const cpx<float> *__restrict__ VN,
+                                             const int *__restrict__ c_group, const int *__restrict__ t_c0,
+                                             const int *__restrict__ t_cn, cpx<double> *__restrict__ C,
+                                             int ngroups, int ntgt) {
+    constexpr int N = 32, NPT = kCPer32;
+    const int st = int(blockIdx.y), slot = st / ntgt, t = st % ntgt;
+    const int pt = int(blockIdx.x) * 64 + int(threadIdx.x);
+    if (pt >= NPT) return;
+    const int c0 = t_c0[t], cn = t_cn[t];
+    const float *nb = NB + int64_t(slot) * ngroups * kNbPer32;
+    cpx<double> acc = {0, 0};
+#pragma unroll 8
+    for (int ci = c0; ci < c0 + cn; ++ci) {
+        const cpx<float> *Z = reinterpret_cast<const cpx<float> *>(nb + int64_t(c_group[ci]) * kNbPer32);
+        fq::cmac(acc, cvt<double>(VN[int64_t(ci) * NPT + pt]), nyq_point<N>(Z, Z + N * N, pt));
+    }
+    C[int64_t(st) * NPT + pt] = acc;
+}
+
+// One volume's pencils of a row pair for lane (J, half).  v1: 16-byte column
+// pairs at the planes half + 2(jo + 2f), jo = J & 1, completed by the
+// exchange with lane ^ 2 in FQ_H_SPECTRA (as in k_accum_lds); v2: the partner
+// column -J of row -r at the planes half + 2e.  Non-temporal loads: the
+// volumes stream through once, and the weight rows X, which the workgroups of
+// one row share, keep their place in L2 (3% faster).
+__device__ __forceinline__ void h_load(const cpx<float> *vol, int r, int J, int half, bool live, cpx<float> *v1,
+                                       cpx<float> *v2) {
+    constexpr int N = 32, E = N / 2;
+    using G = Geo<N>;
+    const int jo = J & 1;
+    const cpx<float> *s1 = vol + int64_t(r) * N + (J & ~1);
+    const cpx<float> *s2 = vol + int64_t((N - r) % N) * N + (N - J) % N;
+#pragma unroll
+    for (int f = 0; f < E / 2; ++f) {
+        cpx2f w = {{0, 0}, {0, 0}};
+        if (live) {
+            const nt_f4 t4 = __builtin_nontemporal_load(
+                reinterpret_cast<const nt_f4 *>(s1 + int64_t(half + 2 * (jo + 2 * f)) * G::N2));
+            w = {{t4.x, t4.y}, {t4.z, t4.w}};
+        }
+        v1[2 * f] = w.a;
+        v1[2 * f + 1] = w.b;
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        cpx<float> t = {0, 0};
+        if (live) {
+            const nt_f2 t2 = __builtin_nontemporal_load(reinterpret_cast<const nt_f2 *>(s2 + int64_t(half + 2 * e) * G::N2));
+            t = {t2.x, t2.y};
+        }
+        v2[e] = t;
+    }
+}
+
+// The pencils as loaded -> s = DFT-_z(v1 + conj v2) in v1 and
+// d = DFT-_z(v1 - conj v2) in v2, at K' = half*E + e.  A macro: inlined from a
+// function, the compiler contracts a few multiply-adds of the transforms
+// another way, and the two accumulations have to give the same bits.
+#define FQ_H_SPECTRA(v1, v2, jo, half)                                                  \
+    do {                                                                                \
+        _Pragma("unroll") for (int f = 0; f < E / 2; ++f) {                             \
+            const cpx<float> a = v1[2 * f], bb = v1[2 * f + 1];                         \
+            const cpx<float> recv = fq::swap_q2(jo ? a : bb);                           \
+            v1[2 * f] = jo ? recv : a;                                                  \
+            v1[2 * f + 1] = jo ? bb : recv;                                             \
+        }                                                                               \
+        _Pragma("unroll") for (int e = 0; e < E; ++e) {                                 \
+            const cpx<float> a = v1[e], q = v2[e];                                      \
+            v1[e] = {a.x + q.x, a.y - q.y};            /* v1 + conj v2 */               \
+            v2[e] = {a.x - q.x, a.y + q.y};            /* v1 - conj v2 */               \
+        }                                                                               \
+        fq::fft2_dit<N, -1>(v1, half);                                                  \
+        fq::fft2_dit<N, -1>(v2, half);                                                  \
+    } while (0)
+
+// Transforms a row's gain and loss spectra back along z and writes
+// Y = DFT+_z(H) + i DFT+_z(Hl) on row r and its conjugate form on row -r.
+__device__ __forceinline__ void h_store(cpx<double> *H, cpx<double> *Hl, cpx<double> *y, int r, int J, int half) {
+    constexpr int N = 32, E = N / 2;
+    using G = Geo<N>;
+    const int I2 = (N - r) % N;
+    const int64_t off1 = int64_t(r) * N + J, off2 = int64_t(I2) * N + (N - J) % N;
+    fq::fft2_dif<N, 1>(H, half);                      // -> vz = half + 2e
+    fq::fft2_dif<N, 1>(Hl, half);
+    // non-temporal stores, as the volume loads (8% faster accumulation)
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+        __builtin_nontemporal_store(nt_d2{H[e].x - Hl[e].y, H[e].y + Hl[e].x},
+                                    reinterpret_cast<nt_d2 *>(y + int64_t(half + 2 * e) * G::N2 + off1));
+    if (I2 != r) {
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            __builtin_nontemporal_store(nt_d2{H[e].x + Hl[e].y, Hl[e].x - H[e].y},
+                                        reinterpret_cast<nt_d2 *>(y + int64_t(half + 2 * e) * G::N2 + off2));
     }
 }
 
@@ -1826,35 +1956,8 @@ __global__ __launch_bounds__(64 * NS, 8 / NS) void k_accum_h(
     cpx<double> wp[CP];
     const cpx<double> *xr = X + int64_t(r) * WR;
     const cpx<float> *pslot = P + int64_t(live ? slot : 0) * nvol * G::VOL;
-    // v1: 16-byte column pairs at the planes half + 2(jo + 2f), completed by
-    // the exchange with lane ^ 2 below (as in k_accum_lds); v2: the partner
-    // column -J of row -r at the planes half + 2e.  Non-temporal loads: the
-    // volumes stream through once, and the weight rows X, which the
-    // workgroups of one row share, keep their place in L2 (3% faster)
     auto load = [&](int ei, cpx<float> *v1, cpx<float> *v2) {
-        const cpx<float> *vol = pslot + int64_t(e_vol[ei]) * G::VOL;
-        const cpx<float> *s1 = vol + int64_t(I1) * N + (J & ~1);
-        const cpx<float> *s2 = vol + int64_t(I2) * N + Jp;
-#pragma unroll
-        for (int f = 0; f < E / 2; ++f) {
-            cpx2f w = {{0, 0}, {0, 0}};
-            if (live) {
-                const nt_f4 t4 = __builtin_nontemporal_load(
-                    reinterpret_cast<const nt_f4 *>(s1 + int64_t(half + 2 * (jo + 2 * f)) * G::N2));
-                w = {{t4.x, t4.y}, {t4.z, t4.w}};
-            }
-            v1[2 * f] = w.a;
-            v1[2 * f + 1] = w.b;
-        }
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            cpx<float> t = {0, 0};
-            if (live) {
-                const nt_f2 t2 = __builtin_nontemporal_load(reinterpret_cast<const nt_f2 *>(s2 + int64_t(half + 2 * e) * G::N2));
-                t = {t2.x, t2.y};
-            }
-            v2[e] = t;
-        }
+        h_load(pslot + int64_t(e_vol[ei]) * G::VOL, r, J, half, live, v1, v2);
     };
     cpx<double> H[E];
 #pragma unroll
@@ -1887,21 +1990,7 @@ __global__ __launch_bounds__(64 * NS, 8 / NS) void k_accum_h(
         for (int e = 0; e < E; ++e) { v1[e] = n1[e]; v2[e] = n2[e]; }
         if (ei + 1 < e0 + en) load(ei + 1, n1, n2);
         if (live) {
-#pragma unroll
-            for (int f = 0; f < E / 2; ++f) {
-                const cpx<float> a = v1[2 * f], bb = v1[2 * f + 1];
-                const cpx<float> recv = fq::swap_q2(jo ? a : bb);
-                v1[2 * f] = jo ? recv : a;
-                v1[2 * f + 1] = jo ? bb : recv;
-            }
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const cpx<float> a = v1[e], q = v2[e];
-                v1[e] = {a.x + q.x, a.y - q.y};            // v1 + conj v2
-                v2[e] = {a.x - q.x, a.y + q.y};            // v1 - conj v2
-            }
-            fq::fft2_dit<N, -1>(v1, half);                 // -> K' = half*E + e
-            fq::fft2_dit<N, -1>(v2, half);
+            FQ_H_SPECTRA(v1, v2, jo, half);
             const cpx<double> *w0 = wl[buf];
 #pragma unroll
             for (int e = 0; e < E; ++e) {
@@ -1942,20 +2031,114 @@ __global__ __launch_bounds__(64 * NS, 8 / NS) void k_accum_h(
             Hl[e] = {Hl[e].x + 0.5 * (a.x + m.x), Hl[e].y + 0.5 * (a.y - m.y)};
         }
     }
-    fq::fft2_dif<N, 1>(H, half);                      // -> vz = half + 2e
-    fq::fft2_dif<N, 1>(Hl, half);
-    // non-temporal stores, as the volume loads (8% faster accumulation)
-    cpx<double> *y = Y + (int64_t(slot) * ntgt + t) * G::VOL;
+    h_store(H, Hl, Y + (int64_t(slot) * ntgt + t) * G::VOL, r, J, half);
+}
+
+// ---------------------------------------------------------------------------
+// The same accumulation in two kernels for batches of few DOFs: k_accum_h
+// then leaves most of the device idle behind its serial chain over the
+// volumes (17 row pairs of one wave per DOF, 158 us for one DOF).  k_hz
+// transforms every volume's row pairs, one wave each, into
+// SD[slot][u][r][m][K'][J'] (m = 0: s, m = 1: d); k_hsum gives every grid
+// point of a row pair its own thread, accumulates over the volumes in
+// k_accum_h's order (the same bits) and finishes the row as k_accum_h does.
+// ---------------------------------------------------------------------------
+constexpr int kSDPer32 = kHRows32 * 2 * 32 * 32;             // SD values per (slot, volume)
+
+__global__ __launch_bounds__(256) void k_hz(const cpx<float> *__restrict__ P, cpx<float> *__restrict__ SD,
+                                            int64_t nunits) {
+    constexpr int N = 32, R = kHRows32;
+    using G = Geo<N>;
+    constexpr int E = G::E;
+    const int lt = threadIdx.x % 64, J = lt >> 1, half = lt & 1;
+    // unit = (slot * nvol + u) * R + r; grid-stride over waves with the next
+    // unit's pencils in flight
+    const int64_t step = int64_t(gridDim.x) * 4;
+    int64_t unit = int64_t(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(int(threadIdx.x) / 64);
+    cpx<float> n1[E], n2[E];
+    if (unit < nunits) h_load(P + unit / R * G::VOL, int(unit % R), J, half, true, n1, n2);
+    for (; unit < nunits; unit += step) {
+        cpx<float> v1[E], v2[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e)
-        __builtin_nontemporal_store(nt_d2{H[e].x - Hl[e].y, H[e].y + Hl[e].x},
-                                    reinterpret_cast<nt_d2 *>(y + int64_t(half + 2 * e) * G::N2 + off1));
-    if (I2 != I1) {
+        for (int e = 0; e < E; ++e) { v1[e] = n1[e]; v2[e] = n2[e]; }
+        const int64_t nx = unit + step;
+        if (nx < nunits) h_load(P + nx / R * G::VOL, int(nx % R), J, half, true, n1, n2);
+        const int jo = J & 1;
+        FQ_H_SPECTRA(v1, v2, jo, half);
+        cpx<float> *out = SD + unit * (2 * N * N) + J;
 #pragma unroll
-        for (int e = 0; e < E; ++e)
-            __builtin_nontemporal_store(nt_d2{H[e].x + Hl[e].y, Hl[e].x - H[e].y},
-                                        reinterpret_cast<nt_d2 *>(y + int64_t(half + 2 * e) * G::N2 + off2));
+        for (int e = 0; e < E; ++e) {
+            out[(half * E + e) * N] = v1[e];
+            out[N * N + (half * E + e) * N] = v2[e];
+        }
     }
+}
+
+// Block b serves row r = b % 8 + 8 (b / 8 / pairs) of pair (slot, target)
+// (b / 8) % pairs: workgroups are dealt round-robin to the eight XCDs, so one
+// XCD's L2 holds the weights of two or three rows (1.6 MB each at 48 volumes)
+// for all the pairs, instead of every XCD streaming all 17.
+__global__ __launch_bounds__(1024) void k_hsum(
+    const cpx<float> *__restrict__ SD, const cpx<double> *__restrict__ F, const cpx<double> *__restrict__ X,
+    const int *__restrict__ e_vol, const int *__restrict__ t_e0, const int *__restrict__ t_en,
+    const cpx<double> *__restrict__ C, const cpx<double> *__restrict__ W, const int *__restrict__ l_src,
+    const int *__restrict__ t_l0, const int *__restrict__ t_ln, int ncontribs, cpx<double> *__restrict__ Y,
+    int nvol, int nsrc, int ntgt, int pairs) {
+    constexpr int N = 32, R = kHRows32, ROW = N + 1;
+    using G = Geo<N>;
+    constexpr int E = G::E;
+    __shared__ cpx<double> sp[2][N * ROW];                       // H and Hl spectra, then their z transforms
+    const int b = int(blockIdx.x);
+    const int r = b % 8 + 8 * (b / 8 / pairs), st = (b / 8) % pairs;
+    if (r >= R) return;                                          // the whole workgroup
+    const int t = st % ntgt, slot = st / ntgt;
+    const int idx = int(threadIdx.x), K = idx / N, J = idx % N;
+    const int e0 = t_e0[t], en = t_en[t];
+    const int I1 = r, I2 = (N - r) % N, Km = (N - K) % N, Jm = (N - J) % N;
+    const cpx<float> *sd = SD + (int64_t(slot) * nvol * R + r) * (2 * N * N) + idx;
+    const cpx<double> *x = X + int64_t(r) * (2 * N * N) + idx;
+    cpx<double> H = {0, 0};
+#pragma unroll 6
+    for (int ei = e0; ei < e0 + en; ++ei) {
+        const cpx<float> *q = sd + int64_t(e_vol[ei]) * kSDPer32;
+        const cpx<double> *w = x + int64_t(ei) * R * (2 * N * N);
+        fq::cmac(H, w[0], cvt<double>(q[0]));
+        fq::cmac(H, w[N * N], cvt<double>(q[N * N]));
+    }
+    if (C) {
+        const cpx<double> *cc = C + int64_t(st) * kCPer32;
+        if (K == N / 2) H = H + cc[r * N + J];
+        if (J == N / 2) H = H + cc[R * N + r * N + K];
+        if (r == N / 2) H = H + cc[2 * R * N + J * N + K];
+    }
+    cpx<double> Hl = {0, 0};
+    const int l0 = t_l0[t], ln = t_ln[t];
+    const int64_t p1 = int64_t(K) * G::N2 + I1 * N + J, p2 = int64_t(Km) * G::N2 + I2 * N + Jm;
+    for (int li = l0; li < l0 + ln; ++li) {
+        const cpx<double> *fs = F + (int64_t(slot) * nsrc + l_src[li]) * G::VOL;
+        const cpx<double> *w = W + int64_t(ncontribs + li) * G::VOL;
+        const cpx<double> a = fq::cmul(w[p1], fs[p1]);
+        const cpx<double> m = fq::cmul(w[p2], fs[p2]);
+        Hl = {Hl.x + 0.5 * (a.x + m.x), Hl.y + 0.5 * (a.y - m.y)};
+    }
+    sp[0][K * ROW + J] = H;
+    sp[1][K * ROW + J] = Hl;
+    __syncthreads();
+    if (idx < 128) {                                             // one wave per spectrum
+        cpx<double> *L = sp[idx / 64];
+        const int c = (idx % 64) >> 1, half = idx & 1;
+        cpx<double> v[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = L[(half * E + e) * ROW + c];
+        fq::fft2_dif<N, 1>(v, half);                             // -> vz = half + 2e
+#pragma unroll
+        for (int e = 0; e < E; ++e) L[(half + 2 * e) * ROW + c] = v[e];
+    }
+    __syncthreads();
+    const cpx<double> h = sp[0][K * ROW + J], l = sp[1][K * ROW + J];      // plane vz = K
+    cpx<double> *y = Y + int64_t(st) * G::VOL + int64_t(K) * G::N2;
+    y[I1 * N + J] = {h.x - l.y, h.y + l.x};
+    if (I2 != I1) y[I2 * N + Jm] = {h.x + l.y, l.x - h.y};
 }
 
 // ---------------------------------------------------------------------------
@@ -2205,60 +2388,75 @@ __global__ __launch_bounds__(256) void k_project(AosoaPtrs ptr, Dof dof, int ns,
 
 // The same projection with the moments of Q taken from the per-plane sums
 // that k_out1 wrote (mom[slot][s][vz][5]), so Q is read once and written once,
-// over blocks of 32 consecutive batch slots and chunks of kProjChunk grid
-// points: lane e of each 32-lane group takes slot s0 + e, so with one solution
+// over blocks of 32 consecutive batch slots and chunks of grid points:
+// lane e of each 32-lane group takes slot s0 + e, so with one solution
 // point per element and 32-aligned DOFs the group's accesses are one
 // contiguous AoSoA row segment (32 elements x 8 bytes) per grid point.
-constexpr int kProjChunk = 1024;
-
+// The points per workgroup, `chunk` (a multiple of 64), shrink for small
+// batches so that the grid still fills the device (launch rule in run_chunk).
+// Latency bound at few DOFs: one DOF took 115 us with 1024 points per
+// workgroup, the plane sums added by 32 threads and one load in flight, and
+// takes 10 us with 64 points, 256 threads and eight.
 __global__ __launch_bounds__(256) void k_project_b(AosoaPtrs ptr, Dof dof, int ns, int N, double L,
-                                                   const double *ginv, const double *mass, const double *mom, int D) {
+                                                   const double *ginv, const double *mass, const double *mom, int D,
+                                                   int chunk) {
     const int64_t n = int64_t(N) * N * N;
-    const int nchunk = int(n / kProjChunk);
+    const int nchunk = int(n / chunk);
     const int blk = int(blockIdx.x) / nchunk, ch = int(blockIdx.x) % nchunk;
     const int s0 = 32 * blk;
     const int K = ns + 4;
-    __shared__ double lam_s[32][kProjMaxRows];
+    __shared__ double part[8][32][5];
+    __shared__ double aq_s[32][kProjMaxRows];
     const int tid = int(threadIdx.x);
-    if (tid < 32) {
-        const int slot = s0 + tid;
-        double aq[kProjMaxRows];
-#pragma unroll
-        for (int i = 0; i < kProjMaxRows; ++i) aq[i] = 0;
-        if (slot < D) {
-            for (int s = 0; s < ns; ++s) {
-                double m[5] = {0, 0, 0, 0, 0};
-                const double *ms = mom + (int64_t(slot) * ns + s) * N * 5;
-                for (int z = 0; z < N; ++z) {
-#pragma unroll
-                    for (int k = 0; k < 5; ++k) m[k] += ms[z * 5 + k];
-                }
-                aq[s] = m[0];
-                for (int k = 1; k < 5; ++k) aq[ns + k - 1] += mass[s] * m[k];
-            }
-        }
-        for (int i = 0; i < K; ++i) {
-            double acc = 0;
-            for (int k = 0; k < K; ++k) acc += ginv[i * K + k] * aq[k];
-            lam_s[tid][i] = acc;
-        }
-    }
-    __syncthreads();
     const int e = tid % 32, vg = tid / 32;
     const int slot = s0 + e;
-    if (slot >= D) return;                        // no barrier follows
-    const int64_t b = dof.base(slot);
-    const double *lam = lam_s[e];
+    // the block's constraint sums: thread (slot e, vg) adds the planes z = vg,
+    // vg + 8, ... of each species, then thread (e, row) the eight partial sums
     for (int s = 0; s < ns; ++s) {
-        double *q = ptr.q[s];
+        double m[5] = {0, 0, 0, 0, 0};
+        if (slot < D) {
+            const double *ms = mom + (int64_t(slot) * ns + s) * N * 5;
+            for (int z = vg; z < N; z += 8) {
+#pragma unroll
+                for (int k = 0; k < 5; ++k) m[k] += ms[z * 5 + k];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 5; ++k) part[vg][e][k] = m[k];
+        __syncthreads();
+        if (vg < 5) {
+            double x = 0;
+#pragma unroll
+            for (int g = 0; g < 8; ++g) x += part[g][e][vg];
+            if (vg == 0) aq_s[e][s] = x;
+            else aq_s[e][ns + vg - 1] = mass[s] * x + (s > 0 ? aq_s[e][ns + vg - 1] : 0.0);
+        }
+        __syncthreads();
+    }
+    if (slot >= D) return;                        // no barrier follows
+    double lam[kProjMaxRows];
+    for (int i = 0; i < K; ++i) {
+        double acc = 0;
+        for (int k = 0; k < K; ++k) acc += ginv[i * K + k] * aq_s[e][k];
+        lam[i] = acc;
+    }
+    const int64_t b = dof.base(slot);
+    const int64_t v0 = int64_t(ch) * chunk + vg;
+    for (int s = 0; s < ns; ++s) {
+        double *q = ptr.q[s] + b;
         const double ms = mass[s];
-        for (int i = vg; i < kProjChunk; i += 8) {
-            const int64_t v = int64_t(ch) * kProjChunk + i;
-            double ph[5];
-            phis(v, N, L, ph);
-            const double corr = lam[s] + ms * (lam[ns] * ph[1] + lam[ns + 1] * ph[2] + lam[ns + 2] * ph[3] +
-                                               lam[ns + 3] * ph[4]);
-            q[b + v * dof.soasz] -= corr;
+        for (int i = 0; i < chunk; i += 64) {
+            double qv[8];                         // eight loads in flight before the first store
+#pragma unroll
+            for (int j = 0; j < 8; ++j) qv[j] = q[(v0 + i + 8 * j) * dof.soasz];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                double ph[5];
+                phis(v0 + i + 8 * j, N, L, ph);
+                const double corr = lam[s] + ms * (lam[ns] * ph[1] + lam[ns + 1] * ph[2] + lam[ns + 2] * ph[3] +
+                                                   lam[ns + 3] * ph[4]);
+                q[(v0 + i + 8 * j) * dof.soasz] = qv[j] - corr;
+            }
         }
     }
 }
@@ -2406,6 +2604,7 @@ struct Scratch {
     float *NB = nullptr;          // group pairs: Nyquist sums of Im G_g (k_prod1 -> k_nyqb)
     cpx<double> *C = nullptr;     // group pairs: Nyquist corrections (k_nyqb -> k_accum_h)
     double *MOM = nullptr;        // group pairs with projection: per-plane sums of Q (k_out1 -> k_project_b)
+    int64_t cap = 0;              // DOF slots the regions hold
 };
 
 struct fq_handle {
@@ -2783,6 +2982,15 @@ int build_hpair(fq_handle *h) {
     return rc;
 }
 
+// (DOF, target) pairs up to which the Nyquist sums and the accumulation of the
+// group-pair path run as two kernels each (k_nyqt + k_nyqc, k_hz + k_hsum; the
+// same bits either way).  k_nyqb takes one workgroup per pair and the same
+// 255 us (M = 12, Nrho = 16) until they pass one per CU; the two kernels take
+// 56 us at one pair, 148 us at 128, and more than k_nyqb beyond 256.  k_accum_h
+// takes 160-211 us up to 60 pairs; k_hz + k_hsum 41 us at one, 74 us at 8,
+// 168 us at 16 and 252 us at 24 (their spectra then pass through HBM).
+constexpr int64_t kNyqFew = 256, kSumFew = 16;
+
 template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, const AosoaPtrs &ptr, const Dof &dof,
                                            int D, bool prof, hipStream_t st) {
     using G = Geo<N>;
@@ -2874,8 +3082,15 @@ template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, cons
                 post(7);
                 if (h->hpair && h->hp_nyq) {
                     pre();
-                    hipLaunchKernelGGL(k_nyqb, dim3(unsigned(int64_t(D) * ntgt)), dim3(256), 0, st, sc.NB, h->VN,
-                                       h->c_group, h->t_c0, h->t_cn, sc.C, ngroups, ntgt);
+                    if (int64_t(D) * ntgt <= kNyqFew) {
+                        const int64_t nu = int64_t(D) * ngroups;
+                        hipLaunchKernelGGL(k_nyqt, dim3(unsigned((nu + 3) / 4)), dim3(256), 0, st, sc.NB, nu);
+                        hipLaunchKernelGGL(k_nyqc, dim3(kCPer32 / 64, unsigned(int64_t(D) * ntgt)), dim3(64), 0, st,
+                                           sc.NB, h->VN, h->c_group, h->t_c0, h->t_cn, sc.C, ngroups, ntgt);
+                    } else {
+                        hipLaunchKernelGGL(k_nyqb, dim3(unsigned(int64_t(D) * ntgt)), dim3(256), 0, st, sc.NB, h->VN,
+                                           h->c_group, h->t_c0, h->t_cn, sc.C, ngroups, ntgt);
+                    }
                     post(9);
                 }
             }
@@ -2928,15 +3143,29 @@ template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, cons
     pre();
     if (h->hpair) {
         if constexpr (N == 32 && sizeof(T) == 4) {
-            // group pairs: rows r = 0..N/2, eight (or with FQ_FLAG_ACCUM_QUAD four)
-            // DOF slots per workgroup
-            const bool eight = !(h->flags & FQ_FLAG_ACCUM_QUAD);
-            auto kacc = eight ? k_accum_h<8> : k_accum_h<4>;
-            const int NS = eight ? 8 : 4;
-            hipLaunchKernelGGL(kacc, dim3(unsigned(int64_t((D + NS - 1) / NS) * ntgt * kHRows32)), dim3(64 * NS), 0,
-                               st, reinterpret_cast<const cpx<float> *>(sc.Pg), sc.F, h->X, h->e_vol, h->t_e0,
-                               h->t_en, h->hp_nyq ? sc.C : nullptr, h->W, h->l_src, h->t_l0, h->t_ln,
-                               int(P.contribs.size()), Y, h->nvol, nsrc, ntgt, D);
+            const cpx<float> *Pf = reinterpret_cast<const cpx<float> *>(sc.Pg);
+            const cpx<double> *Cn = h->hp_nyq ? sc.C : nullptr;
+            // few DOFs: two kernels, the row spectra in the unused slots of Pg
+            const int64_t nv = int64_t(D) * h->nvol;
+            if (int64_t(D) * ntgt <= kSumFew && nv * (G::VOL + kSDPer32) <= sc.cap * h->nvol * G::VOL) {
+                cpx<float> *SD = reinterpret_cast<cpx<float> *>(sc.Pg) + nv * G::VOL;
+                const int pairs = D * ntgt;
+                hipLaunchKernelGGL(k_hz, dim3(unsigned(std::min<int64_t>((nv * kHRows32 + 3) / 4, 8 * h->cus))),
+                                   dim3(256), 0, st, Pf, SD, nv * kHRows32);
+                hipLaunchKernelGGL(k_hsum, dim3(unsigned(8 * ((kHRows32 + 7) / 8) * pairs)), dim3(1024), 0, st, SD,
+                                   sc.F, h->X, h->e_vol, h->t_e0, h->t_en, Cn, h->W, h->l_src, h->t_l0, h->t_ln,
+                                   int(P.contribs.size()), Y, h->nvol, nsrc, ntgt, pairs);
+            } else {
+                // rows r = 0..N/2, eight (or with FQ_FLAG_ACCUM_QUAD four) DOF slots per
+                // workgroup; four as well while that leaves no CU a second workgroup
+                const bool eight = !(h->flags & FQ_FLAG_ACCUM_QUAD) &&
+                                   int64_t((D + 3) / 4) * ntgt * kHRows32 > h->cus;
+                auto kacc = eight ? k_accum_h<8> : k_accum_h<4>;
+                const int NS = eight ? 8 : 4;
+                hipLaunchKernelGGL(kacc, dim3(unsigned(int64_t((D + NS - 1) / NS) * ntgt * kHRows32)), dim3(64 * NS),
+                                   0, st, Pf, sc.F, h->X, h->e_vol, h->t_e0, h->t_en, Cn, h->W, h->l_src, h->t_l0,
+                                   h->t_ln, int(P.contribs.size()), Y, h->nvol, nsrc, ntgt, D);
+            }
         }
     } else if constexpr (N == 32) {
         // FP32 pencils: eight DOF slots per workgroup (one per CU) unless
@@ -2972,8 +3201,13 @@ template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, cons
         // per batch, right after k_out: the batch's Q is still in L2
         pre();
         if (h->hpair)
-            hipLaunchKernelGGL(k_project_b, dim3(unsigned((D + 31) / 32 * (int64_t(N) * N * N / kProjChunk))),
-                               dim3(256), 0, st, ptr, dof, ntgt, N, P.L, h->ginv, h->pmass, sc.MOM, int(D));
+{
+            // 1024 points per workgroup, fewer until there are four workgroups per CU
+            int pc = 1024;
+            while (pc > 64 && (D + 31) / 32 * (G::VOL / pc) < 4 * h->cus) pc /= 2;
+            hipLaunchKernelGGL(k_project_b, dim3(unsigned((D + 31) / 32 * (G::VOL / pc))), dim3(256), 0, st, ptr,
+                               dof, ntgt, N, P.L, h->ginv, h->pmass, sc.MOM, int(D), pc);
+        }
         else
         hipLaunchKernelGGL(k_project, dim3(unsigned(8 * ((D + 7) / 8))), dim3(256), 0, st, ptr, dof, ntgt, N, P.L,
                            h->ginv, h->pmass, int(D));
@@ -3213,6 +3447,7 @@ int eval_own(fq_handle *h, const AosoaPtrs &ptr, int32_t nupts, int64_t ldim, in
         sc[k].NB = static_cast<float *>(at(h->NB, h->per_dof_NB));
         sc[k].C = static_cast<cpx<double> *>(at(h->Cn, h->per_dof_C));
         sc[k].MOM = static_cast<double *>(at(h->MOM, h->per_dof_M));
+        sc[k].cap = h->chunk;
     }
     return eval_impl(h, sc, h->nsets, h->chunk, h->prof, ptr, nupts, ldim, neles, first_dof, ndof, stream);
 }
@@ -3265,6 +3500,7 @@ Scratch noalloc_carve(const fq_handle *h, unsigned char *base, int64_t c) {
     sc.NB = static_cast<float *>(take(h->per_dof_NB));
     sc.C = static_cast<cpx<double> *>(take(h->per_dof_C));
     sc.MOM = static_cast<double *>(take(h->per_dof_M));
+    sc.cap = c;
     return sc;
 }
 
