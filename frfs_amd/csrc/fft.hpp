@@ -107,7 +107,7 @@ template <int E, int S, int K, typename T> __device__ __forceinline__ cpx<T> twm
 
 // ---------------------------------------------------------------------------
 // In-register FFT of length E, natural order in and out.
-// Mixed radix (4, 2, 3) decimation: n = m*a + b, k = c + r*d.
+// Mixed radix (4, 2, 3, 5, 7) decimation: n = m*a + b, k = c + r*d.
 // ---------------------------------------------------------------------------
 template <int E, int S> struct LFFT;
 
@@ -150,12 +150,45 @@ template <int S> struct LFFT<4, S> {
     }
 };
 
+// Odd prime lengths 5 and 7, folded: with t_k = x_k + x_{p-k} and
+// d_k = x_k - x_{p-k}, X_m = x_0 + sum_k cos(2 pi mk/p) t_k + S i sum_k
+// sin(2 pi mk/p) d_k and X_{p-m} with the other sign of the second sum.
+template <int P, int S> struct PrimeFFT {
+    template <typename T> __device__ __forceinline__ static void run(cpx<T> *x) {
+        constexpr int H = P / 2;
+        cpx<T> t[H], d[H], y[P];
+        y[0] = x[0];
+        sfor<0, H>([&](auto kk) {
+            constexpr int k = decltype(kk)::value;
+            t[k] = x[k + 1] + x[P - 1 - k];
+            d[k] = x[k + 1] - x[P - 1 - k];
+            y[0] = y[0] + t[k];
+        });
+        sfor<1, H + 1>([&](auto mm) {
+            constexpr int m = decltype(mm)::value;
+            cpx<T> a = x[0], b = {0, 0};
+            sfor<0, H>([&](auto kk) {
+                constexpr int k = decltype(kk)::value;
+                using W = Twiddle<P, m * (k + 1)>;
+                const T c = T(W::c), s = T(S * W::s);
+                a = {fmadd(c, t[k].x, a.x), fmadd(c, t[k].y, a.y)};
+                b = {fmadd(-s, d[k].y, b.x), fmadd(s, d[k].x, b.y)};
+            });
+            y[m] = a + b;
+            y[P - m] = a - b;
+        });
+        sfor<0, P>([&](auto mm) { constexpr int m = decltype(mm)::value; x[m] = y[m]; });
+    }
+};
+template <int S> struct LFFT<5, S> : PrimeFFT<5, S> {};
+template <int S> struct LFFT<7, S> : PrimeFFT<7, S> {};
+
 template <int E> struct Radix {
     static constexpr int r = (E % 4 == 0 && E > 4) ? 4 : (E % 2 == 0 ? 2 : (E % 3 == 0 ? 3 : E));
 };
 
 template <int E, int S> struct LFFT {
-    static_assert(E % 2 == 0 || E % 3 == 0, "unsupported FFT length");
+    static_assert(E % 2 == 0 || E % 3 == 0, "unsupported FFT length");   // a length of odd primes 3, 5, 7
     template <typename T> __device__ __forceinline__ static void run(cpx<T> *x) {
         constexpr int r = Radix<E>::r;
         constexpr int m = E / r;

@@ -18,6 +18,9 @@
 //                                              L += Lt . F, DFT+ along z of H and L
 //   k_out      Y -> Q (AoSoA, per target)    : DFT+ x,y; Q = Re gain - f Re loss
 //   k_project  optional conservation projection (FP64)
+// FP64 plans with one target on grids up to 20^3 run k_cube_fwd, k_cube and
+// k_cube_out instead, batches of few DOFs of the 32^3 group-pair path k_nyqt,
+// k_nyqc, k_hz and k_hsum in the place of k_nyqb and k_accum_h.
 // T = double (FQ_PREC_FP64) or float (FQ_PREC_MIXED).
 //
 // Lane mapping: a "unit" (one plane or one row of N pencils) is LPP = 2*NP
@@ -2462,6 +2465,468 @@ __global__ __launch_bounds__(256) void k_project_b(AosoaPtrs ptr, Dof dof, int n
 }
 
 // ---------------------------------------------------------------------------
+// The cube kernels: FP64 plans with one target on the grids whose volume fits
+// one CU's LDS (even N up to 20), the whole operator in three launches.
+//   k_cube_fwd  f -> F, R_loss         per (slot, source): gather, DFT-, / n; Re DFT+(Lt . F)
+//   k_cube      F -> R (real)          per (slot, segment): see below
+//   k_cube_out  R, f -> Q              Q = sum_seg R_seg - f R_loss
+// A segment is up to kSegProds products of one group, or several groups of one
+// product each.  Its workgroup keeps one volume in LDS and one pencil per lane
+// in registers: per product the packed volume T_1 + i T_2 (k_prod1's pair
+// packing) is transformed along z, x and y with two LDS transposes, multiplied
+// out against the Nyquist corrections and summed; per group the sum is
+// transformed forward, weighted and added to H; at the end Re DFT+(H) is
+// written.  One wave computes
+// the product's three Nyquist planes (k_nyq's pieces).  Plans whose groups sum products (VHS: MG false) have
+// real even weights, so only the real part of a product reaches Q; in plans
+// of single-product groups (VSS: MG true) a workgroup takes several groups and
+// keeps H in registers between them.
+// Against the k_prod path nothing but F and one real volume per segment passes
+// through memory, z pencils are whole transforms instead of four pruned ones,
+// and products are packed on every such grid.
+// Every sum runs in an order the plan fixes, so a DOF gets the same bits in any
+// batch.  Measured against the k_prod path (16^3, M = 6, Nrho = 8): 134 -> 77 us
+// for 64 DOFs, 12.5 -> 7.1 ms for 8192 with the projection; against the library
+// path (20^3, Nrho = 10, 153 DOFs): 13.4 ms -> 420 us.  k_cube issues FP64 VALU
+// in 45% of the cycles and keeps the LDS busy in 32%; its barriers and the one
+// wave with the Nyquist planes, at two waves per SIMD (LDS, registers), are the
+// rest.
+// ---------------------------------------------------------------------------
+constexpr int kCubeMaxN = 20;
+constexpr int kSegProds = 8;
+
+struct CubeSeg { int g, p0, np; };      // products [p0, p0 + np); their group (MG: product p is group p)
+
+template <int N> struct CubeGeo {
+    static constexpr int N2 = N * N, VOL = N * N * N, ROW = N + 1, PLANE = N * ROW;
+    static constexpr int MAIN = (N2 + 63) / 64 * 64, NW = MAIN / 64;
+    // Above 16^3 (one workgroup per CU) a wave of its own computes the Nyquist
+    // planes beside the z and x stages; up to 16^3 a fifth wave would keep the
+    // second workgroup off the CU (4.6 ms against 3.1 ms per 4096 DOFs), so the
+    // main waves take them in turn (20^3: 434 us with the wave, 504 in turn)
+    static constexpr bool NYQ_WAVE = N > 16;
+    static constexpr int THREADS = MAIN + (NYQ_WAVE ? 64 : 0);
+    static_assert(3 * N <= 64, "three Nyquist pieces in one wave");
+};
+
+// rotated N x N array of the Nyquist wave (rows and columns both spread over the banks, no padding)
+template <int N> __device__ __forceinline__ int rot(int a, int c) {
+    const int x = a + c;
+    return a * N + (x >= N ? x - N : x);
+}
+
+// Forward transform of one (slot, source), and for the loss term's source
+// Re DFT+(Lt . F) as well, in the volume behind the slot's segments.
+template <int N>
+__global__ __launch_bounds__(CubeGeo<N>::MAIN) void k_cube_fwd(AosoaPtrs ptr, Dof dof, cpx<double> *__restrict__ F,
+                                                               int nsrc, const cpx<double> *__restrict__ Lt, int lsrc,
+                                                               double *__restrict__ Rv, int nseg) {
+    using C = CubeGeo<N>;
+    __shared__ cpx<double> L[N * C::PLANE];
+    const int64_t unit = (gridDim.x & 7) == 0 ? xcd_block() : int64_t(blockIdx.x);
+    const int s = int(unit % nsrc), slot = int(unit / nsrc);
+    const int tid = int(threadIdx.x);
+    const bool act = tid < C::N2;
+    const int a = act ? tid / N : 0, b = act ? tid % N : 0;
+    // pencils of the lane in L: along the plane index, along the row, along the column
+    cpx<double> *Lz = L + a * C::ROW + b, *Lx = L + a * C::PLANE + b, *Ly = L + a * C::PLANE + b * C::ROW;
+    cpx<double> v[N];
+    const double *f = ptr.f[s] + dof.base(slot);
+    // lane (vx, vy) over vz
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = {act ? f[int64_t(tid * N + k) * dof.soasz] : 0.0, 0.0};
+    fq::LFFT<N, -1>::run(v);                                   // -> K
+    if (act) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) Lz[k * C::PLANE] = v[k];
+    }
+    __syncthreads();
+    // lane (K, vy) over vx, in place
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = Lx[k * C::ROW];
+    fq::LFFT<N, -1>::run(v);                                   // -> I
+    if (act) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) Lx[k * C::ROW] = v[k];
+    }
+    __syncthreads();
+    // lane (K, I) over vy, in place
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = Ly[k];
+    fq::LFFT<N, -1>::run(v);                                   // -> J
+    if (act) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) Ly[k] = v[k];
+    }
+    __syncthreads();
+    // lane (I, J) over K
+    const double nn = double(C::VOL);
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const cpx<double> x = Lz[k * C::PLANE];
+        v[k] = {x.x / nn, x.y / nn};                           // FTf /= vsize (vhs-gll.mako:120)
+    }
+    if (act) {
+        cpx<double> *dst = F + unit * C::VOL + tid;
+#pragma unroll
+        for (int k = 0; k < N; ++k) dst[k * C::N2] = v[k];
+    }
+    if (s != lsrc) return;                                     // the whole workgroup
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = fq::cmul(Lt[k * C::N2 + a * N + b], v[k]);
+    fq::LFFT<N, 1>::run(v);                                    // -> vz, into the lane's own column
+    if (act) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) Lz[k * C::PLANE] = v[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = Lx[k * C::ROW];
+    fq::LFFT<N, 1>::run(v);                                    // lane (vz, J): I -> vx
+    if (act) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) Lx[k * C::ROW] = v[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = Ly[k];
+    fq::LFFT<N, 1>::run(v);                                    // lane (vz, vx): J -> vy
+    if (act) {
+        double *r = Rv + (int64_t(slot) * (nseg + 1) + nseg) * C::VOL + tid;
+#pragma unroll
+        for (int k = 0; k < N; ++k) r[k * C::N2] = v[k].x;
+    }
+}
+
+// The Nyquist planes X_K, X_J, X_I of one product (see k_prod1 and k_nyq) on
+// lanes c of the three pieces, into ny[piece * N2 + .]: X_K [vy][vx],
+// X_J [vz][vx], X_I [vy][vz].  First the gather and the pass over the rows.
+template <int N, bool CONJ>
+__device__ __forceinline__ void cube_nyq1(const cpx<double> *__restrict__ F1, const cpx<double> *__restrict__ F2,
+                                         const cpx<double> *__restrict__ p1, const cpx<double> *__restrict__ p2,
+                                         cpx<double> *ny, int lane) {
+    using C = CubeGeo<N>;
+    constexpr int H = N / 2;
+    asm volatile("" : "+v"(lane));        // keeps the lane's 3 N addresses from being hoisted out of the product loop (and spilled)
+    const bool act = lane < 3 * N;
+    const int piece = act ? lane / N : 0, c = act ? lane % N : 0;
+    // element a of this lane's column, byte offset base + a * stride
+    constexpr uint32_t SZ = uint32_t(sizeof(cpx<double>));
+    const uint32_t base = uint32_t(piece == 0 ? H * C::N2 + c : (piece == 1 ? c * C::N2 + H : H * N + c)) * SZ;
+    const uint32_t stride = uint32_t(piece == 2 ? C::N2 : N) * SZ;
+    const BufView f1(F1, C::VOL * SZ), f2(F2, C::VOL * SZ);
+    // dims (x = 0, y = 1, z = 2) of the row, lane and fixed coordinate
+    const int drow = piece == 2 ? 2 : 0, dlane = piece == 1 ? 2 : 1, dfix = piece == 0 ? 2 : (piece == 1 ? 1 : 0);
+    const bool drop = piece != 0 && c == H, dropH = drop || piece == 2;
+    cpx<double> v[N];
+    if constexpr (CONJ) {
+        // A_1 + i A_2 = (1 + i) F Re((1 - i) psi h), psi the item's phase, h = (1 - e^{i N theta.nyq}) / 2
+        auto nq = [&](int d) { const cpx<double> u = {p1[d * N + H].x, -p1[d * N + H].y}; return fq::cmul(u, u); };
+        const cpx<double> q = fq::cmul(p1[dlane * N + c], p1[dfix * N + H]);
+        cpx<double> w0 = nq(dfix);
+        if (c == H) w0 = fq::cmul(w0, nq(dlane));
+        const cpx<double> wH = fq::cmul(w0, nq(drow));
+        auto qh = [&](cpx<double> w) {
+            const cpx<double> hq = fq::cmul(q, cpx<double>{0.5 * (1.0 - w.x), -0.5 * w.y});
+            return cpx<double>{hq.x + hq.y, hq.y - hq.x};                       // (1 - i) q h
+        };
+        const cpx<double> Q0 = drop ? cpx<double>{0, 0} : qh(w0);
+        const cpx<double> QH = dropH ? cpx<double>{0, 0} : qh(wH);
+#pragma unroll
+        for (int a = 0; a < N; ++a) {
+            const cpx<double> Q = a == H ? QH : Q0;
+            const cpx<double> r = p1[drow * N + a], x = f1.ld<double>(base + a * stride, 0);
+            const double w = fq::fmadd(r.x, Q.x, -(r.y * Q.y));
+            v[a] = {x.x * w, x.y * w};
+        }
+    } else {
+        // A_1 + i A_2 with A_t = psi_t h_t F_t
+        cpx<double> Q0[2], QH[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const cpx<double> *p = t ? p2 : p1;
+            auto nq = [&](int d) { const cpx<double> u = {p[d * N + H].x, -p[d * N + H].y}; return fq::cmul(u, u); };
+            const cpx<double> q = fq::cmul(p[dlane * N + c], p[dfix * N + H]);
+            cpx<double> w0 = nq(dfix);
+            if (c == H) w0 = fq::cmul(w0, nq(dlane));
+            const cpx<double> wH = fq::cmul(w0, nq(drow));
+            auto qh = [&](cpx<double> w) {
+                const cpx<double> hq = fq::cmul(q, cpx<double>{0.5 * (1.0 - w.x), -0.5 * w.y});
+                return t ? cpx<double>{-hq.y, hq.x} : hq;
+            };
+            Q0[t] = drop ? cpx<double>{0, 0} : qh(w0);
+            QH[t] = dropH ? cpx<double>{0, 0} : qh(wH);
+        }
+#pragma unroll
+        for (int a = 0; a < N; ++a) {
+            const cpx<double> x1 = f1.ld<double>(base + a * stride, 0), x2 = f2.ld<double>(base + a * stride, 0);
+            v[a] = fq::cmul(x1, fq::cmul(p1[drow * N + a], a == H ? QH[0] : Q0[0]));
+            fq::cmac(v[a], x2, fq::cmul(p2[drow * N + a], a == H ? QH[1] : Q0[1]));
+        }
+    }
+    fq::LFFT<N, 1>::run(v);                                    // over a, lane c
+    cpx<double> *L = ny + piece * C::N2;
+    if (act) {
+#pragma unroll
+        for (int a = 0; a < N; ++a) L[rot<N>(a, c)] = v[a];
+    }
+}
+
+// Their second pass, over the lane coordinate of the first.
+template <int N, bool CONJ> __device__ __forceinline__ void cube_nyq2(cpx<double> *ny, int lane) {
+    using C = CubeGeo<N>;
+    asm volatile("" : "+v"(lane));
+    const bool act = lane < 3 * N;
+    const int piece = act ? lane / N : 0, c = act ? lane % N : 0;
+    cpx<double> *L = ny + piece * C::N2;
+    cpx<double> v[N];
+#pragma unroll
+    for (int b = 0; b < N; ++b) v[b] = L[rot<N>(c, b)];
+    fq::LFFT<N, 1>::run(v);
+    plane_sync<32>();                                          // the three pieces live in one wave
+    if (act) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const cpx<double> x = v[j];
+            L[j * N + c] = CONJ ? cpx<double>{x.x - x.y, x.x + x.y} : x;        // (1 + i) X
+        }
+    }
+}
+
+template <int N, bool CONJ, bool MG>
+__global__ __launch_bounds__(CubeGeo<N>::THREADS, 2) void k_cube(
+    const cpx<double> *__restrict__ F, double *__restrict__ Rv, const cpx<double> *__restrict__ ph,
+    const DevProd *__restrict__ prods, const int *__restrict__ item_src, const CubeSeg *__restrict__ segs, int nseg,
+    const cpx<double> *__restrict__ W, int nsrc) {
+    using C = CubeGeo<N>;
+    __shared__ cpx<double> L[N * C::PLANE + 3 * C::N2];
+    cpx<double> *ny = L + N * C::PLANE;
+    // the segments of a slot stay on one XCD when the grid allows it: they share F
+    const int64_t unit = (gridDim.x & 7) == 0 ? xcd_block() : int64_t(blockIdx.x);
+    const int sg = int(unit % nseg), slot = int(unit / nseg);
+    const int tid = int(threadIdx.x);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const bool act = tid < C::N2;
+    const int a = act ? tid / N : 0, b = act ? tid % N : 0;
+    const int ab = a * N + b;
+    constexpr uint32_t PB = uint32_t(C::N2 * sizeof(cpx<double>)), VB = N * PB;    // plane and volume bytes
+    const uint32_t vo = uint32_t(ab * sizeof(cpx<double>));
+    const cpx<double> *Fs = F + int64_t(slot) * nsrc * C::VOL;
+    if (C::NYQ_WAVE && tid >= C::MAIN) {
+        // the Nyquist wave: a product's planes in two passes beside the other
+        // waves' z and x stages, with the barriers of the main path below
+        const CubeSeg sd = segs[sg];
+        for (int pi = sd.p0; pi < sd.p0 + sd.np; ++pi) {
+            const DevProd pr = prods[pi];
+            cube_nyq1<N, CONJ>(Fs + int64_t(item_src[pr.i1]) * C::VOL, Fs + int64_t(item_src[pr.i2]) * C::VOL,
+                               ph + int64_t(pr.i1) * 3 * N, ph + int64_t(pr.i2) * 3 * N, ny, tid - C::MAIN);
+            __syncthreads();                                   // z stage written
+            cube_nyq2<N, CONJ>(ny, tid - C::MAIN);
+            __syncthreads();                                   // x stage written
+            if (MG) { __syncthreads(); __syncthreads(); }      // forward
+            __syncthreads();                                   // L and ny free
+        }
+        if (!MG) { __syncthreads(); __syncthreads(); }         // forward
+        __syncthreads();                                       // inverse
+        __syncthreads();
+        return;
+    }
+    // pencils of the lane in L: along the plane index, along the row, along the column
+    cpx<double> *Lz = L + a * C::ROW + b, *Lx = L + a * C::PLANE + b, *Ly = L + a * C::PLANE + b * C::ROW;
+    cpx<double> H[N];
+    if constexpr (MG) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) H[k] = {0, 0};
+    }
+    const CubeSeg sd = segs[sg];
+    // one product: leaves its values over vy in v, lane (vz, vx)
+    auto product = [&](int pi, cpx<double> *v) {
+        const DevProd pr = prods[pi];
+        const cpx<double> *F1 = Fs + int64_t(item_src[pr.i1]) * C::VOL;
+        const cpx<double> *F2 = Fs + int64_t(item_src[pr.i2]) * C::VOL;
+        const cpx<double> *p1 = ph + int64_t(pr.i1) * 3 * N, *p2 = ph + int64_t(pr.i2) * 3 * N;
+        // z: lane (I, J), the packed T_1 + i T_2 over K
+        const cpx<double> q1 = fq::cmul(p1[a], p1[N + b]);
+        const BufView f1(F1, VB), f2(F2, VB);
+        if constexpr (CONJ) {
+            // (1 + i) Re((1 - i) gamma) F, gamma = q1 phi_z(K); the (1 + i) is applied after the transforms
+            const double A = q1.x + q1.y, B = q1.x - q1.y;
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                const cpx<double> z = p1[2 * N + k], x = f1.ld<double>(vo, k * PB);
+                const double w = fq::fmadd(z.x, A, z.y * B);
+                v[k] = {x.x * w, x.y * w};
+            }
+        } else {
+            const cpx<double> q2 = fq::cmul(p2[a], p2[N + b]);
+            const cpx<double> i2 = {-q2.y, q2.x};
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                v[k] = fq::cmul(f1.ld<double>(vo, k * PB), fq::cmul(p1[2 * N + k], q1));
+                fq::cmac(v[k], f2.ld<double>(vo, k * PB), fq::cmul(p2[2 * N + k], i2));
+            }
+        }
+        fq::LFFT<N, 1>::run(v);                            // -> vz
+        if (act) {
+#pragma unroll
+            for (int k = 0; k < N; ++k) Lz[k * C::PLANE] = v[k];
+        }
+        if (!C::NYQ_WAVE && wave == pi % C::NW) {
+            cube_nyq1<N, CONJ>(F1, F2, p1, p2, ny, tid % 64);
+            plane_sync<32>();
+            cube_nyq2<N, CONJ>(ny, tid % 64);
+        }
+        __syncthreads();
+        // x: lane (vz, J) over I, in place
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] = Lx[k * C::ROW];
+        fq::LFFT<N, 1>::run(v);                            // -> vx
+        if (act) {
+#pragma unroll
+            for (int k = 0; k < N; ++k) Lx[k * C::ROW] = v[k];
+        }
+        __syncthreads();
+        // y: lane (vz, vx) over J
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] = Ly[k];
+        fq::LFFT<N, 1>::run(v);                            // -> vy
+        const double cf = pr.coef, sz = (a & 1) ? -1.0 : 1.0, sx = (b & 1) ? -1.0 : 1.0;
+        const cpx<double> xj = ny[C::N2 + ab];
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const cpx<double> xk = ny[j * N + b], xi = ny[2 * C::N2 + j * N + a];
+            const double jx = (j & 1) ? -xj.x : xj.x, jy = (j & 1) ? -xj.y : xj.y;
+            const double ux = fq::fmadd(sx, xi.x, fq::fmadd(sz, xk.x, jx));
+            const double uy = fq::fmadd(sx, xi.y, fq::fmadd(sz, xk.y, jy));
+            const double ex = CONJ ? v[j].x - v[j].y : v[j].x, ey = CONJ ? v[j].x + v[j].y : v[j].y;
+            const double rx = ex - ux, ry = ey - uy;
+            // (rx + i uy)(ry - i ux)
+            v[j].x = cf * fq::fmadd(rx, ry, uy * ux);
+            if constexpr (MG) v[j].y = cf * fq::fmadd(uy, ry, -(rx * ux));
+        }
+    };
+    // forward: lane (vz, vx) over vy -> lane (I, J) over K (the first pass
+    // goes into the lane's own row, which no other lane reads)
+    auto forward = [&](cpx<double> *v) {
+        fq::LFFT<N, -1>::run(v);
+        if (act) {
+#pragma unroll
+            for (int k = 0; k < N; ++k) Ly[k] = v[k];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] = Lx[k * C::ROW];
+        fq::LFFT<N, -1>::run(v);                           // vx -> I
+        if (act) {
+#pragma unroll
+            for (int k = 0; k < N; ++k) Lx[k * C::ROW] = v[k];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] = Lz[k * C::PLANE];
+        fq::LFFT<N, -1>::run(v);                           // vz -> K
+    };
+    if constexpr (MG) {
+        for (int pi = sd.p0; pi < sd.p0 + sd.np; ++pi) {
+            cpx<double> v[N];
+            product(pi, v);
+            forward(v);
+            const BufView w(W + int64_t(pi) * C::VOL, VB);
+#pragma unroll
+            for (int k = 0; k < N; ++k) fq::cmac(H[k], w.ld<double>(vo, k * PB), v[k]);
+            __syncthreads();                               // the columns are read before the next product's z stage
+        }
+    } else {
+        double acc[N];                                     // real part of the group sum
+#pragma unroll
+        for (int j = 0; j < N; ++j) acc[j] = 0;
+        for (int pi = sd.p0; pi < sd.p0 + sd.np; ++pi) {
+            cpx<double> v[N];
+            product(pi, v);
+#pragma unroll
+            for (int j = 0; j < N; ++j) acc[j] += v[j].x;
+            __syncthreads();                               // L and ny free
+        }
+        cpx<double> v[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) v[j] = {acc[j], 0.0};
+        forward(v);
+        const BufView w(W + int64_t(sd.g) * C::VOL, VB);
+#pragma unroll
+        for (int k = 0; k < N; ++k) H[k] = fq::cmul(w.ld<double>(vo, k * PB), v[k]);
+    }
+    // Re DFT+(H): lane (I, J), K -> vz, into the lane's own column
+    fq::LFFT<N, 1>::run(H);
+    if (act) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) Lz[k * C::PLANE] = H[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; ++k) H[k] = Lx[k * C::ROW];
+    fq::LFFT<N, 1>::run(H);                                    // lane (vz, J): I -> vx
+    if (act) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) Lx[k * C::ROW] = H[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; ++k) H[k] = Ly[k];
+    fq::LFFT<N, 1>::run(H);                                    // lane (vz, vx): J -> vy
+    if (act) {
+        double *r = Rv + (int64_t(slot) * (nseg + 1) + sg) * C::VOL + tid;      // [vy][vz][vx]
+#pragma unroll
+        for (int k = 0; k < N; ++k) r[k * C::N2] = H[k].x;
+    }
+}
+
+// Q = sum_seg R_seg - f R_loss, 32 batch slots x 64 points per workgroup: the
+// volumes are read along the points, Q written with the slots on adjacent
+// lanes (consecutive elements of one solution point share an AoSoA row).
+__global__ __launch_bounds__(256) void k_cube_out(const double *__restrict__ Rv, AosoaPtrs ptr, Dof dof, int N,
+                                                  int nseg, int D) {
+    __shared__ double sg[32][65], sl[32][65];
+    const int n2 = N * N, n = n2 * N, nt = (n + 63) / 64;
+    const int tid = int(threadIdx.x);
+    const int s0 = int(blockIdx.x) / nt * 32, r0 = int(blockIdx.x) % nt * 64;
+    const int p = tid % 64;
+    if (r0 + p < n) {
+        // eight slots per thread side by side, so their loads are in flight together
+        const double *r[8];
+        double x[8], l[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int e = tid / 64 + 4 * i;
+            r[i] = Rv + int64_t(s0 + e < D ? s0 + e : s0) * (nseg + 1) * n + r0 + p;
+            x[i] = 0;
+            l[i] = r[i][int64_t(nseg) * n];
+        }
+        for (int k = 0; k < nseg; ++k) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[i] += r[i][int64_t(k) * n];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int e = tid / 64 + 4 * i;
+            sg[e][p] = x[i];
+            sl[e][p] = l[i];
+        }
+    }
+    __syncthreads();
+    const int e = tid % 32;
+    if (s0 + e >= D) return;
+    const int64_t b = dof.base(s0 + e);
+    const double *f = ptr.f[0] + b;
+    double *q = ptr.q[0] + b;
+#pragma unroll 4
+    for (int i = tid / 32; i < 64 && r0 + i < n; i += 8) {
+        const int r = r0 + i, vy = r / n2, vz = (r / N) % N, vx = r % N;
+        const int64_t at = ((int64_t(vx) * N + vy) * N + vz) * dof.soasz;
+        q[at] = sg[e][i] - f[at] * sl[e][i];
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Grids without native kernels (any even N other than 8, 16, 24 and 32).
 // The batched 3D transforms run in the ROCm FFT library (hipFFT plans, the
 // counterpart of the reference's cuFFT plans, frfs/solvers/dgfs/scattering.py:
@@ -2646,6 +3111,10 @@ struct fq_handle {
     float *NB = nullptr;         // scratch [chunk][groups][kNbPer32]
     cpx<double> *Cn = nullptr;   // scratch [chunk][targets][kCPer32]
     double *MOM = nullptr;       // scratch [chunk][targets][N][5]
+    // cube kernels (FP64, one target, even N up to 20): segments of the plan
+    bool cube = false;
+    CubeSeg *segs = nullptr;
+    int nseg = 0;
     // grids without native kernels: hipFFT plans for `chunk` slots (F,
     // the items A and B, the group volume G, the gain and loss Y) sharing one
     // work area, and the contributions of each group
@@ -2678,6 +3147,44 @@ static const char *kKernelNames[FQ_NKERNELS] = {"k_fwd_z", "k_fwd_xy", "k_inv_z"
                                                 "k_out",   "k_project", "k_prod",  "k_nyq",   "k_nyqb"};
 
 namespace {
+
+bool conj_product(const fq::Plan &P, const fq::PProd &pr) {
+    bool c = P.items[pr.i1].src == P.items[pr.i2].src;
+    for (int d = 0; d < 3; ++d) c = c && P.items[pr.i2].th[d] == -P.items[pr.i1].th[d];
+    return c;
+}
+
+// The plan's segments for k_cube (false: it has no form for this plan): runs
+// of at most kSegProds products, within one group (VHS) or of as many
+// single-product groups (VSS, conjugate products).  The weights are indexed by
+// group, so contribution g has to be group g.
+bool cube_segments(const fq::Plan &P, std::vector<CubeSeg> &segs, bool &conj) {
+    conj = true;
+    for (auto &pr : P.prods) conj = conj && conj_product(P, pr);
+    if (int(P.contribs.size()) != P.ngroups || P.loss.size() != 1) return false;
+    for (int g = 0; g < P.ngroups; ++g)
+        if (P.contribs[g].group != g || P.group_np[g] < 1) return false;
+    segs.clear();
+    if (P.model == FQ_MODEL_VSS) {
+        for (int g = 0; g < P.ngroups; ++g)
+            if (P.group_np[g] != 1 || P.group_p0[g] != g) return false;
+        if (!conj) return false;
+        const int ns = (P.ngroups + kSegProds - 1) / kSegProds;
+        for (int i = 0; i < ns; ++i) {
+            const int b = int(int64_t(P.ngroups) * i / ns), e = int(int64_t(P.ngroups) * (i + 1) / ns);
+            segs.push_back({b, b, e - b});
+        }
+        return true;
+    }
+    for (int g = 0; g < P.ngroups; ++g) {
+        const int np = P.group_np[g], ns = (np + kSegProds - 1) / kSegProds;
+        for (int i = 0; i < ns; ++i) {
+            const int b = np * i / ns, e = np * (i + 1) / ns;
+            segs.push_back({g, P.group_p0[g] + b, e - b});
+        }
+    }
+    return true;
+}
 
 template <typename T> int upload_phases(fq_handle *h) {
     const fq::Plan &P = h->P;
@@ -2733,8 +3240,7 @@ template <typename T> int upload_nyq(fq_handle *h) {
     bool conj = true, anyconj = false;
     for (size_t p = 0; p < P.prods.size(); ++p) {
         const auto &pr = P.prods[p];
-        bool c = P.items[pr.i1].src == P.items[pr.i2].src;
-        for (int d = 0; d < 3; ++d) c = c && P.items[pr.i2].th[d] == -P.items[pr.i1].th[d];
+        const bool c = conj_product(P, pr);
         pc[p] = c ? 1 : 0;
         conj = conj && c;
         anyconj = anyconj || c;
@@ -3218,6 +3724,54 @@ template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, cons
     return FQ_SUCCESS;
 }
 
+// One batch of D DOFs through the cube kernels.
+template <int N>
+int run_chunk_cube(fq_handle *h, const Scratch &sc, const AosoaPtrs &ptr, const Dof &dof, int D, bool prof,
+                   hipStream_t st) {
+    using C = CubeGeo<N>;
+    const fq::Plan &P = h->P;
+    std::pair<hipEvent_t, hipEvent_t> cur{};
+    auto pre = [&]() {
+        if (!prof) return;
+        auto get = [&]() {
+            hipEvent_t e;
+            if (!h->ev_pool.empty()) { e = h->ev_pool.back(); h->ev_pool.pop_back(); }
+            else (void)hipEventCreate(&e);
+            return e;
+        };
+        cur = {get(), get()};
+        (void)hipEventRecord(cur.first, st);
+    };
+    auto post = [&](int k) {
+        if (prof) { (void)hipEventRecord(cur.second, st); h->ev_rec.push_back({k, cur}); }
+    };
+    double *R = reinterpret_cast<double *>(sc.Pg);
+    const bool mg = P.model == FQ_MODEL_VSS;
+    pre();
+    hipLaunchKernelGGL(k_cube_fwd<N>, dim3(unsigned(D * P.nsrc)), dim3(C::MAIN), 0, st, ptr, dof, sc.F, P.nsrc,
+                       h->W + int64_t(P.contribs.size()) * C::VOL, P.loss[0].src, R, h->nseg);
+    post(1);
+    pre();
+    auto kern = mg ? k_cube<N, true, true> : (h->pack_conj ? k_cube<N, true, false> : k_cube<N, false, false>);
+    hipLaunchKernelGGL(kern, dim3(unsigned(int64_t(D) * h->nseg)), dim3(C::THREADS), 0, st, sc.F, R,
+                       reinterpret_cast<const cpx<double> *>(h->ph), h->prods, h->item_src, h->segs, h->nseg, h->W,
+                       P.nsrc);
+    post(7);
+    pre();
+    hipLaunchKernelGGL(k_cube_out, dim3(unsigned((D + 31) / 32 * ((C::VOL + 63) / 64))), dim3(256), 0, st, R, ptr, dof,
+                       N, h->nseg, D);
+    post(5);
+    if (h->flags & FQ_FLAG_PROJECT) {
+        pre();
+        hipLaunchKernelGGL(k_project, dim3(unsigned(8 * ((D + 7) / 8))), dim3(256), 0, st, ptr, dof, 1, N, P.L,
+                           h->ginv, h->pmass, D);
+        post(6);
+    }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(FQ_ERR_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
+    return FQ_SUCCESS;
+}
+
 // One batch of D DOFs on a grid without native kernels (see k_gen_gather):
 // library transforms of `chunk` slots and grid-stride pointwise kernels.
 #define FFTCHK(x)                                                                          \
@@ -3404,6 +3958,22 @@ int eval_impl(fq_handle *h, const Scratch *sc, int nsets, int64_t chunk, bool pr
         const Scratch &s = sc[two ? i % 2 : 0];
         const hipStream_t bs = two && (i % 2) ? h->st2 : st;
         int rc;
+        if (h->cube) {
+            switch (h->P.N) {
+            case 4: rc = run_chunk_cube<4>(h, s, ptr, dof, D, prof, bs); break;
+            case 6: rc = run_chunk_cube<6>(h, s, ptr, dof, D, prof, bs); break;
+            case 8: rc = run_chunk_cube<8>(h, s, ptr, dof, D, prof, bs); break;
+            case 10: rc = run_chunk_cube<10>(h, s, ptr, dof, D, prof, bs); break;
+            case 12: rc = run_chunk_cube<12>(h, s, ptr, dof, D, prof, bs); break;
+            case 14: rc = run_chunk_cube<14>(h, s, ptr, dof, D, prof, bs); break;
+            case 16: rc = run_chunk_cube<16>(h, s, ptr, dof, D, prof, bs); break;
+            case 18: rc = run_chunk_cube<18>(h, s, ptr, dof, D, prof, bs); break;
+            case 20: rc = run_chunk_cube<20>(h, s, ptr, dof, D, prof, bs); break;
+            default: rc = fail(FQ_ERR_UNSUPPORTED, "grid size not built");
+            }
+            if (rc != FQ_SUCCESS) return rc;
+            continue;
+        }
         if (h->generic) {
             rc = h->precision == FQ_PREC_MIXED ? run_chunk_gen<float>(h, s, ptr, dof, D, prof, bs)
                                                : run_chunk_gen<double>(h, s, ptr, dof, D, prof, bs);
@@ -3589,6 +4159,16 @@ int fq_create(const fq_params *prm, fq_handle **out) {
     h->two_lane = !generic && (prm->flags & FQ_FLAG_TWO_LANE) != 0;
     h->pack = !generic && h->fused && !(h->two_lane && h->precision == FQ_PREC_MIXED) &&
               (prm->Nv == 24 || prm->Nv == 32) && !(prm->flags & FQ_FLAG_NO_PACK);
+    // the cube kernels: FP64 (the volume and the Nyquist planes of 22^3 pass the
+    // LDS), one target (H of one target fits the registers), default schedule
+    // (the flags that name another way to run the products keep it).  Against
+    // the path that served the grid before they are 1.03-2.5 times as fast on 8^3
+    // and 16^3 from 1 to 4096 DOFs, and 20-60 times on the library path's grids.
+    h->cube = prm->precision == FQ_PREC_FP64 && h->P.ntgt == 1 && (!n_supported(prm->Nv) || prm->Nv == 8 || prm->Nv == 16) &&
+              prm->Nv <= kCubeMaxN && !(prm->flags & (FQ_FLAG_LIBRARY_FFT | FQ_FLAG_UNFUSED | FQ_FLAG_NO_PACK));
+    std::vector<CubeSeg> segs;
+    if (h->cube) h->cube = cube_segments(h->P, segs, h->pack_conj);
+    h->nseg = int(segs.size());
     h->nvol = generic ? 3 : h->P.ngroups;         // library path: the items A, B and the group G
     if (h->pack && !h->two_lane && prm->Nv == 32 && h->precision == FQ_PREC_MIXED && !(prm->flags & FQ_FLAG_NO_HPAIR)) {
         bool single = true;
@@ -3629,6 +4209,7 @@ int fq_create(const fq_params *prm, fq_handle **out) {
     chk(upload(&h->l_src, ls));
     chk(upload(&h->t_l0, tl0));
     chk(upload(&h->t_ln, tln));
+    if (h->cube) chk(upload(&h->segs, segs));
     if (rc == FQ_SUCCESS) rc = build_tables(h);
     if (rc == FQ_SUCCESS) rc = build_projection(h);
     if (rc == FQ_SUCCESS && h->pack)
@@ -3638,10 +4219,11 @@ int fq_create(const fq_params *prm, fq_handle **out) {
     const size_t tsz = h->precision == FQ_PREC_MIXED ? sizeof(cpx<float>) : sizeof(cpx<double>);
     const size_t per_dof_F = size_t(P.nsrc) * n * sizeof(cpx<double>);
     // Z holds the staged inverse transforms (three-kernel path only), T0 and Y
-    const size_t per_dof_Z = std::max({h->fused ? size_t(0) : P.items.size() * n * tsz,
+    const size_t per_dof_Z = h->cube ? 0 : std::max({h->fused ? size_t(0) : P.items.size() * n * tsz,
                                        size_t(P.nsrc) * n * sizeof(cpx<double>),
                                        size_t(2 * P.ntgt) * n * sizeof(cpx<double>)});
-    const size_t per_dof_P = size_t(h->nvol) * n * tsz;
+    // cube kernels: one real volume per segment and the loss
+    const size_t per_dof_P = h->cube ? size_t(h->nseg + 1) * n * sizeof(double) : size_t(h->nvol) * n * tsz;
     const size_t per_dof_F32 = h->precision == FQ_PREC_MIXED ? size_t(P.nsrc) * n * sizeof(cpx<float>) : 0;
     // Nyquist-plane corrections of the pair-packed product kernel and the
     // spectrum slices they are computed from
@@ -3669,7 +4251,7 @@ int fq_create(const fq_params *prm, fq_handle **out) {
         const size_t budget = size_t(8) << 30;    // 8 GiB default scratch budget (of 288 GB HBM)
         // the library path also holds an FFT work area of up to one Y per DOF
         chunk = std::max<int64_t>(1, int64_t(budget / ((per_dof + (generic ? per_dof_Z : 0)) * ns)));
-        chunk = std::min<int64_t>(chunk, generic ? 512 : 4096);
+        chunk = std::min<int64_t>(chunk, generic && !h->cube ? 512 : 4096);
     }
     h->chunk = chunk;
     if (rc == FQ_SUCCESS && (h->flags & FQ_FLAG_NO_SCRATCH)) {
@@ -3677,7 +4259,7 @@ int fq_create(const fq_params *prm, fq_handle **out) {
     } else if (rc == FQ_SUCCESS) {
         const size_t cs = size_t(chunk) * ns;
         hipError_t e1 = hipMalloc(&h->F, per_dof_F * cs);
-        hipError_t e2 = hipMalloc(&h->Z, per_dof_Z * cs);
+        hipError_t e2 = per_dof_Z ? hipMalloc(&h->Z, per_dof_Z * cs) : hipSuccess;
         hipError_t e3 = hipMalloc(&h->Pg, per_dof_P * cs);
         hipError_t e4 = hipSuccess;
         if (h->precision == FQ_PREC_MIXED) e4 = hipMalloc(&h->F32, per_dof_F32 * cs);
@@ -3694,7 +4276,7 @@ int fq_create(const fq_params *prm, fq_handle **out) {
         if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess || e4 != hipSuccess || e5 != hipSuccess)
             rc = fail(FQ_ERR_ALLOC, "hipMalloc scratch failed (reduce max_chunk)");
         h->scratch = per_dof * cs;
-        if (rc == FQ_SUCCESS && generic) {
+        if (rc == FQ_SUCCESS && generic && !h->cube) {
             // unused batch slots of A, B and G start as zeros, not stale bits
             if (hipMemset(h->Pg, 0, per_dof_P * cs) != hipSuccess) rc = fail(FQ_ERR_HIP, "hipMemset scratch");
             if (rc == FQ_SUCCESS) rc = make_gen_plans(h);
@@ -3780,7 +4362,7 @@ int fq_destroy(fq_handle *h) {
                     (void *)h->t_ln, (void *)h->W, (void *)h->ginv, (void *)h->pmass, (void *)h->F, h->Z,
                     h->Pg, h->zc, (void *)h->F32, h->NY, h->FJ, (void *)h->nyv, (void *)h->zq,
                     (void *)h->pconj, (void *)h->X, (void *)h->VN, (void *)h->e_vol, (void *)h->t_e0,
-                    (void *)h->t_en, (void *)h->NB, (void *)h->Cn, (void *)h->MOM})
+                    (void *)h->t_en, (void *)h->NB, (void *)h->Cn, (void *)h->MOM, (void *)h->segs})
         if (p) (void)hipFree(p);
     (void)hipThreadExchangeStreamCaptureMode(&mode);
     delete h;

@@ -231,7 +231,9 @@ enum fq_path {
     FQ_PATH_PAIR_PACK = 4,    /* the two items of a product as one complex volume */
     FQ_PATH_GROUP_PAIRS = 8,  /* two groups' real parts as one product volume */
     FQ_PATH_OVERLAP = 16,     /* two scratch sets and two streams */
-    FQ_PATH_LIBRARY_FFT = 32  /* grid without native kernels: hipFFT transforms */
+    FQ_PATH_LIBRARY_FFT = 32  /* grid without a schedule of its own: hipFFT
+                                 transforms, or in FP64 with one target up to
+                                 20^3 the kernels that keep a volume in LDS */
 };
 int fq_get_paths(const fq_handle *h, int32_t *paths);
 
