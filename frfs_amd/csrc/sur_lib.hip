@@ -14,7 +14,11 @@
 // Weight gradients are per-workgroup sums over 512 grid points, added with
 // vector-memory atomics into a caller-zeroed gradient vector.
 //
-// Layouts: activations are [batch][channel][x] FP32 with x = (I*N+J)*N+K;
+// Inference (one or more folded layers) does not use those: it runs the real
+// 9-coefficient transforms on the matrix cores (k_fno_*, further down).
+//
+// Layouts: activations are [batch][channel][x] FP32 with x = (I*N+J)*N+K
+// ([batch][x][channel] in the inference pass, FP32 or 16 bit);
 // mode arrays are [batch][channel][k] complex with k = (px*8+py)*8+pz and
 // wavenumber index kidx(p) per axis; theta holds P, p0, per layer
 // (R (i,o,k) complex interleaved, Wm (o,i), b), Qw, q0.
@@ -60,6 +64,31 @@ __device__ constexpr float kCos32[32] = {
 template <int N> __device__ __forceinline__ float cosN(int j) { return kCos32[(j * (32 / N)) & 31]; }
 template <int N> __device__ __forceinline__ float sinN(int j) { return cosN<N>(j - N / 4); }
 
+// 1 + erf(z / sqrt 2) = 2 - E for z > 0, else E, with E = erfc(|z| / sqrt 2) =
+// 2^{-q(|z|)} and q a degree-10 fit of -log2 erfc (weighted least squares for
+// the error of gelu, |z| <= 6.2; positive and growing beyond).  About 20
+// instructions without a branch (erff takes both of its ranges in most waves).
+// The FP32 gelu from it is off by 7.0e-8 rms and 3.8e-7 at most on [-6, 6]
+// (7.9e-8 and 4.5e-7 with a correctly rounded erf).
+__device__ __forceinline__ float one_plus_erf(float z) {
+    const float u = fabsf(z);
+    float a = 1.756848888589957e-08f;
+    a = __builtin_fmaf(a, u, -5.725348728446988e-07f);
+    a = __builtin_fmaf(a, u, 7.934887435112614e-06f);
+    a = __builtin_fmaf(a, u, -5.907857484999113e-05f);
+    a = __builtin_fmaf(a, u, 0.00022106834512669593f);
+    a = __builtin_fmaf(a, u, 0.00011856652417918667f);
+    a = __builtin_fmaf(a, u, -0.007087948732078075f);
+    a = __builtin_fmaf(a, u, 0.05253392457962036f);
+    a = __builtin_fmaf(a, u, 0.4591914415359497f);
+    a = __builtin_fmaf(a, u, 1.1511074304580688f);
+    const float e = __builtin_amdgcn_exp2f(-(a * u));
+    return z > 0.f ? 2.0f - e : e;
+}
+__device__ __forceinline__ float gelu_fit(float z) { return 0.5f * z * one_plus_erf(z); }
+// Training keeps erff in both directions: gelu' needs 1 + erf itself, for which
+// the fit (weighed by z) is less exact near zero, and the passes there are
+// bound by memory.
 __device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
 // Activation storage: FP32, or FP16 / BF16 for inference (arithmetic stays
 // FP32; conversions round to nearest even).
@@ -887,6 +916,7 @@ __global__ __launch_bounds__(256) void k_sur_cons(int N, double c0, double dc, d
 constexpr int64_t FRC0 = 2LL * SW * SM3, FRQ = FRC0 + 2 * SW, FA = FRQ + 2LL * SW * SM3;
 constexpr int64_t FA0 = FA + SW, FQW = FA0 + SW, FQB = FQW + SW, FTOT = FQB + 1;
 static_assert(FTOT == FQ_SUR_FUSED_FLOATS, "folded weight layout");
+static_assert(FA0 == FA + SW && FQB == FQW + SW, "k_fno_plane reads A, a0 and QW, qb side by side");
 
 __global__ __launch_bounds__(256) void k_sur_fuse(const float *__restrict__ th, int L, float *__restrict__ fw) {
     const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
@@ -945,75 +975,466 @@ __global__ __launch_bounds__(256) void k_sur_fuse(const float *__restrict__ th, 
     }
 }
 
-// Y(b,o,k) = Xg(b,k) Rp(o,k) + [k = 0] c0(o)
-__global__ __launch_bounds__(256) void k_sur_mix_first(const float2 *__restrict__ Xg, const float *__restrict__ fw,
-                                                       float2 *__restrict__ Y, int64_t total) {
-    const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= total) return;
-    const int k = int(idx & (SM3 - 1));
-    const int o = int((idx >> 9) & (SW - 1));
-    const int64_t b = idx >> 14;
-    const float2 x = Xg[b * SM3 + k];
-    const float2 r = reinterpret_cast<const float2 *>(fw)[o * SM3 + k];
-    float2 y = make_float2(x.x * r.x - x.y * r.y, x.x * r.y + x.y * r.x);
-    if (k == 0) {
-        const float2 c = reinterpret_cast<const float2 *>(fw + FRC0)[o];
-        y.x += c.x;
-        y.y += c.y;
-    }
-    Y[idx] = y;
+// ---------------------------------------------------------------------------
+// The inference pass on the matrix cores.
+//
+// The retained modes of one axis, wavenumbers -4..3, are the span of the nine
+// real functions beta_r: 1; cos(q t), q = 1..3; sin(q t), q = 1..3; cos(4 t);
+// sin(4 t) (t = 2 pi x / N).  For a real input the mode X(k) with signs
+// s_d = sign k_d and q_d = |k_d| is a signed sum of the eight products of
+// cos / sin coefficients of its class (q_x, q_y, q_z),
+//   e^{-i k.x} = prod_d (cos - i s_d sin),
+// and the real part of the inverse transform needs only the transposed sums,
+// so both transforms are real and separable, 9 coefficients per axis:
+//   P[xr][yr][zr] = sum_{I,J,K} beta_xr(I) beta_yr(J) beta_zr(K) v(I,J,K)
+//   s(I,J,K) = sum_{xr,yr,zr} beta_xr(I) beta_yr(J) beta_zr(K) Q[xr][yr][zr],
+// with Q the folded mode outputs Y(k) = sum_i X_i(k) R(i,o,k).  Every stage is
+// a small dense product of FP32 values and runs as
+// v_mfma_f32_16x16x4_f32 (FP32 operands, FP32 sums):
+//   k_fno_plane   one plane I of one DOF: z = Wm v + b + s from the plane's
+//                 T[yr][zr][c] (y stage, then the z stage fused into the
+//                 channel product), gelu, the new v, and the z and y stages of
+//                 its forward transform, U[yr][zr][c]
+//   k_fno_x       the x stages: U -> P (forward) and Q -> T (inverse)
+//   k_fno_mix     P -> Q, a workgroup per class and 64 DOFs
+// so one layer reads and writes the activations once (the transforms' volume s
+// and the second and third pass over v are gone), and the last layer's input is
+// never stored.  Activations are kept as
+// [b][x][channel], so a lane's operands are contiguous.
+//
+// What bounds it: the plane kernel's two streams of v (8.4 MB per DOF and
+// layer on the 32^3 grid, 1 MB on 16^3) and, nearly as long, its 30 matrix
+// instructions and 8 gelu per lane for every 16 points.  Measured for L = 4:
+// 4096 DOFs on 16^3 20.5 ms with one VALU pass over v per stage, 11.6 ms now;
+// 700 DOFs on 32^3 10.99 -> 4.64 ms, of it the plane kernels 4.13 ms (first
+// layer 1.10, writing 2.9 GB; middle 1.60, reading and writing them; last
+// 1.43, reading), the mode product 0.16 and the x stages 0.38.  Error against
+// 64 bits 2.4e-7 -> 1.4e-7.
+// Channels of a column tile t: o = 2 * (lane % 16) + t, so that the two tiles
+// of a lane are neighbours (8-byte accesses).
+// ---------------------------------------------------------------------------
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int NR = 9, NR2 = NR * NR, NR3 = NR2 * NR;     // real coefficients per axis, plane, volume
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// v_1(o) = gelu(A_o g + a0_o + s_0(o)) per point
-template <int N, typename TA>
-__global__ __launch_bounds__(256) void k_sur_pw_first(const float *__restrict__ g, const TA *__restrict__ s,
-                                                      const float *__restrict__ fw, TA *__restrict__ vout,
-                                                      int64_t total) {
-    const int64_t idx = 2 * (int64_t(blockIdx.x) * 256 + threadIdx.x);   // two points per thread
-    if (idx >= total) return;
-    const int64_t b = idx >> SG<N>::LOG3;
-    const int x = int(idx & (SG<N>::N3 - 1));
-    const float2 gv = ld2(g, idx);
-#pragma unroll 8
-    for (int o = 0; o < SW; ++o) {
-        const int64_t at = (b * SW + o) * SG<N>::N3 + x;
-        const float2 sv = ld2(s, at);
-        st2(vout, at, make_float2(gelu(fw[FA + o] * gv.x + fw[FA0 + o] + sv.x),
-                                  gelu(fw[FA + o] * gv.y + fw[FA0 + o] + sv.y)));
+// beta_r(j); zero for the padding rows r >= 9.
+template <int N> __device__ __forceinline__ float beta(int r, int j) {
+    const bool sn = (r >= 4 && r <= 6) || r == 8;
+    const int q = r < 4 ? r : (r < 7 ? r - 3 : 4);
+    const float v = kCos32[(q * j * (32 / N) - (sn ? 8 : 0)) & 31];
+    return r < NR ? v : 0.f;
+}
+
+// Eight consecutive activations as floats.
+__device__ __forceinline__ void ld8(const float *p, float *v) {
+    const f32x4 a = reinterpret_cast<const f32x4 *>(p)[0], b = reinterpret_cast<const f32x4 *>(p)[1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { v[i] = a[i]; v[4 + i] = b[i]; }
+}
+template <typename TA> __device__ __forceinline__ void ld8(const TA *p, float *v) {
+    const Pack8<TA> a = *reinterpret_cast<const Pack8<TA> *>(p);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = float(a.v[i]);
+}
+
+// Sum over the 16 lanes of a row (DPP rotations by 8, 4, 2, 1).
+__device__ __forceinline__ float row_sum(float x) {
+    auto ror = [](float y, auto c) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, y), decltype(c)::value, 0xF, 0xF, true));
+    };
+    x += ror(x, std::integral_constant<int, 0x128>{});
+    x += ror(x, std::integral_constant<int, 0x124>{});
+    x += ror(x, std::integral_constant<int, 0x122>{});
+    x += ror(x, std::integral_constant<int, 0x121>{});
+    return x;
+}
+
+// One plane I of DOF b per workgroup; FIRST: v_1 from g (lw: the folded first
+// layer's A, a0), else v_{l+1} from v_l in place (lw: the layer's Wm, b).
+// LAST: v_{L-1} is not stored; its part of the projection, QW . v + qb, goes
+// to out (qw: QW, qb) and its modes to U.
+template <int N, typename TA, bool FIRST, bool LAST>
+__global__ __launch_bounds__(256) void k_fno_plane(const float *__restrict__ T, const float *__restrict__ g,
+                                                   const float *__restrict__ lw, TA *__restrict__ v,
+                                                   float *__restrict__ U, const float *__restrict__ qw,
+                                                   float *__restrict__ out) {
+    constexpr int KT = N / 16;                               // 16-point tiles of a row, 16-row tiles of the plane
+    __shared__ float Fz[N * NR * SW];                        // [J][zr][c]: the row's z coefficients, in then out
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, q = lane >> 4;
+    const int64_t plane = blockIdx.x;                        // b * N + I
+    const float *tp = T + plane * (NR2 * SW);
+    // inverse y stage: Fz[J][zr] = sum_yr beta_yr(J) T[yr][zr]
+    for (int u = wave; u < NR * KT; u += 4) {
+        const int zr = u % NR, j0 = u / NR * 16;
+        f32x4 d0 = {0, 0, 0, 0}, d1 = d0;
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            const int yr = q + 4 * s;
+            const float2 t = *reinterpret_cast<const float2 *>(tp + ((yr < NR ? yr : NR - 1) * NR + zr) * SW + 2 * col);
+            const float a = beta<N>(yr, j0 + col);
+            d0 = mfma4(a, t.x, d0);
+            d1 = mfma4(a, t.y, d1);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<float2 *>(Fz + ((j0 + 4 * q + i) * NR + zr) * SW + 2 * col) = make_float2(d0[i], d1[i]);
+    }
+    // operands that stay: the channel matrix and bias of this lane's two outputs, the z tables
+    float wm[2][FIRST ? 1 : 8], w0[2], b0[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int o = 2 * col + t;
+        if constexpr (FIRST) {
+            w0[t] = lw[o];                                   // A
+            b0[t] = lw[SW + o];                              // a0
+        } else {
+            b0[t] = lw[SW * SW + o];
+#pragma unroll
+            for (int s = 0; s < 8; ++s) wm[t][s] = lw[o * SW + 8 * q + s];
+        }
+    }
+    float qw0 = 0.f, qw1 = 0.f, qb = 0.f;
+    if constexpr (LAST) { qw0 = qw[2 * col]; qw1 = qw[2 * col + 1]; qb = qw[SW]; }
+    float ez[KT][3], ef[KT][4];
+#pragma unroll
+    for (int k = 0; k < KT; ++k) {
+#pragma unroll
+        for (int s = 0; s < 3; ++s) ez[k][s] = beta<N>(q + 4 * s, 16 * k + col);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ef[k][i] = beta<N>(col, 16 * k + 4 * q + i);
+    }
+    __syncthreads();
+    for (int J = wave; J < N; J += 4) {
+        TA *row = v + ((plane * N + J) * N) * SW;
+        float2 f[3];
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            const int zr = q + 4 * s;
+            f[s] = *reinterpret_cast<const float2 *>(Fz + (J * NR + (zr < NR ? zr : NR - 1)) * SW + 2 * col);
+        }
+        f32x4 az0 = {0, 0, 0, 0}, az1 = az0;
+#pragma unroll
+        for (int k = 0; k < KT; ++k) {
+            f32x4 d0, d1;
+            if constexpr (FIRST) {
+                const float *gp = g + (plane * N + J) * N + 16 * k + 4 * q;
+                const float2 ga = reinterpret_cast<const float2 *>(gp)[0], gb = reinterpret_cast<const float2 *>(gp)[1];
+                const float gv[4] = {ga.x, ga.y, gb.x, gb.y};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    d0[i] = w0[0] * gv[i] + b0[0];
+                    d1[i] = w0[1] * gv[i] + b0[1];
+                }
+            } else {
+                float a[8];
+                ld8(row + (16 * k + col) * SW + 8 * q, a);
+                d0 = {b0[0], b0[0], b0[0], b0[0]};
+                d1 = {b0[1], b0[1], b0[1], b0[1]};
+#pragma unroll
+                for (int s = 0; s < 8; ++s) {
+                    d0 = mfma4(a[s], wm[0][s], d0);
+                    d1 = mfma4(a[s], wm[1][s], d1);
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+                d0 = mfma4(ez[k][s], f[s].x, d0);
+                d1 = mfma4(ez[k][s], f[s].y, d1);
+            }
+            float pv = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                // the transform and the projection take the value as stored
+                const TA x0 = TA(gelu_fit(d0[i])), x1 = TA(gelu_fit(d1[i]));
+                if constexpr (LAST) {
+                    const float r = row_sum(__builtin_fmaf(qw0, float(x0), qw1 * float(x1)));
+                    if (col == i) pv = r;                    // lane col < 4 keeps point 4 q + col
+                } else {
+                    Pair<TA> h;
+                    h.a = x0;
+                    h.b = x1;
+                    *reinterpret_cast<Pair<TA> *>(row + (16 * k + 4 * q + i) * SW + 2 * col) = h;
+                }
+                az0 = mfma4(ef[k][i], float(x0), az0);
+                az1 = mfma4(ef[k][i], float(x1), az1);
+            }
+            if (LAST && col < 4) out[(plane * N + J) * N + 16 * k + 4 * q + col] = pv + qb;
+        }
+        // the row's coefficients take the place of the ones just read (same wave, LDS in order)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (4 * q + i < NR)
+                *reinterpret_cast<float2 *>(Fz + (J * NR + 4 * q + i) * SW + 2 * col) = make_float2(az0[i], az1[i]);
+    }
+    __syncthreads();
+    // forward y stage: U[yr][zr] = sum_J beta_yr(J) Fz[J][zr]
+    for (int zr = wave; zr < NR; zr += 4) {
+        f32x4 d0 = {0, 0, 0, 0}, d1 = d0;
+#pragma unroll
+        for (int s = 0; s < N / 4; ++s) {
+            const int J = q + 4 * s;
+            const float2 t = *reinterpret_cast<const float2 *>(Fz + (J * NR + zr) * SW + 2 * col);
+            const float a = beta<N>(col, J);
+            d0 = mfma4(a, t.x, d0);
+            d1 = mfma4(a, t.y, d1);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (4 * q + i < NR)
+                *reinterpret_cast<float2 *>(U + plane * (NR2 * SW) + ((4 * q + i) * NR + zr) * SW + 2 * col) =
+                    make_float2(d0[i], d1[i]);
     }
 }
 
-// Y1(b,k) = sum_i X(b,i,k) Rq(i,k)
-__global__ __launch_bounds__(256) void k_sur_mix_last(const float2 *__restrict__ X, const float *__restrict__ fw,
-                                                      float2 *__restrict__ Y1, int64_t total) {
+// x stages, one wave per (b, yr, zr) and 32 channels.
+// FWD: P[b][xr][yz][c] = scale sum_I beta_xr(I) U[b][I][yz][c];
+// else T[b][I][yz][c] = sum_xr beta_xr(I) Q[b][xr][yz][c].
+template <int N, bool FWD>
+__global__ __launch_bounds__(256) void k_fno_x(const float *__restrict__ in, float *__restrict__ out, float scale,
+                                               int64_t units) {
+    const int lane = threadIdx.x & 63, col = lane & 15, q = lane >> 4;
+    const int64_t u = int64_t(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (u >= units) return;
+    const int64_t b = u / NR2;
+    const int yz = int(u % NR2);
+    if constexpr (FWD) {
+        const float *p = in + (b * N * NR2 + yz) * SW + 2 * col;
+        f32x4 d0 = {0, 0, 0, 0}, d1 = d0;
+#pragma unroll
+        for (int s = 0; s < N / 4; ++s) {
+            const int I = q + 4 * s;
+            const float2 t = *reinterpret_cast<const float2 *>(p + I * NR2 * SW);
+            const float a = beta<N>(col, I);
+            d0 = mfma4(a, t.x, d0);
+            d1 = mfma4(a, t.y, d1);
+        }
+        float *o = out + (b * NR3 + yz) * SW + 2 * col;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (4 * q + i < NR)
+                *reinterpret_cast<float2 *>(o + (4 * q + i) * NR2 * SW) = make_float2(scale * d0[i], scale * d1[i]);
+    } else {
+        const float *p = in + (b * NR3 + yz) * SW + 2 * col;
+        float2 t[3];
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            const int xr = q + 4 * s;
+            t[s] = *reinterpret_cast<const float2 *>(p + (xr < NR ? xr : NR - 1) * NR2 * SW);
+        }
+        float *o = out + (b * N * NR2 + yz) * SW + 2 * col;
+#pragma unroll
+        for (int k = 0; k < N / 16; ++k) {
+            f32x4 d0 = {0, 0, 0, 0}, d1 = d0;
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+                const float a = beta<N>(q + 4 * s, 16 * k + col);
+                d0 = mfma4(a, t[s].x, d0);
+                d1 = mfma4(a, t[s].y, d1);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                *reinterpret_cast<float2 *>(o + (16 * k + 4 * q + i) * NR2 * SW) = make_float2(d0[i], d1[i]);
+        }
+    }
+}
+
+// Class (q_x, q_y, q_z), q in 0..4, of the modes: class index cls = (q_x*5 + q_y)*5 + q_z.
+// Real coefficient e (bits x, y, z: 0 cos, 1 sin) of the class in the 9^3
+// layout, or -1 where a sine of q = 0 does not exist.
+__device__ __forceinline__ int cls_coef(int cls, int e) {
+    const int qd[3] = {cls / 25, cls / 5 % 5, cls % 5};
+    int at = 0;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const int sn = (e >> (2 - d)) & 1, qq = qd[d];
+        if (sn && qq == 0) return -1;
+        at = at * NR + (qq == 4 ? 7 + sn : qq + (sn ? 3 : 0));
+    }
+    return at;
+}
+// Mode m (bits x, y, z: 1 the negative wavenumber) of the class: index in the
+// 8^3 mode set and the signs, or -1 where the class has no such mode.
+__device__ __forceinline__ int cls_mode(int cls, int m, float *sg) {
+    const int qd[3] = {cls / 25, cls / 5 % 5, cls % 5};
+    int at = 0;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const int neg = (m >> (2 - d)) & 1, qq = qd[d];
+        if (qq == 0 && neg) return -1;                   // zero has one sign
+        if (qq == 4 && !neg) return -1;                  // only -4 is retained
+        at = at * SM + (neg ? SM - qq : qq);
+        sg[d] = qq == 0 ? 0.f : (neg ? -1.f : 1.f);
+    }
+    return at;
+}
+// X(k) from the class's real coefficients p[e], signs s.
+__device__ __forceinline__ float2 cls_x(const float *p, const float *s) {
+    return make_float2(p[0] - s[1] * s[2] * p[3] - s[0] * s[2] * p[5] - s[0] * s[1] * p[6],
+                       -(s[2] * p[1] + s[1] * p[2] + s[0] * p[4]) + s[0] * s[1] * s[2] * p[7]);
+}
+// Q += the folded Y(k).
+__device__ __forceinline__ void cls_fold(float *Q, float yr, float yi, const float *s) {
+    Q[0] += yr;
+    Q[3] -= s[1] * s[2] * yr;
+    Q[5] -= s[0] * s[2] * yr;
+    Q[6] -= s[0] * s[1] * yr;
+    Q[1] -= s[2] * yi;
+    Q[2] -= s[1] * yi;
+    Q[4] -= s[0] * yi;
+    Q[7] += s[0] * s[1] * s[2] * yi;
+}
+
+// Q = fold(X R) for the modes of class blockIdx.x and the 64 DOFs from
+// 64 * blockIdx.y, sixteen per wave.  The class's weights (up to 8 modes,
+// 64 KB) are staged in LDS; row rho of a mode holds input channel
+// i = 8 (rho % 4) + rho / 4, so the four lane groups read neighbouring rows.
+__global__ __launch_bounds__(256) void k_fno_mix(const float *__restrict__ P, const float2 *__restrict__ R,
+                                                 float *__restrict__ Q, int batch) {
+    __shared__ float Rl[8][2][SW * SW];
+    const int cls = blockIdx.x, tid = threadIdx.x, lane = tid & 63, col = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    for (int e = tid; e < SW * SW; e += 256) {
+        const int i = e / SW, o = e % SW, rho = (i % 8) * 4 + i / 8;
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            float sg[3];
+            const int k = cls_mode(cls, m, sg);
+            if (k < 0) continue;
+            const float2 r = R[int64_t(e) * SM3 + k];
+            Rl[m][0][rho * SW + o] = r.x;
+            Rl[m][1][rho * SW + o] = r.y;
+        }
+    }
+    __syncthreads();
+    const int b0 = blockIdx.y * 64 + wave * 16;
+    if (b0 >= batch) return;                             // no barrier follows
+    const int bl = b0 + col < batch ? b0 + col : batch - 1;
+    float p[8][8];                                       // [coefficient][s], input channel 8 q + s
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int at = cls_coef(cls, e);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) p[e][s] = 0.f;
+        if (at >= 0) ld8(P + (int64_t(bl) * NR3 + at) * SW + 8 * q, p[e]);
+    }
+    float acc[2][4][8];                                  // [tile][row][coefficient]
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[t][i][e] = 0.f;
+#pragma unroll 1
+    for (int m = 0; m < 8; ++m) {
+        float sg[3];
+        if (cls_mode(cls, m, sg) < 0) continue;
+        f32x4 yr[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, yi[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const float pe[8] = {p[0][s], p[1][s], p[2][s], p[3][s], p[4][s], p[5][s], p[6][s], p[7][s]};
+            const float2 x = cls_x(pe, sg);
+            const float2 rr = *reinterpret_cast<const float2 *>(&Rl[m][0][(4 * s + q) * SW + 2 * col]);
+            const float2 ri = *reinterpret_cast<const float2 *>(&Rl[m][1][(4 * s + q) * SW + 2 * col]);
+            yr[0] = mfma4(x.x, rr.x, yr[0]);
+            yr[1] = mfma4(x.x, rr.y, yr[1]);
+            yr[0] = mfma4(-x.y, ri.x, yr[0]);
+            yr[1] = mfma4(-x.y, ri.y, yr[1]);
+            yi[0] = mfma4(x.x, ri.x, yi[0]);
+            yi[1] = mfma4(x.x, ri.y, yi[1]);
+            yi[0] = mfma4(x.y, rr.x, yi[0]);
+            yi[1] = mfma4(x.y, rr.y, yi[1]);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) cls_fold(acc[t][i], yr[t][i], yi[t][i], sg);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int b = b0 + 4 * q + i;
+        if (b >= batch) continue;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int at = cls_coef(cls, e);
+            if (at >= 0)
+                *reinterpret_cast<float2 *>(Q + (int64_t(b) * NR3 + at) * SW + 2 * col) =
+                    make_float2(acc[0][i][e], acc[1][i][e]);
+        }
+    }
+}
+
+// First layer's Q from the one-channel modes Xg: Y(o,k) = Xg(k) Rp(o,k) +
+// [k = 0] c0(o).  One thread per (b, class, o).
+__global__ __launch_bounds__(256) void k_fno_first(const float2 *__restrict__ Xg, const float *__restrict__ fw,
+                                                   float *__restrict__ Q, int64_t total) {
     const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
     if (idx >= total) return;
-    const int k = int(idx & (SM3 - 1));
-    const int64_t b = idx >> 9;
+    const int o = int(idx % SW), cls = int(idx / SW % 125);
+    const int64_t b = idx / (SW * 125);
+    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+        float sg[3];
+        const int k = cls_mode(cls, m, sg);
+        if (k < 0) continue;
+        const float2 x = Xg[b * SM3 + k], r = reinterpret_cast<const float2 *>(fw)[o * SM3 + k];
+        float2 y = make_float2(x.x * r.x - x.y * r.y, x.x * r.y + x.y * r.x);
+        if (k == 0) {
+            const float2 c = reinterpret_cast<const float2 *>(fw + FRC0)[o];
+            y.x += c.x;
+            y.y += c.y;
+        }
+        cls_fold(acc, y.x, y.y, sg);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int at = cls_coef(cls, e);
+        if (at >= 0) Q[(b * NR3 + at) * SW + o] = acc[e];
+    }
+}
+
+// Last layer's one output channel: Y1(b,k) = sum_i X(b,i,k) Rq(i,k).  One
+// half-wave per (b, class), a lane per input channel.
+__global__ __launch_bounds__(256) void k_fno_last(const float *__restrict__ P, const float *__restrict__ fw,
+                                                  float2 *__restrict__ Y1, int64_t units) {
+    const int64_t u = int64_t(blockIdx.x) * 8 + threadIdx.x / 32;
+    if (u >= units) return;
+    const int i = threadIdx.x & 31, cls = int(u % 125);
+    const int64_t b = u / 125;
     const float2 *Rq = reinterpret_cast<const float2 *>(fw + FRQ);
-    float2 a = make_float2(0.f, 0.f);
-    for (int i = 0; i < SW; ++i) {
-        const float2 x = X[(b * SW + i) * SM3 + k];
-        const float2 r = Rq[i * SM3 + k];
-        a.x += x.x * r.x - x.y * r.y;
-        a.y += x.x * r.y + x.y * r.x;
+    float p[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int at = cls_coef(cls, e);
+        p[e] = at >= 0 ? P[(b * NR3 + at) * SW + i] : 0.f;
     }
-    Y1[idx] = a;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+        float sg[3];
+        const int k = cls_mode(cls, m, sg);
+        if (k < 0) continue;
+        const float2 x = cls_x(p, sg), r = Rq[i * SM3 + k];
+        float yr = x.x * r.x - x.y * r.y, yi = x.x * r.y + x.y * r.x;
+#pragma unroll
+        for (int s = 16; s > 0; s >>= 1) {
+            yr += __shfl_xor(yr, s);
+            yi += __shfl_xor(yi, s);
+        }
+        if (i == 0) Y1[b * SM3 + k] = make_float2(yr, yi);
+    }
 }
 
-// out(b,x) = QW . v(b,:,x) + qb + s1(b,x)
-template <int N, typename TA>
-__global__ __launch_bounds__(256) void k_sur_pw_last(const TA *__restrict__ v, const TA *__restrict__ s1,
-                                                     const float *__restrict__ fw, float *__restrict__ out,
-                                                     int64_t total) {
+// out += s1
+__global__ __launch_bounds__(256) void k_fno_add(const float *__restrict__ s1, float *__restrict__ out, int64_t pts) {
     const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= total) return;
-    const int64_t b = idx >> SG<N>::LOG3;
-    const int x = int(idx & (SG<N>::N3 - 1));
-    float a = fw[FQB] + ldA(s1, idx);
-#pragma unroll 8
-    for (int i = 0; i < SW; ++i) a += fw[FQW + i] * ldA(v, (b * SW + i) * SG<N>::N3 + x);
-    out[idx] = a;
+    if (idx < pts) out[idx] += s1[idx];
 }
 
 inline unsigned nblk(int64_t n) { return unsigned((n + 255) / 256); }
@@ -1072,38 +1493,43 @@ ActPtrs act_ptrs(int N3, float *acts, int L, int64_t B, bool training) {
     return p;
 }
 
-// The folded inference pass with activations stored as A (FP32 or FP16) in
-// the FP32-sized regions of the inference activation layout.
+// The folded inference pass with activations stored as A (FP32 or 16 bits),
+// in the inference activation space: v [b][x][c], then T and U
+// [b][I][yr][zr][c], P and Q [b][xr][yr][zr][c], the one-channel modes X and
+// the one-channel volume s.
 template <int N, typename A>
 void forward_fused(int L, const float *theta, const float *fused, const float *g, int64_t batch, float *acts,
                    float *out, hipStream_t st) {
-    const ActPtrs p = act_ptrs(SG<N>::N3, acts, L, batch, false);
-    A *v[2] = {reinterpret_cast<A *>(p.v[0]), reinterpret_cast<A *>(p.v[1])};
-    A *sa = reinterpret_cast<A *>(p.s);
-    const int64_t pts = batch * SG<N>::N3;
-    const unsigned slices = unsigned(batch * SW);
+    constexpr int N3 = SG<N>::N3;
+    const int64_t vol = batch * SW * N3, tp = batch * N * NR2 * SW, pq = batch * NR3 * SW;
+    A *v = reinterpret_cast<A *>(acts);
+    float *T = acts + vol, *U = T + tp, *P = U + tp, *Q = P + pq;
+    float2 *X = reinterpret_cast<float2 *>(Q + pq);
+    float *s1 = Q + pq + 2 * batch * SM3;
+    static_assert(int64_t(SW) * N3 + 2 * N * NR2 * SW + 2 * NR3 * SW + 2 * SM3 + N3 <=
+                  3LL * SW * N3 + 4 * SW * SM3, "fits the inference activation space");
+    const int64_t pts = batch * N3, xu = batch * NR2;
+    const dim3 blk(256), pg(unsigned(batch * N)), xg(unsigned((xu + 3) / 4));
     // first layer from the one-channel transform of g
-    launch_dft<N, float>(g, 1.0f / SG<N>::N3, p.X[0], unsigned(batch), st);
-    hipLaunchKernelGGL(k_sur_mix_first, dim3(nblk(batch * SW * SM3)), dim3(256), 0, st, p.X[0], fused, p.Y,
-                       batch * SW * SM3);
-    launch_idft<N, A>(p.Y, 1.0f, 0, sa, slices, st);
-    hipLaunchKernelGGL((k_sur_pw_first<N, A>), dim3(nblk(pts / 2)), dim3(256), 0, st, g, sa, fused, v[1], pts);
+    launch_dft<N, float>(g, 1.0f / N3, X, unsigned(batch), st);
+    hipLaunchKernelGGL(k_fno_first, dim3(nblk(batch * 125 * SW)), blk, 0, st, X, fused, Q, batch * 125 * SW);
+    hipLaunchKernelGGL((k_fno_x<N, false>), xg, blk, 0, st, Q, T, 1.0f, xu);
+    hipLaunchKernelGGL((L == 2 ? k_fno_plane<N, A, true, true> : k_fno_plane<N, A, true, false>), pg, blk, 0, st, T, g,
+                       fused + FA, v, U, fused + FQW, out);
     for (int l = 1; l < L - 1; ++l) {
         const float *lay = theta + 2 * SW + l * SLAYER;
-        const float2 *R = reinterpret_cast<const float2 *>(lay);
-        launch_dft<N, A>(v[l & 1], 1.0f / SG<N>::N3, p.X[l], slices, st);
-        hipLaunchKernelGGL(k_sur_mix_lds<0>, dim3(SM3 / 8, unsigned((batch + 31) / 32)), dim3(256), 0, st, p.X[l],
-                           R, p.Y, batch);
-        launch_idft<N, A>(p.Y, 1.0f, 0, sa, slices, st);
-        hipLaunchKernelGGL((k_sur_pw<N, A>), dim3(nblk(pts / 2)), dim3(256), 0, st, v[l & 1], sa, lay + SR, 1, nullptr,
-                           v[(l + 1) & 1], pts);
+        hipLaunchKernelGGL((k_fno_x<N, true>), xg, blk, 0, st, U, P, 1.0f / N3, xu);
+        hipLaunchKernelGGL(k_fno_mix, dim3(125, unsigned((batch + 63) / 64)), blk, 0, st, P,
+                           reinterpret_cast<const float2 *>(lay), Q, int(batch));
+        hipLaunchKernelGGL((k_fno_x<N, false>), xg, blk, 0, st, Q, T, 1.0f, xu);
+        hipLaunchKernelGGL((l == L - 2 ? k_fno_plane<N, A, false, true> : k_fno_plane<N, A, false, false>), pg, blk, 0,
+                           st, T, g, lay + SR, v, U, fused + FQW, out);
     }
     // last layer and projection as one output channel
-    launch_dft<N, A>(v[(L - 1) & 1], 1.0f / SG<N>::N3, p.X[L - 1], slices, st);
-    hipLaunchKernelGGL(k_sur_mix_last, dim3(nblk(batch * SM3)), dim3(256), 0, st, p.X[L - 1], fused, p.Y,
-                       batch * SM3);
-    launch_idft<N, A>(p.Y, 1.0f, 0, sa, unsigned(batch), st);
-    hipLaunchKernelGGL((k_sur_pw_last<N, A>), dim3(nblk(pts)), dim3(256), 0, st, v[(L - 1) & 1], sa, fused, out, pts);
+    hipLaunchKernelGGL((k_fno_x<N, true>), xg, blk, 0, st, U, P, 1.0f / N3, xu);
+    hipLaunchKernelGGL(k_fno_last, dim3(unsigned((batch * 125 + 7) / 8)), blk, 0, st, P, fused, X, batch * 125);
+    launch_idft<N, float>(X, 1.0f, 0, s1, unsigned(batch), st);
+    hipLaunchKernelGGL(k_fno_add, dim3(nblk(pts)), blk, 0, st, s1, out, pts);
 }
 
 // The unfolded pass (training keeps v_l, z_l and X_l) with activations

@@ -20,7 +20,8 @@
  * with g = f / (rho f_ref) and out ~ Q / (rho^2 q_ref) (Q is quadratic in f).
  * theta layout (floats): P (W), p0 (W), per layer [R (W*W*m^3 complex,
  * (i, o, k) order, interleaved), Wm (W*W, (o, i)), b (W)], Qw (W), q0.
- * Activation arrays are [batch][channel][x] FP32, x = (I*N + J)*N + K.
+ * Activation arrays are [batch][channel][x] FP32, x = (I*N + J)*N + K; the
+ * inference pass uses its acts as scratch in an order of its own.
  *
  * All buffers are caller-owned device memory; nothing here allocates.
  * Errors: FQ_SUCCESS or a negative FQ_ERR_* code with fq_last_error().
