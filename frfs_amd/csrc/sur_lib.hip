@@ -9,13 +9,9 @@
 //   s_l(x)   = Re sum_k Y_l(k) e^{+2 pi i k.x/N}        (k_sur_idft, per channel)
 //   z_l      = Wm_l v_l + b_l + s_l,  v_{l+1} = gelu(z_l) (last layer: z_l)
 //   out      = Qw . v_L + q0                            (projection)
-// Backward passes reuse the same transforms: the adjoint of Re(IDFT) is the
-// unscaled forward DFT and the adjoint of (1/n) DFT is (1/n) Re(IDFT).
-// Weight gradients are per-workgroup sums over 512 grid points, added with
-// vector-memory atomics into a caller-zeroed gradient vector.
-//
-// Inference (one or more folded layers) does not use those: it runs the real
-// 9-coefficient transforms on the matrix cores (k_fno_*, further down).
+// This is the unfolded pass (training, one layer).  Inference with the lift and
+// the projection folded in, and the gradients, run on the matrix cores with real
+// 9-coefficient transforms (k_fno_*, k_fnt_*, further down).
 //
 // Layouts: activations are [batch][channel][x] FP32 with x = (I*N+J)*N+K
 // ([batch][x][channel] in the inference pass, FP32 or 16 bit);
@@ -86,9 +82,8 @@ __device__ __forceinline__ float one_plus_erf(float z) {
     return z > 0.f ? 2.0f - e : e;
 }
 __device__ __forceinline__ float gelu_fit(float z) { return 0.5f * z * one_plus_erf(z); }
-// Training keeps erff in both directions: gelu' needs 1 + erf itself, for which
-// the fit (weighed by z) is less exact near zero, and the passes there are
-// bound by memory.
+// Training keeps erff: gelu' needs 1 + erf itself, for which the fit (weighed by
+// z) is less exact near zero.
 __device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
 // Activation storage: FP32, or FP16 / BF16 for inference (arithmetic stays
 // FP32; conversions round to nearest even).
@@ -109,8 +104,10 @@ template <typename TA> __device__ __forceinline__ void st2(TA *p, int64_t i, flo
 // eight 16-bit values, one 16-byte store
 template <typename TA> struct alignas(16) Pack8 { TA v[8]; };
 
-__device__ __forceinline__ float gelu_grad(float z) {
-    return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * __expf(-0.5f * z * z);
+// gelu(z), gelu'(z)
+__device__ __forceinline__ float2 gelu_both(float z) {
+    const float h = 0.5f * (1.0f + erff(z * 0.70710678118654752f));
+    return make_float2(z * h, h + z * 0.39894228040143268f * __expf(-0.5f * z * z));
 }
 
 // X[slice] = scale * sum_x v[slice](x) e^{-i k.x} over the retained modes.
@@ -189,11 +186,10 @@ __global__ __launch_bounds__(256) void k_sur_dft16(const TA *__restrict__ v, flo
     }
 }
 
-// out[slice](x) = (accumulate ? out : 0) + scale * Re sum_k Y[slice](k) e^{+i k.x}
+// out[slice](x) = Re sum_k Y[slice](k) e^{+i k.x}
 // (16^3 grid).
 template <typename TA>
-__global__ __launch_bounds__(256) void k_sur_idft16(const float2 *__restrict__ Y, float scale, int accumulate,
-                                                  TA *__restrict__ out) {
+__global__ __launch_bounds__(256) void k_sur_idft16(const float2 *__restrict__ Y, TA *__restrict__ out) {
     __shared__ float2 Ys[SM3];               // [px][py][pz]
     __shared__ float2 T1[16 * SM * SM];      // [I][py][pz]
     __shared__ float2 T2[SG<16>::N2 * 9];           // [I][J][pz]
@@ -251,23 +247,15 @@ __global__ __launch_bounds__(256) void k_sur_idft16(const float2 *__restrict__ Y
         float sum = 0.f;
 #pragma unroll
         for (int pz = 0; pz < SM; ++pz) sum += a[pz].x * cosN<16>(kidx<16>(pz) * K) - a[pz].y * sinN<16>(kidx<16>(pz) * K);
-        o[K] = scale * sum;
+        o[K] = sum;
     }
     if constexpr (std::is_same<TA, float>::value) {
         float4 *dst = reinterpret_cast<float4 *>(out + slice * SG<16>::N3 + t * 16);
 #pragma unroll
         for (int q = 0; q < 16 / 4; ++q) {
-            float4 w = make_float4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);
-            if (accumulate) {
-                const float4 p0 = dst[q];
-                w.x += p0.x;
-                w.y += p0.y;
-                w.z += p0.z;
-                w.w += p0.w;
-            }
-            dst[q] = w;
+            dst[q] = make_float4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);
         }
-    } else {                                  // 16-bit inference output (never accumulated)
+    } else {                                  // 16-bit activations
         static_assert(sizeof(TA) == 2, "16-bit storage");
         Pack8<TA> *dst = reinterpret_cast<Pack8<TA> *>(out + slice * SG<16>::N3 + t * 16);
 #pragma unroll
@@ -387,8 +375,7 @@ __global__ __launch_bounds__(kDft32Threads) void k_sur_dft32(const TA *__restric
 // thread t computes row t's 32 outputs into LDS (ob) and the workgroup writes
 // the pass with coalesced 16-byte stores.
 template <typename TA>
-__global__ __launch_bounds__(kDft32Threads) void k_sur_idft32(const float2 *__restrict__ Y, float scale,
-                                                            int accumulate, TA *__restrict__ out) {
+__global__ __launch_bounds__(kDft32Threads) void k_sur_idft32(const float2 *__restrict__ Y, TA *__restrict__ out) {
     constexpr int N = 32, N3 = SG<32>::N3, T = kDft32Threads, RS = N + 1;
     __shared__ float2 T2[N * kRowsI];         // [I][J][pz] (aidx32); first the modes [px][py][pz]
     __shared__ float ob[T * RS];              // T1 [I][py][pz], then one pass of output rows
@@ -448,7 +435,7 @@ __global__ __launch_bounds__(kDft32Threads) void k_sur_idft32(const float2 *__re
 #pragma unroll
             for (int pz = 0; pz < SM; ++pz)
                 sum += a[pz].x * cosN<N>(kidx<N>(pz) * K) - a[pz].y * sinN<N>(kidx<N>(pz) * K);
-            ob[t * RS + K] = scale * sum;
+            ob[t * RS + K] = sum;
         }
         __syncthreads();
         TA *rows = out + slice * N3 + int64_t(q) * T * N;
@@ -457,18 +444,9 @@ __global__ __launch_bounds__(kDft32Threads) void k_sur_idft32(const float2 *__re
             for (int w = 0; w < T * N / 4 / T; ++w) {
                 const int e4 = t + T * w;
                 const float *sp = ob + (e4 >> 3) * RS + (e4 & 7) * 4;
-                float4 x = make_float4(sp[0], sp[1], sp[2], sp[3]);
-                float4 *dp = reinterpret_cast<float4 *>(rows) + e4;
-                if (accumulate) {
-                    const float4 p0 = *dp;
-                    x.x += p0.x;
-                    x.y += p0.y;
-                    x.z += p0.z;
-                    x.w += p0.w;
-                }
-                *dp = x;
+                reinterpret_cast<float4 *>(rows)[e4] = make_float4(sp[0], sp[1], sp[2], sp[3]);
             }
-        } else {                              // 16-bit inference output (never accumulated)
+        } else {                              // 16-bit activations
 #pragma unroll
             for (int w = 0; w < T * N / 8 / T; ++w) {
                 const int e8 = t + T * w;
@@ -490,76 +468,57 @@ void launch_dft(const TA *v, float scale, float2 *X, unsigned slices, hipStream_
     else hipLaunchKernelGGL(k_sur_dft32<TA>, dim3(slices), dim3(kDft32Threads), 0, st, v, scale, X);
 }
 template <int N, typename TA>
-void launch_idft(const float2 *Y, float scale, int accumulate, TA *out, unsigned slices, hipStream_t st) {
-    if constexpr (N == 16) hipLaunchKernelGGL(k_sur_idft16<TA>, dim3(slices), dim3(256), 0, st, Y, scale, accumulate, out);
-    else hipLaunchKernelGGL(k_sur_idft32<TA>, dim3(slices), dim3(kDft32Threads), 0, st, Y, scale, accumulate, out);
+void launch_idft(const float2 *Y, TA *out, unsigned slices, hipStream_t st) {
+    if constexpr (N == 16) hipLaunchKernelGGL(k_sur_idft16<TA>, dim3(slices), dim3(256), 0, st, Y, out);
+    else hipLaunchKernelGGL(k_sur_idft32<TA>, dim3(slices), dim3(kDft32Threads), 0, st, Y, out);
 }
 
-// Weight gradient of the mixing: gR(i,o,k) += sum_b conj X(b,i,k) gY(b,o,k).
-// One thread per (i, o, k), k fastest, so every access is coalesced.
-__global__ __launch_bounds__(256) void k_sur_mix_grad(const float2 *__restrict__ X, const float2 *__restrict__ gY,
-                                                      float2 *__restrict__ gR, int64_t batch) {
-    const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= int64_t(SW) * SW * SM3) return;
-    const int k = int(idx & (SM3 - 1));
-    const int o = int((idx >> 9) & (SW - 1));
-    const int i = int(idx >> 14);
-    float2 acc = make_float2(0.f, 0.f);
-    for (int64_t b = 0; b < batch; ++b) {
-        const float2 x = X[(b * SW + i) * SM3 + k];
-        const float2 g = gY[(b * SW + o) * SM3 + k];
-        acc.x += x.x * g.x + x.y * g.y;
-        acc.y += x.x * g.y - x.y * g.x;
-    }
-    gR[idx].x += acc.x;
-    gR[idx].y += acc.y;
-}
-
-// The forward and input-gradient mixing:
-// MODE 0: Y(b,o,k) = sum_i X(b,i,k) R(i,o,k);
-// MODE 1: gX(b,i,k) = sum_o gY(b,o,k) conj R(i,o,k).
-// A workgroup takes 8 consecutive modes and 32 DOFs and stages the 8 modes'
-// 32 x 32 weights in LDS (64 KB) once; thread (mode m = t % 8, DOF d = t / 8)
-// keeps its 32 outputs in registers.  Within a wave the eight DOFs of a mode
-// read the same LDS word (a broadcast), so the weight reads are conflict-free.
-template <int MODE>
+// The mode product of the unfolded forward pass, Y(b,o,k) = sum_i X(b,i,k) R(i,o,k).
+// A workgroup takes 8 consecutive modes and 16 DOFs and stages the 8 modes'
+// 32 x 32 weights in LDS (64 KB) once; thread (mode m = t % 8, DOF t / 8 % 16,
+// half t / 128 of the outputs) keeps its 16 outputs in registers.  Within a
+// wave the eight DOFs of a mode read the same LDS word (a broadcast), so the
+// weight reads are conflict-free.  Bound by latency for a training batch: 64
+// DOFs 40 us with 32 DOFs and 32 outputs per thread (128 workgroups, the
+// weights loaded one LDS store at a time), 20 us now; the sums are the same.
 __global__ __launch_bounds__(256) void k_sur_mix_lds(const float2 *__restrict__ a, const float2 *__restrict__ R,
                                                      float2 *__restrict__ c, int64_t batch) {
     __shared__ float2 Rl[SW * SW * 8];               // [(i*32 + o)*8 + m]
     const int t = threadIdx.x;
     const int k0 = blockIdx.x * 8;
-    for (int e = t; e < SW * SW * 8; e += 256) Rl[e] = R[int64_t(e >> 3) * SM3 + k0 + (e & 7)];
-    __syncthreads();
-    const int m = t & 7;
-    const int64_t b = int64_t(blockIdx.y) * 32 + (t >> 3);
-    if (b >= batch) return;
+    const int m = t & 7, h = (t >> 7) * (SW / 2);
+    const int64_t b = int64_t(blockIdx.y) * 16 + ((t >> 3) & 15);
     const int k = k0 + m;
-    float2 acc[SW];
-#pragma unroll
-    for (int j = 0; j < SW; ++j) acc[j] = make_float2(0.f, 0.f);
-    // all 32 inputs in flight at once: occupancy is set by the LDS tile (two
-    // waves per SIMD), so the registers are free
+    // all 32 inputs in flight at once, before the weights: occupancy is set by
+    // the LDS tile (two waves per SIMD), so the registers are free
     float2 xs[SW];
 #pragma unroll
-    for (int j = 0; j < SW; ++j) xs[j] = a[(b * SW + j) * SM3 + k];
+    for (int j = 0; j < SW; ++j) xs[j] = a[((b < batch ? b : batch - 1) * SW + j) * SM3 + k];
+#pragma unroll 1
+    for (int e = t; e < SW * SW * 8; e += 256 * 16) {
+        float2 r[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) r[u] = R[int64_t((e + 256 * u) >> 3) * SM3 + k0 + (e & 7)];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) Rl[e + 256 * u] = r[u];
+    }
+    __syncthreads();
+    if (b >= batch) return;
+    float2 acc[SW / 2];
+#pragma unroll
+    for (int j = 0; j < SW / 2; ++j) acc[j] = make_float2(0.f, 0.f);
 #pragma unroll
     for (int j = 0; j < SW; ++j) {
         const float2 x = xs[j];
 #pragma unroll
-        for (int q = 0; q < SW; ++q) {
-            if constexpr (MODE == 0) {      // j = i, q = o
-                const float2 r = Rl[(j * SW + q) * 8 + m];
-                acc[q].x += x.x * r.x - x.y * r.y;
-                acc[q].y += x.x * r.y + x.y * r.x;
-            } else {                        // j = o, q = i
-                const float2 r = Rl[(q * SW + j) * 8 + m];
-                acc[q].x += x.x * r.x + x.y * r.y;
-                acc[q].y += x.y * r.x - x.x * r.y;
-            }
+        for (int q = 0; q < SW / 2; ++q) {
+            const float2 r = Rl[(j * SW + h + q) * 8 + m];
+            acc[q].x += x.x * r.x - x.y * r.y;
+            acc[q].y += x.x * r.y + x.y * r.x;
         }
     }
 #pragma unroll
-    for (int j = 0; j < SW; ++j) c[(b * SW + j) * SM3 + k] = acc[j];
+    for (int j = 0; j < SW / 2; ++j) c[(b * SW + h + j) * SM3 + k] = acc[j];
 }
 
 // v_0(b, c, x) = P_c g(b, x) + p0_c
@@ -619,94 +578,6 @@ __global__ __launch_bounds__(256) void k_sur_proj(const TA *__restrict__ v, cons
     out[idx] = s;
 }
 
-// gv(b, c, x) = Qw_c gout(b, x)
-template <int N>
-__global__ __launch_bounds__(256) void k_sur_proj_bwd(const float *__restrict__ gout, const float *__restrict__ qw,
-                                                      float *__restrict__ gv, int64_t total) {
-    const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= total) return;
-    const int64_t b = idx >> SG<N>::LOG3;
-    const int x = int(idx & (SG<N>::N3 - 1));
-    const float g = gout[idx];
-#pragma unroll 8
-    for (int c = 0; c < SW; ++c) gv[(b * SW + c) * SG<N>::N3 + x] = qw[c] * g;
-}
-
-// gz = gv * gelu'(z) (or gv for the last layer), written over gv;
-// gvin = Wm^T gz.
-template <int N, typename TA>
-__global__ __launch_bounds__(256) void k_sur_pw_bwd(float *__restrict__ gv, const TA *__restrict__ z,
-                                                    const float *__restrict__ lw, int act, float *__restrict__ gvin,
-                                                    int64_t total) {
-    // weight rows are read at uniform addresses (scalar loads), row o scaled
-    // by gz_o and added into the 32 input-channel sums
-    const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= total) return;
-    const int64_t b = idx >> SG<N>::LOG3;
-    const int x = int(idx & (SG<N>::N3 - 1));
-    float a[SW];
-#pragma unroll
-    for (int i = 0; i < SW; ++i) a[i] = 0.f;
-#pragma unroll 4
-    for (int o = 0; o < SW; ++o) {
-        const int64_t at = (b * SW + o) * SG<N>::N3 + x;
-        const float g = gv[at];
-        const float gz = act ? g * gelu_grad(ldA(z, at)) : g;
-        gv[at] = gz;
-#pragma unroll
-        for (int i = 0; i < SW; ++i) a[i] += lw[o * SW + i] * gz;
-    }
-#pragma unroll
-    for (int i = 0; i < SW; ++i) gvin[(b * SW + i) * SG<N>::N3 + x] = a[i];
-}
-
-// G(o, i) += sum_{b, x} A(b, o, x) V(b, i, x);  gb(o) += sum_{b, x} A(b, o, x).
-// Grid T * batch with T = N^3 / 512 tiles per DOF: workgroup w sums the 512
-// points from (w % T) * 512 of DOF w / T in LDS tiles of 64.
-template <int N, int COUT, int CIN, typename TV>
-__global__ __launch_bounds__(256) void k_sur_wgrad(const float *__restrict__ A, const TV *__restrict__ V,
-                                                   float *__restrict__ G, float *__restrict__ gb) {
-    constexpr int NO = COUT * CIN;
-    constexpr int PER = (NO + 255) / 256;
-    __shared__ float As[COUT][65];
-    __shared__ float Vs[CIN][65];
-    const int t = threadIdx.x;
-    constexpr int TILES = SG<N>::N3 / 512;
-    const int64_t b = blockIdx.x / TILES;
-    const int x0 = int(blockIdx.x % TILES) * 512;
-    float acc[PER];
-#pragma unroll
-    for (int q = 0; q < PER; ++q) acc[q] = 0.f;
-    float accb = 0.f;
-    for (int p0 = x0; p0 < x0 + 512; p0 += 64) {
-        for (int e = t; e < COUT * 64; e += 256) As[e >> 6][e & 63] = A[(b * COUT + (e >> 6)) * SG<N>::N3 + p0 + (e & 63)];
-        for (int e = t; e < CIN * 64; e += 256) Vs[e >> 6][e & 63] = ldA(V, (b * CIN + (e >> 6)) * SG<N>::N3 + p0 + (e & 63));
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < PER; ++q) {
-            const int j = t + 256 * q;
-            if (j < NO) {
-                const int o = j / CIN, i = j % CIN;
-                float s = 0.f;
-#pragma unroll 16
-                for (int p = 0; p < 64; ++p) s += As[o][p] * Vs[i][p];
-                acc[q] += s;
-            }
-        }
-        if (t < COUT) {
-#pragma unroll 16
-            for (int p = 0; p < 64; ++p) accb += As[t][p];
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-        const int j = t + 256 * q;
-        if (j < NO) atomicAdd(&G[j], acc[q]);
-    }
-    if (t < COUT) atomicAdd(&gb[t], accb);
-}
-
 // Per-DOF workgroups are dealt round-robin to the eight XCDs; workgroup w
 // takes DOF (w % 8) * per + w / 8 so that each XCD works through a contiguous
 // DOF range and neighbouring elements, which share AoSoA cache lines, meet in
@@ -718,30 +589,29 @@ __device__ __forceinline__ int64_t xcd_slot(int64_t count) {
 
 inline unsigned xcd_grid(int64_t count) { return unsigned(8 * ((count + 7) / 8)); }
 
+// Sum over the 256 threads, to all of them.
 __device__ __forceinline__ double block_sum(double v, double *red) {
-    red[threadIdx.x] = v;
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) v += __shfl_xor(v, s);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-    }
-    const double r = red[0];
+    const double r = (red[0] + red[1]) + (red[2] + red[3]);
     __syncthreads();
     return r;
 }
 
 // gout = 2 (out - target) / count; sums[0] += sum (out - target)^2,
-// sums[1] += sum target^2.
+// sums[1] += sum target^2.  At most 256 workgroups: the FP64 atomics on the two
+// sums are serial, 28 us for 2048 of them (262144 values), 8 us now.
 __global__ __launch_bounds__(256) void k_sur_loss(const float *__restrict__ out, const float *__restrict__ tgt,
                                                   float *__restrict__ gout, double *__restrict__ sums, int64_t count) {
-    __shared__ double red[256];
-    const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    __shared__ double red[4];
     double d2 = 0, t2 = 0;
-    if (idx < count) {
+    for (int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x; idx < count; idx += int64_t(gridDim.x) * 256) {
         const float d = out[idx] - tgt[idx];
         gout[idx] = float(2.0 / double(count)) * d;
-        d2 = double(d) * d;
-        t2 = double(tgt[idx]) * tgt[idx];
+        d2 += double(d) * d;
+        t2 += double(tgt[idx]) * tgt[idx];
     }
     const double s0 = block_sum(d2, red);
     const double s1 = block_sum(t2, red);
@@ -771,7 +641,7 @@ __global__ __launch_bounds__(256) void k_sur_gather(int n, double cw, double sca
                                                     int64_t first, const double *__restrict__ rho_in,
                                                     double *__restrict__ rho_out, float *__restrict__ dst,
                                                     int64_t ndof) {
-    __shared__ double red[256];
+    __shared__ double red[4];
     const int64_t b = xcd_slot(ndof);
     if (b >= ndof) return;
     const int64_t dof = first + b;
@@ -808,7 +678,7 @@ __global__ __launch_bounds__(256) void k_sur_finish(int N, double c0, double dc,
                                                     SurGram gm, double *__restrict__ dst, int nupts, int64_t ldim,
                                                     int64_t first, double *__restrict__ defect,
                                                     int32_t *__restrict__ flag, int64_t ndof) {
-    __shared__ double red[256];
+    __shared__ double red[4];
     const int n = N * N * N;
     const int64_t b = xcd_slot(ndof);
     if (b >= ndof) return;
@@ -867,7 +737,7 @@ __global__ __launch_bounds__(256) void k_sur_finish(int N, double c0, double dc,
 __global__ __launch_bounds__(256) void k_sur_cons(int N, double c0, double dc, double cw, SurGram gm, double coef,
                                                   const float *__restrict__ out, float *__restrict__ gout,
                                                   double *__restrict__ sums) {
-    __shared__ double red[256];
+    __shared__ double red[4];
     const int n = N * N * N;
     const int64_t b = blockIdx.x;
     const float *ob = out + b * n;
@@ -1052,6 +922,44 @@ __device__ __forceinline__ float row_sum(float x) {
     return x;
 }
 
+// The y stages of a plane kernel's LDS array Fz[J][zr][c], four waves: from
+// T[yr][zr][c] (a barrier has to follow), and into U[yr][zr][c] (after one).
+template <int N> __device__ __forceinline__ void plane_y_in(const float *__restrict__ tp, float *Fz, int wave, int col, int q) {
+    constexpr int KT = N / 16;
+    for (int u = wave; u < NR * KT; u += 4) {                // Fz[J][zr] = sum_yr beta_yr(J) T[yr][zr]
+        const int zr = u % NR, j0 = u / NR * 16;
+        f32x4 d0 = {0, 0, 0, 0}, d1 = d0;
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            const int yr = q + 4 * s;
+            const float2 t = *reinterpret_cast<const float2 *>(tp + ((yr < NR ? yr : NR - 1) * NR + zr) * SW + 2 * col);
+            const float a = beta<N>(yr, j0 + col);
+            d0 = mfma4(a, t.x, d0);
+            d1 = mfma4(a, t.y, d1);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<float2 *>(Fz + ((j0 + 4 * q + i) * NR + zr) * SW + 2 * col) = make_float2(d0[i], d1[i]);
+    }
+}
+template <int N> __device__ __forceinline__ void plane_y_out(const float *Fz, float *__restrict__ up, int wave, int col, int q) {
+    for (int zr = wave; zr < NR; zr += 4) {                  // U[yr][zr] = sum_J beta_yr(J) Fz[J][zr]
+        f32x4 d0 = {0, 0, 0, 0}, d1 = d0;
+#pragma unroll
+        for (int s = 0; s < N / 4; ++s) {
+            const int J = q + 4 * s;
+            const float2 t = *reinterpret_cast<const float2 *>(Fz + (J * NR + zr) * SW + 2 * col);
+            const float a = beta<N>(col, J);
+            d0 = mfma4(a, t.x, d0);
+            d1 = mfma4(a, t.y, d1);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (4 * q + i < NR)
+                *reinterpret_cast<float2 *>(up + ((4 * q + i) * NR + zr) * SW + 2 * col) = make_float2(d0[i], d1[i]);
+    }
+}
+
 // One plane I of DOF b per workgroup; FIRST: v_1 from g (lw: the folded first
 // layer's A, a0), else v_{l+1} from v_l in place (lw: the layer's Wm, b).
 // LAST: v_{L-1} is not stored; its part of the projection, QW . v + qb, goes
@@ -1067,23 +975,7 @@ __global__ __launch_bounds__(256) void k_fno_plane(const float *__restrict__ T, 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, q = lane >> 4;
     const int64_t plane = blockIdx.x;                        // b * N + I
-    const float *tp = T + plane * (NR2 * SW);
-    // inverse y stage: Fz[J][zr] = sum_yr beta_yr(J) T[yr][zr]
-    for (int u = wave; u < NR * KT; u += 4) {
-        const int zr = u % NR, j0 = u / NR * 16;
-        f32x4 d0 = {0, 0, 0, 0}, d1 = d0;
-#pragma unroll
-        for (int s = 0; s < 3; ++s) {
-            const int yr = q + 4 * s;
-            const float2 t = *reinterpret_cast<const float2 *>(tp + ((yr < NR ? yr : NR - 1) * NR + zr) * SW + 2 * col);
-            const float a = beta<N>(yr, j0 + col);
-            d0 = mfma4(a, t.x, d0);
-            d1 = mfma4(a, t.y, d1);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            *reinterpret_cast<float2 *>(Fz + ((j0 + 4 * q + i) * NR + zr) * SW + 2 * col) = make_float2(d0[i], d1[i]);
-    }
+    plane_y_in<N>(T + plane * (NR2 * SW), Fz, wave, col, q);
     // operands that stay: the channel matrix and bias of this lane's two outputs, the z tables
     float wm[2][FIRST ? 1 : 8], w0[2], b0[2];
 #pragma unroll
@@ -1174,28 +1066,12 @@ __global__ __launch_bounds__(256) void k_fno_plane(const float *__restrict__ T, 
                 *reinterpret_cast<float2 *>(Fz + (J * NR + 4 * q + i) * SW + 2 * col) = make_float2(az0[i], az1[i]);
     }
     __syncthreads();
-    // forward y stage: U[yr][zr] = sum_J beta_yr(J) Fz[J][zr]
-    for (int zr = wave; zr < NR; zr += 4) {
-        f32x4 d0 = {0, 0, 0, 0}, d1 = d0;
-#pragma unroll
-        for (int s = 0; s < N / 4; ++s) {
-            const int J = q + 4 * s;
-            const float2 t = *reinterpret_cast<const float2 *>(Fz + (J * NR + zr) * SW + 2 * col);
-            const float a = beta<N>(col, J);
-            d0 = mfma4(a, t.x, d0);
-            d1 = mfma4(a, t.y, d1);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (4 * q + i < NR)
-                *reinterpret_cast<float2 *>(U + plane * (NR2 * SW) + ((4 * q + i) * NR + zr) * SW + 2 * col) =
-                    make_float2(d0[i], d1[i]);
-    }
+    plane_y_out<N>(Fz, U + plane * (NR2 * SW), wave, col, q);
 }
 
 // x stages, one wave per (b, yr, zr) and 32 channels.
 // FWD: P[b][xr][yz][c] = scale sum_I beta_xr(I) U[b][I][yz][c];
-// else T[b][I][yz][c] = sum_xr beta_xr(I) Q[b][xr][yz][c].
+// else T[b][I][yz][c] = scale sum_xr beta_xr(I) Q[b][xr][yz][c].
 template <int N, bool FWD>
 __global__ __launch_bounds__(256) void k_fno_x(const float *__restrict__ in, float *__restrict__ out, float scale,
                                                int64_t units) {
@@ -1240,7 +1116,7 @@ __global__ __launch_bounds__(256) void k_fno_x(const float *__restrict__ in, flo
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                *reinterpret_cast<float2 *>(o + (16 * k + 4 * q + i) * NR2 * SW) = make_float2(d0[i], d1[i]);
+                *reinterpret_cast<float2 *>(o + (16 * k + 4 * q + i) * NR2 * SW) = make_float2(scale * d0[i], scale * d1[i]);
         }
     }
 }
@@ -1291,81 +1167,142 @@ __device__ __forceinline__ void cls_fold(float *Q, float yr, float yi, const flo
     Q[7] += s[0] * s[1] * s[2] * yi;
 }
 
-// Q = fold(X R) for the modes of class blockIdx.x and the 64 DOFs from
-// 64 * blockIdx.y, sixteen per wave.  The class's weights (up to 8 modes,
-// 64 KB) are staged in LDS; row rho of a mode holds input channel
-// i = 8 (rho % 4) + rho / 4, so the four lane groups read neighbouring rows.
-__global__ __launch_bounds__(256) void k_fno_mix(const float *__restrict__ P, const float2 *__restrict__ R,
-                                                 float *__restrict__ Q, int batch) {
-    __shared__ float Rl[8][2][SW * SW];
-    const int cls = blockIdx.x, tid = threadIdx.x, lane = tid & 63, col = lane & 15, q = lane >> 4;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    for (int e = tid; e < SW * SW; e += 256) {
-        const int i = e / SW, o = e % SW, rho = (i % 8) * 4 + i / 8;
+// Packed weights: mode k's matrix as 1024 complex values in the order in which
+// k_fno_mix stages it, a half of the output channels o after the other, row rho
+// = 4 (i % 8) + i / 8 of input channel i (the four lane groups then read
+// neighbouring rows, each 32 LDS banks).  In theta a mode's weights are 4096
+// bytes apart, 8 of 64 or 128 bytes fetched are used.
+constexpr int kPack = SW * SW * SM3;                     // complex values of a layer
+constexpr int kHalf = SW * SW / 2;
+__device__ __forceinline__ int stage_at(int i, int o) {
+    const int rho = (i % 8) * 4 + i / 8;
+    return o / 16 * kHalf + rho * 16 + o % 16;
+}
+
+// Rp = packed R of the layers blockIdx.z (R: the first layer's, layers stride
+// complex values apart); ADJ: of conj(R)^T.  64 (i, o) x 64 modes through LDS.
+template <bool ADJ>
+__global__ __launch_bounds__(256) void k_fno_pack(const float *__restrict__ R, int64_t stride, float2 *__restrict__ Rp) {
+    __shared__ float2 tile[64][65];
+    const int t = threadIdx.x, k0 = blockIdx.y * 64;
+    const float2 *src = reinterpret_cast<const float2 *>(R + blockIdx.z * stride);
+    float2 *dst = Rp + int64_t(blockIdx.z) * kPack;
+    const int row = 2 * blockIdx.x;                          // two rows of the packed matrix, 32 columns
 #pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            float sg[3];
-            const int k = cls_mode(cls, m, sg);
-            if (k < 0) continue;
-            const float2 r = R[int64_t(e) * SM3 + k];
-            Rl[m][0][rho * SW + o] = r.x;
-            Rl[m][1][rho * SW + o] = r.y;
-        }
+    for (int j = 0; j < 16; ++j) {
+        const int e = (t >> 6) + 4 * j, i = ADJ ? e % SW : row + e / SW, o = ADJ ? row + e / SW : e % SW;
+        tile[e][t & 63] = src[int64_t(i * SW + o) * SM3 + k0 + (t & 63)];
     }
     __syncthreads();
-    const int b0 = blockIdx.y * 64 + wave * 16;
-    if (b0 >= batch) return;                             // no barrier follows
-    const int bl = b0 + col < batch ? b0 + col : batch - 1;
-    float p[8][8];                                       // [coefficient][s], input channel 8 q + s
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int at = cls_coef(cls, e);
-#pragma unroll
-        for (int s = 0; s < 8; ++s) p[e][s] = 0.f;
-        if (at >= 0) ld8(P + (int64_t(bl) * NR3 + at) * SW + 8 * q, p[e]);
+    for (int j = 0; j < 16; ++j) {
+        const int e = t & 63, k = (t >> 6) + 4 * j;
+        const float2 r = tile[e][k];
+        dst[int64_t(k0 + k) * (SW * SW) + stage_at(row + e / SW, e % SW)] = make_float2(r.x, ADJ ? -r.y : r.y);
     }
-    float acc[2][4][8];                                  // [tile][row][coefficient]
+}
+
+// gR += the modes-first gradient g[k][i * 32 + o] of the layers blockIdx.z.
+__global__ __launch_bounds__(256) void k_fnt_unpack(const float2 *__restrict__ g, int64_t stride, float *__restrict__ gR) {
+    __shared__ float2 tile[64][65];
+    const int t = threadIdx.x, k0 = blockIdx.y * 64, e0 = blockIdx.x * 64;
+    const float2 *src = g + int64_t(blockIdx.z) * kPack;
+    float2 *dst = reinterpret_cast<float2 *>(gR + blockIdx.z * stride);
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int j = 0; j < 16; ++j) {
+        const int k = (t >> 6) + 4 * j;
+        tile[k][t & 63] = src[int64_t(k0 + k) * (SW * SW) + e0 + (t & 63)];
+    }
+    __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < 16; ++j) {
+        const int e = (t >> 6) + 4 * j;
+        const int64_t at = int64_t(e0 + e) * SM3 + k0 + (t & 63);
+        const float2 r = tile[t & 63][e], w = dst[at];
+        dst[at] = make_float2(w.x + r.x, w.y + r.y);
+    }
+}
+
+// Q = fold(X R) for the modes of class blockIdx.x, the output channels o = 16
+// blockIdx.z + col and 64 DOFs at a time (blockIdx.y, then by gridDim.y), sixteen
+// per wave.  The class's weights (up to 8 modes, 32 KB) are staged in LDS, from
+// the packed ones or (PACKED false, where there is no room for those) from
+// theta.  ADJ: conj(R)^T in place of R, the backward product (P = gQ, Q = gP).
+// Bound by the matrix instructions of the classes with 8 modes, 32 of 32 cycles
+// per mode, wave and tile: 64 DOFs 24 us with both halves in one workgroup (125
+// of them), 14 us now; 4096 DOFs 773 -> 645.
+template <bool ADJ, bool PACKED>
+__global__ __launch_bounds__(256) void k_fno_mix(const float *__restrict__ P, const float2 *__restrict__ R,
+                                                 float *__restrict__ Q, int batch) {
+    __shared__ float2 Rl[8][kHalf];
+    const int cls = blockIdx.x, half = blockIdx.z, tid = threadIdx.x, lane = tid & 63, col = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    {
+        constexpr int E = kHalf / 256;
+        float2 r[E][8];                                  // all loads in flight, then the LDS stores
 #pragma unroll
-            for (int e = 0; e < 8; ++e) acc[t][i][e] = 0.f;
+        for (int j = 0; j < E; ++j)
+#pragma unroll
+            for (int m = 0; m < 8; ++m) {
+                float sg[3];
+                const int k = cls_mode(cls, m, sg), e = tid + 256 * j, rho = e / 16;
+                r[j][m] = make_float2(0.f, 0.f);
+                if (k < 0) continue;
+                const int i = rho % 4 * 8 + rho / 4, o = 16 * half + e % 16;
+                if constexpr (PACKED) r[j][m] = R[int64_t(k) * (SW * SW) + half * kHalf + e];
+                else r[j][m] = R[int64_t(ADJ ? o * SW + i : i * SW + o) * SM3 + k];
+            }
+#pragma unroll
+        for (int j = 0; j < E; ++j)
+#pragma unroll
+            for (int m = 0; m < 8; ++m)
+                Rl[m][tid + 256 * j] = make_float2(r[j][m].x, ADJ && !PACKED ? -r[j][m].y : r[j][m].y);
+    }
+    __syncthreads();
+    const int o = 16 * half + col, ro = q * 16 + col;
 #pragma unroll 1
-    for (int m = 0; m < 8; ++m) {
-        float sg[3];
-        if (cls_mode(cls, m, sg) < 0) continue;
-        f32x4 yr[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, yi[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
-#pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            const float pe[8] = {p[0][s], p[1][s], p[2][s], p[3][s], p[4][s], p[5][s], p[6][s], p[7][s]};
-            const float2 x = cls_x(pe, sg);
-            const float2 rr = *reinterpret_cast<const float2 *>(&Rl[m][0][(4 * s + q) * SW + 2 * col]);
-            const float2 ri = *reinterpret_cast<const float2 *>(&Rl[m][1][(4 * s + q) * SW + 2 * col]);
-            yr[0] = mfma4(x.x, rr.x, yr[0]);
-            yr[1] = mfma4(x.x, rr.y, yr[1]);
-            yr[0] = mfma4(-x.y, ri.x, yr[0]);
-            yr[1] = mfma4(-x.y, ri.y, yr[1]);
-            yi[0] = mfma4(x.x, ri.x, yi[0]);
-            yi[1] = mfma4(x.x, ri.y, yi[1]);
-            yi[0] = mfma4(x.y, rr.x, yi[0]);
-            yi[1] = mfma4(x.y, rr.y, yi[1]);
-        }
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) cls_fold(acc[t][i], yr[t][i], yi[t][i], sg);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int b = b0 + 4 * q + i;
-        if (b >= batch) continue;
+    for (int b0 = blockIdx.y * 64 + wave * 16; b0 < batch; b0 += gridDim.y * 64) {   // no barrier inside
+        const int bl = b0 + col < batch ? b0 + col : batch - 1;
+        float p[8][8];                                   // [coefficient][s], input channel 8 q + s
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int at = cls_coef(cls, e);
-            if (at >= 0)
-                *reinterpret_cast<float2 *>(Q + (int64_t(b) * NR3 + at) * SW + 2 * col) =
-                    make_float2(acc[0][i][e], acc[1][i][e]);
+#pragma unroll
+            for (int s = 0; s < 8; ++s) p[e][s] = 0.f;
+            if (at >= 0) ld8(P + (int64_t(bl) * NR3 + at) * SW + 8 * q, p[e]);
+        }
+        float acc[4][8];                                 // [row][coefficient]
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[i][e] = 0.f;
+#pragma unroll 1
+        for (int m = 0; m < 8; ++m) {
+            float sg[3];
+            if (cls_mode(cls, m, sg) < 0) continue;
+            f32x4 yr[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, yi[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const float pe[8] = {p[0][s], p[1][s], p[2][s], p[3][s], p[4][s], p[5][s], p[6][s], p[7][s]};
+                const float2 x = cls_x(pe, sg);
+                const float2 r = Rl[m][4 * s * 16 + ro];
+                yr[0] = mfma4(x.x, r.x, yr[0]);
+                yi[0] = mfma4(x.x, r.y, yi[0]);
+                yr[1] = mfma4(-x.y, r.y, yr[1]);
+                yi[1] = mfma4(x.y, r.x, yi[1]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) cls_fold(acc[i], yr[0][i] + yr[1][i], yi[0][i] + yi[1][i], sg);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int b = b0 + 4 * q + i;
+            if (b >= batch) continue;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int at = cls_coef(cls, e);
+                if (at >= 0) Q[(int64_t(b) * NR3 + at) * SW + o] = acc[i][e];
+            }
         }
     }
 }
@@ -1437,7 +1374,376 @@ __global__ __launch_bounds__(256) void k_fno_add(const float *__restrict__ s1, f
     if (idx < pts) out[idx] += s1[idx];
 }
 
+// ---------------------------------------------------------------------------
+// The gradients on the same transforms.
+//
+// With V the (real) analysis of all three axes, s = V^T Q and P = V v, so the
+// backward pass runs the forward transforms on gz_l = dLoss/dz_l: gQ = V gz_l,
+// and gv_l gains V^T gP; in the modes gX = gY conj(R)^T and gR = sum_b conj(X)
+// gY, with the 1/n of the analysis on X and on gX.  v_l is taken as
+// gelu(z_{l-1}), or the lift of g, where it is needed.
+//   k_fnt_top    coefficients of gz_{L-1} = Qw gout, and dQw
+//   k_fnt_back   from gz_l and T: dWm, db, gv_l, then gz_{l-1} and its U, or
+//                the lift's gradients; gz_{l-1} takes the place of gz_l
+//   k_fnt_sum    adds the planes' weight gradients
+// gz is [b][x][c]; z and X are the forward pass's, [b][c][x] and [b][c][k].
+// A layer reads gz_l and z_{l-1} and writes gz_{l-1}, three streams of the
+// activations (15 with a kernel per product and transform), and its matrix
+// instructions, 46 for 16 points, and 8 gelu and gelu' per lane take about as
+// long.  A plane's weight gradients stay in registers, and the sums over planes
+// are taken from one partial per plane, not with an atomic per plane and weight.
+// 64 rows on 16^3, 4 layers: forward and backward 1467 us, 732 us now; the
+// backward kernels of one layer 226 -> 74 us (k_fnt_back 33, k_fno_mix 14,
+// k_fnt_mix_grad 15, k_fno_x 12).  Error of the gradient against 64 bits 2.5e-7
+// -> 1.3e-7.  The forward pass in training keeps its kernels and their rounding.
+// ---------------------------------------------------------------------------
+constexpr int kPart = SW * SW + 3 * SW;      // partials of a plane: dWm, db, dP, dp0
+constexpr int kPart0 = 2 * SW;               // and of the start: dQw, dq0 (the rest unused)
+
+// Sum of a lane's value over the four lane groups.
+__device__ __forceinline__ float group_sum(float x) {
+    x += __shfl_xor(x, 16);
+    return x + __shfl_xor(x, 32);
+}
+
+// z [b][c][x] at four neighbouring points, channels c and c + 1 (p: channel c).
+template <int N, typename TA> __device__ __forceinline__ void ld4x2(const TA *p, float2 *v) {
+    struct alignas(4 * sizeof(TA)) Four { TA v[4]; };
+    const Four a = *reinterpret_cast<const Four *>(p), b = *reinterpret_cast<const Four *>(p + SG<N>::N3);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = make_float2(float(a.v[i]), float(b.v[i]));
+}
+
+// One plane of gz_{L-1} = Qw gout: its coefficients U, and the plane's sums of
+// gout z_{L-1} (dQw) and gout (dq0).
+template <int N, typename TA>
+__global__ __launch_bounds__(256) void k_fnt_top(const float *__restrict__ gout, const float *__restrict__ qw,
+                                                 const TA *__restrict__ z, float *__restrict__ U,
+                                                 float *__restrict__ part) {
+    constexpr int KT = N / 16;
+    __shared__ float Fz[N * NR * SW];
+    const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t plane = blockIdx.x;
+    const TA *zp = z + (plane / N * SW + 2 * col) * SG<N>::N3 + plane % N * SG<N>::N2;
+    const float w0 = qw[2 * col], w1 = qw[2 * col + 1];
+    float ef[KT][4];
+#pragma unroll
+    for (int k = 0; k < KT; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ef[k][i] = beta<N>(col, 16 * k + 4 * q + i);
+    float s0 = 0.f, s1 = 0.f, sg = 0.f;
+    for (int J = wave; J < N; J += 4) {
+        f32x4 az0 = {0, 0, 0, 0}, az1 = az0;
+#pragma unroll
+        for (int k = 0; k < KT; ++k) {
+            const int at = J * N + 16 * k + 4 * q;
+            float2 zz[4];
+            ld4x2<N>(zp + at, zz);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float v = gout[plane * SG<N>::N2 + at + i];
+                s0 += v * zz[i].x;
+                s1 += v * zz[i].y;
+                sg += v;
+                az0 = mfma4(ef[k][i], w0 * v, az0);
+                az1 = mfma4(ef[k][i], w1 * v, az1);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (4 * q + i < NR)
+                *reinterpret_cast<float2 *>(Fz + (J * NR + 4 * q + i) * SW + 2 * col) = make_float2(az0[i], az1[i]);
+    }
+    __syncthreads();
+    plane_y_out<N>(Fz, U + plane * (NR2 * SW), wave, col, q);
+    __syncthreads();
+    s0 = group_sum(s0);
+    s1 = group_sum(s1);
+    sg = group_sum(sg);
+    if (q == 0) {
+        *reinterpret_cast<float2 *>(Fz + wave * kPart0 + 2 * col) = make_float2(s0, s1);
+        if (col == 0) Fz[wave * kPart0 + SW] = sg;
+    }
+    __syncthreads();
+    if (tid <= SW)
+        part[plane * kPart0 + tid] = (Fz[tid] + Fz[kPart0 + tid]) + (Fz[2 * kPart0 + tid] + Fz[3 * kPart0 + tid]);
+}
+
+// One plane of layer l backward.  gz_l: Qw gout (TOP) or from gz; v_l: the lift
+// of g (BOT) or gelu(z_{l-1}) (zin).  part: this plane's dWm = gz_l v_l^T and
+// db = gz_l, and for BOT the lift's gradients.  Otherwise gz_{l-1} =
+// (Wm^T gz_l + s) gelu'(z_{l-1}) is written to gz and its coefficients to U.
+template <int N, typename TA, bool TOP, bool BOT>
+__global__ __launch_bounds__(256) void k_fnt_back(const float *__restrict__ T, const float *__restrict__ g,
+                                                  const float *__restrict__ gout, const float *__restrict__ th,
+                                                  const float *__restrict__ lw, const float *__restrict__ qw,
+                                                  const TA *__restrict__ zin, float *gz, float *__restrict__ U,
+                                                  float *__restrict__ part) {
+    constexpr int KT = N / 16;
+    __shared__ float Fz[N * NR * SW];
+    static_assert(N * NR * SW >= 4 * kPart, "the waves' partials fit");
+    const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t plane = blockIdx.x;
+    plane_y_in<N>(T + plane * (NR2 * SW), Fz, wave, col, q);
+    const TA *zp = zin + (plane / N * SW + 2 * col) * SG<N>::N3 + plane % N * SG<N>::N2;
+    float wm[2][8], qa[TOP ? 8 : 1];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        wm[0][s] = lw[(8 * q + s) * SW + 2 * col];
+        wm[1][s] = lw[(8 * q + s) * SW + 2 * col + 1];
+        if constexpr (TOP) qa[s] = qw[8 * q + s];
+    }
+    float qw0 = 0.f, qw1 = 0.f, p0 = 0.f, p1 = 0.f, c0 = 0.f, c1 = 0.f;
+    if constexpr (TOP) { qw0 = qw[2 * col]; qw1 = qw[2 * col + 1]; }
+    if constexpr (BOT) { p0 = th[2 * col]; p1 = th[2 * col + 1]; c0 = th[SW + 2 * col]; c1 = th[SW + 2 * col + 1]; }
+    float ez[KT][3], ef[KT][4];
+#pragma unroll
+    for (int k = 0; k < KT; ++k) {
+#pragma unroll
+        for (int s = 0; s < 3; ++s) ez[k][s] = beta<N>(q + 4 * s, 16 * k + col);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ef[k][i] = beta<N>(col, 16 * k + 4 * q + i);
+    }
+    f32x4 dw[2][2] = {{{0, 0, 0, 0}, {0, 0, 0, 0}}, {{0, 0, 0, 0}, {0, 0, 0, 0}}};   // [o parity][i parity]
+    float db0 = 0.f, db1 = 0.f, dp0 = 0.f, dp1 = 0.f, dc0 = 0.f, dc1 = 0.f;
+    __syncthreads();
+    for (int J = wave; J < N; J += 4) {
+        const int64_t row = (plane * N + J) * N;
+        float2 f[3];
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            const int zr = q + 4 * s;
+            f[s] = *reinterpret_cast<const float2 *>(Fz + (J * NR + (zr < NR ? zr : NR - 1)) * SW + 2 * col);
+        }
+        f32x4 az0 = {0, 0, 0, 0}, az1 = az0;
+#pragma unroll
+        for (int k = 0; k < KT; ++k) {
+            const int64_t pt = row + 16 * k;
+            float a[8], gv[4];
+            float2 gd[4], zd[4];                             // gz_l and z_{l-1} of points 4 q + i, channels 2 col, + 1
+            if constexpr (TOP) {
+                const float go = gout[pt + col];
+#pragma unroll
+                for (int s = 0; s < 8; ++s) a[s] = qa[s] * go;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float gi = gout[pt + 4 * q + i];
+                    gd[i] = make_float2(qw0 * gi, qw1 * gi);
+                }
+            } else {
+                ld8(gz + (pt + col) * SW + 8 * q, a);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) gd[i] = ld2(gz, (pt + 4 * q + i) * SW + 2 * col);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (BOT) gv[i] = g[pt + 4 * q + i];
+            }
+            if constexpr (!BOT) ld4x2<N>(zp + J * N + 16 * k + 4 * q, zd);
+            f32x4 d0 = {0, 0, 0, 0}, d1 = d0;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                d0 = mfma4(a[s], wm[0][s], d0);
+                d1 = mfma4(a[s], wm[1][s], d1);
+            }
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+                d0 = mfma4(ez[k][s], f[s].x, d0);
+                d1 = mfma4(ez[k][s], f[s].y, d1);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float v0, v1;
+                if constexpr (BOT) {
+                    v0 = p0 * gv[i] + c0;
+                    v1 = p1 * gv[i] + c1;
+                    dp0 += d0[i] * gv[i];
+                    dp1 += d1[i] * gv[i];
+                    dc0 += d0[i];
+                    dc1 += d1[i];
+                } else {
+                    const float2 e0 = gelu_both(zd[i].x), e1 = gelu_both(zd[i].y);
+                    v0 = e0.x;
+                    v1 = e1.x;
+                    const float x0 = d0[i] * e0.y, x1 = d1[i] * e1.y;
+                    *reinterpret_cast<float2 *>(gz + (pt + 4 * q + i) * SW + 2 * col) = make_float2(x0, x1);
+                    az0 = mfma4(ef[k][i], x0, az0);
+                    az1 = mfma4(ef[k][i], x1, az1);
+                }
+                dw[0][0] = mfma4(gd[i].x, v0, dw[0][0]);
+                dw[0][1] = mfma4(gd[i].x, v1, dw[0][1]);
+                dw[1][0] = mfma4(gd[i].y, v0, dw[1][0]);
+                dw[1][1] = mfma4(gd[i].y, v1, dw[1][1]);
+                db0 += gd[i].x;
+                db1 += gd[i].y;
+            }
+        }
+        if constexpr (!BOT) {
+            // the row's coefficients take the place of the ones just read (same wave, LDS in order)
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (4 * q + i < NR)
+                    *reinterpret_cast<float2 *>(Fz + (J * NR + 4 * q + i) * SW + 2 * col) = make_float2(az0[i], az1[i]);
+        }
+    }
+    __syncthreads();
+    if constexpr (!BOT) {
+        plane_y_out<N>(Fz, U + plane * (NR2 * SW), wave, col, q);
+        __syncthreads();
+    }
+    float *mine = Fz + wave * kPart;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            *reinterpret_cast<float2 *>(mine + (2 * (4 * q + r) + t) * SW + 2 * col) = make_float2(dw[t][0][r], dw[t][1][r]);
+    float *tail = mine + SW * SW;
+    db0 = group_sum(db0);
+    db1 = group_sum(db1);
+    if (q == 0) *reinterpret_cast<float2 *>(tail + 2 * col) = make_float2(db0, db1);
+    if constexpr (BOT) {
+        dp0 = group_sum(dp0);
+        dp1 = group_sum(dp1);
+        dc0 = group_sum(dc0);
+        dc1 = group_sum(dc1);
+        if (q == 0) {
+            *reinterpret_cast<float2 *>(tail + SW + 2 * col) = make_float2(dp0, dp1);
+            *reinterpret_cast<float2 *>(tail + 2 * SW + 2 * col) = make_float2(dc0, dc1);
+        }
+    }
+    __syncthreads();
+    for (int j = tid; j < (BOT ? kPart : SW * SW + SW); j += 256)
+        part[plane * kPart + j] = (Fz[j] + Fz[kPart + j]) + (Fz[2 * kPart + j] + Fz[3 * kPart + j]);
+}
+
+// grad[to + j] += sum over the planes of part[plane][j], for each of the L + 2
+// blocks blockIdx.z: the layers' dWm and db, the lift's and the projection's
+// gradients.  64 columns and 64 planes per workgroup; one launch for all.
+__global__ __launch_bounds__(256) void k_fnt_sum(const float *__restrict__ part, const float *__restrict__ part0, int L,
+                                                 int64_t planes, float *__restrict__ grad) {
+    __shared__ float red[256];
+    const int t = threadIdx.x, j = blockIdx.x * 64 + (t & 63), z = blockIdx.z;
+    const float *from = part + int64_t(z < L ? z : 0) * planes * kPart + (z == L ? SW * SW + SW : 0);
+    int stride = kPart, cols = z < L ? SW * SW + SW : 2 * SW;
+    float *to = z < L ? grad + 2 * SW + z * SLAYER + SR : grad;
+    if (z == L + 1) {
+        from = part0;
+        stride = kPart0;
+        cols = SW + 1;
+        to = grad + 2 * SW + L * SLAYER;
+    }
+    const int64_t r0 = int64_t(blockIdx.y) * 64 + (t >> 6);
+    if (int(blockIdx.x) * 64 >= cols) return;                // uniform
+    float s = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        const int64_t r = r0 + 4 * k;
+        if (j < cols && r < planes) s += from[r * stride + j];
+    }
+    red[t] = s;
+    __syncthreads();
+    if (t < 64 && j < cols) atomicAdd(&to[j], (red[t] + red[t + 64]) + (red[t + 128] + red[t + 192]));
+}
+
+// Xt[k][r] = X[r][k] of the layers blockIdx.z (rows r = (b, c), cols a multiple
+// of 64), 64 x 64 through LDS.
+__global__ __launch_bounds__(256) void k_fnt_modes(const float2 *__restrict__ X, float2 *__restrict__ Xt, int64_t rows) {
+    __shared__ float2 tile[64][65];
+    const int t = threadIdx.x, k0 = blockIdx.y * 64;
+    const int64_t r0 = int64_t(blockIdx.x) * 64, base = int64_t(blockIdx.z) * rows * SM3;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const int64_t r = r0 + (t >> 6) + 4 * j;
+        if (r < rows) tile[(t >> 6) + 4 * j][t & 63] = X[base + r * SM3 + k0 + (t & 63)];
+    }
+    __syncthreads();
+    if (r0 + (t & 63) >= rows) return;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const int k = (t >> 6) + 4 * j;
+        Xt[base + (k0 + k) * rows + r0 + (t & 63)] = tile[t & 63][k];
+    }
+}
+
+// gR(i,o,k) = sum_b conj X(b,i,k) gY(b,o,k) for the modes of class blockIdx.x,
+// one mode per wave, and the input channels i = 16 blockIdx.y + col, from Xt[k][b][i] and the coefficients gQ of gz.  The DOFs
+// are the inner dimension of the product.  Stored modes first (PACKED:
+// gR[k][i * 32 + o]), or added into the gradient.
+template <bool PACKED>
+__global__ __launch_bounds__(512) void k_fnt_mix_grad(const float2 *__restrict__ Xt, const float *__restrict__ gQ,
+                                                      float2 *__restrict__ gR, int batch) {
+    const int cls = blockIdx.x, lane = threadIdx.x & 63, col = lane & 15, q = lane >> 4;
+    float sg[3];
+    const int k = cls_mode(cls, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), sg);
+    if (k < 0) return;                                       // no barrier in this kernel
+    int at[8];
+    float has[8];                                            // 0 where the class has no such coefficient
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int c = cls_coef(cls, e);
+        at[e] = (c < 0 ? 0 : c) * SW + 2 * col;
+        has[e] = c < 0 ? 0.f : 1.f;
+    }
+    const float2 *xk = Xt + int64_t(k) * batch * SW + 16 * blockIdx.y + col;
+    f32x4 re[2][2], im[2][2];                                // [o parity][term]
+#pragma unroll
+    for (int t = 0; t < 4; ++t) re[t >> 1][t & 1] = im[t >> 1][t & 1] = {0, 0, 0, 0};
+#pragma unroll 4
+    for (int b0 = 0; b0 < batch; b0 += 4) {
+        const int b = b0 + q, bl = b < batch ? b : batch - 1;
+        const bool live = b < batch;
+        float py[2][8];
+        float2 X = xk[int64_t(bl) * SW];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float2 y = *reinterpret_cast<const float2 *>(gQ + int64_t(bl) * (NR3 * SW) + at[e]);
+            py[0][e] = has[e] != 0.f ? y.x : 0.f;
+            py[1][e] = has[e] != 0.f ? y.y : 0.f;
+        }
+        float2 Y[2] = {cls_x(py[0], sg), cls_x(py[1], sg)};
+        if (!live) X = Y[0] = Y[1] = make_float2(0.f, 0.f);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            re[u][0] = mfma4(X.x, Y[u].x, re[u][0]);
+            re[u][1] = mfma4(X.y, Y[u].y, re[u][1]);
+            im[u][0] = mfma4(X.x, Y[u].y, im[u][0]);
+            im[u][1] = mfma4(-X.y, Y[u].x, im[u][1]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int i = 16 * blockIdx.y + 4 * q + r;
+        float w[4];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            w[2 * u] = re[u][0][r] + re[u][1][r];
+            w[2 * u + 1] = im[u][0][r] + im[u][1][r];
+        }
+        if constexpr (PACKED) {
+            *reinterpret_cast<f32x4 *>(gR + int64_t(k) * (SW * SW) + i * SW + 2 * col) = f32x4{w[0], w[1], w[2], w[3]};
+        } else {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                float2 *p = gR + int64_t(i * SW + 2 * col + u) * SM3 + k;
+                const float2 old = *p;
+                *p = make_float2(old.x + w[2 * u], old.y + w[2 * u + 1]);
+            }
+        }
+    }
+}
+
 inline unsigned nblk(int64_t n) { return unsigned((n + 255) / 256); }
+
+// Workgroups of k_fno_mix: 64 DOFs each, but more of them per staged class
+// beyond 16 * 64 DOFs (the chip is full by then).
+inline dim3 mix_grid(int64_t batch) {
+    const int64_t t = (batch + 63) / 64;
+    return dim3(125, unsigned(t < 16 ? t : 16), 2);
+}
 
 int check_shape(const fq_sur_shape *s, const char *who) {
     if (!s) return fq_internal_fail(FQ_ERR_INVALID, std::string(who) + ": null shape");
@@ -1493,6 +1799,21 @@ ActPtrs act_ptrs(int N3, float *acts, int L, int64_t B, bool training) {
     return p;
 }
 
+// Room for n layers' packed weights between `from` and `end` (floats), 16-byte
+// aligned as the arrays before them are, or null: few DOFs (16^3: fewer than 9
+// in training, 6 in inference) leave none, and read theta in place.
+inline float2 *pack_room(float *from, float *end, int n) {
+    float *at = from + (-(reinterpret_cast<uintptr_t>(from) / sizeof(float)) & 3);
+    return end - at >= 2LL * n * kPack ? reinterpret_cast<float2 *>(at) : nullptr;
+}
+template <bool ADJ> void pack(const float *R, int layers, float2 *Rp, hipStream_t st) {
+    hipLaunchKernelGGL(k_fno_pack<ADJ>, dim3(16, 8, layers), dim3(256), 0, st, R, SLAYER, Rp);
+}
+template <bool ADJ> void mix(const float *P, const float *R, const float2 *Rp, float *Q, int64_t batch, hipStream_t st) {
+    hipLaunchKernelGGL((Rp ? k_fno_mix<ADJ, true> : k_fno_mix<ADJ, false>), mix_grid(batch), dim3(256), 0, st, P,
+                       Rp ? Rp : reinterpret_cast<const float2 *>(R), Q, int(batch));
+}
+
 // The folded inference pass with activations stored as A (FP32 or 16 bits),
 // in the inference activation space: v [b][x][c], then T and U
 // [b][I][yr][zr][c], P and Q [b][xr][yr][zr][c], the one-channel modes X and
@@ -1508,6 +1829,7 @@ void forward_fused(int L, const float *theta, const float *fused, const float *g
     float *s1 = Q + pq + 2 * batch * SM3;
     static_assert(int64_t(SW) * N3 + 2 * N * NR2 * SW + 2 * NR3 * SW + 2 * SM3 + N3 <=
                   3LL * SW * N3 + 4 * SW * SM3, "fits the inference activation space");
+    float2 *Rp = pack_room(s1 + batch * N3, acts + act_floats(N3, L, batch, false), 1);
     const int64_t pts = batch * N3, xu = batch * NR2;
     const dim3 blk(256), pg(unsigned(batch * N)), xg(unsigned((xu + 3) / 4));
     // first layer from the one-channel transform of g
@@ -1519,8 +1841,8 @@ void forward_fused(int L, const float *theta, const float *fused, const float *g
     for (int l = 1; l < L - 1; ++l) {
         const float *lay = theta + 2 * SW + l * SLAYER;
         hipLaunchKernelGGL((k_fno_x<N, true>), xg, blk, 0, st, U, P, 1.0f / N3, xu);
-        hipLaunchKernelGGL(k_fno_mix, dim3(125, unsigned((batch + 63) / 64)), blk, 0, st, P,
-                           reinterpret_cast<const float2 *>(lay), Q, int(batch));
+        if (Rp) pack<false>(lay, 1, Rp, st);
+        mix<false>(P, lay, Rp, Q, batch, st);
         hipLaunchKernelGGL((k_fno_x<N, false>), xg, blk, 0, st, Q, T, 1.0f, xu);
         hipLaunchKernelGGL((l == L - 2 ? k_fno_plane<N, A, false, true> : k_fno_plane<N, A, false, false>), pg, blk, 0,
                            st, T, g, lay + SR, v, U, fused + FQW, out);
@@ -1528,7 +1850,7 @@ void forward_fused(int L, const float *theta, const float *fused, const float *g
     // last layer and projection as one output channel
     hipLaunchKernelGGL((k_fno_x<N, true>), xg, blk, 0, st, U, P, 1.0f / N3, xu);
     hipLaunchKernelGGL(k_fno_last, dim3(unsigned((batch * 125 + 7) / 8)), blk, 0, st, P, fused, X, batch * 125);
-    launch_idft<N, float>(X, 1.0f, 0, s1, unsigned(batch), st);
+    launch_idft<N, float>(X, s1, unsigned(batch), st);
     hipLaunchKernelGGL(k_fno_add, dim3(nblk(pts)), blk, 0, st, s1, out, pts);
 }
 
@@ -1547,9 +1869,9 @@ void forward_impl(int L, const float *theta, const float *g, int64_t batch, bool
         const float2 *R = reinterpret_cast<const float2 *>(lay);
         A *vl = reinterpret_cast<A *>(p.v[l]), *vn = reinterpret_cast<A *>(p.v[l + 1]);
         launch_dft<N, A>(vl, 1.0f / SG<N>::N3, p.X[l], slices, st);
-        hipLaunchKernelGGL(k_sur_mix_lds<0>, dim3(SM3 / 8, unsigned((batch + 31) / 32)), dim3(256), 0, st, p.X[l],
+        hipLaunchKernelGGL(k_sur_mix_lds, dim3(SM3 / 8, unsigned((batch + 15) / 16)), dim3(256), 0, st, p.X[l],
                            R, p.Y, batch);
-        launch_idft<N, A>(p.Y, 1.0f, 0, sa, slices, st);
+        launch_idft<N, A>(p.Y, sa, slices, st);
         hipLaunchKernelGGL((k_sur_pw<N, A>), dim3(nblk(pts / 2)), dim3(256), 0, st, vl, sa, lay + SR, int(l < L - 1),
                            tr ? reinterpret_cast<A *>(p.z[l]) : nullptr, vn, pts);
     }
@@ -1558,40 +1880,44 @@ void forward_impl(int L, const float *theta, const float *g, int64_t batch, bool
 }
 
 // Gradients from the activations of a training forward_impl<A>; the
-// gradients themselves (gv, gz, the mode arrays) stay FP32.
+// gradients themselves (gz, the coefficient arrays) stay FP32.  work: gz, then
+// T, U, gQ and gP.  The backward pass does not read the v_l; their place takes
+// the planes' partial sums, the transposed X_l and the packed weights.
 template <int N, typename A>
 void backward_impl(int L, const float *theta, const float *g, int64_t batch, float *acts, const float *gout,
                    float *grad, float *work, hipStream_t st) {
+    constexpr int64_t V = int64_t(SW) * SG<N>::N3, TP = int64_t(N) * NR2 * SW, PQ = int64_t(NR3) * SW, MD = 2LL * SW * SM3;
+    static_assert(2 * TP + 2 * PQ <= V + 2 * MD, "fits the work size");
+    static_assert(N * kPart0 <= V && MD + N * kPart <= V, "the partial sums and X fit in place of v");
     const ActPtrs p = act_ptrs(SG<N>::N3, acts, L, batch, true);
-    const int64_t pts = batch * SG<N>::N3, vol = batch * SW * SG<N>::N3;
-    const unsigned slices = unsigned(batch * SW);
-    float *gv = work, *gvin = work + vol;
-    float2 *gY = reinterpret_cast<float2 *>(work + 2 * vol);
-    float2 *gX = gY + batch * SW * SM3;
-    const dim3 wg(unsigned(batch * (SG<N>::N3 / 512)));
-    const int64_t qoff = 2 * SW + L * SLAYER;
-    hipLaunchKernelGGL((k_sur_wgrad<N, 1, SW, A>), wg, dim3(256), 0, st, gout, reinterpret_cast<const A *>(p.v[L]),
-                       grad + qoff, grad + qoff + SW);
-    hipLaunchKernelGGL(k_sur_proj_bwd<N>, dim3(nblk(pts)), dim3(256), 0, st, gout, theta + qoff, gv, pts);
+    float *gz = work, *T = gz + batch * V, *U = T + batch * TP, *gQ = U + batch * TP, *gP = gQ + batch * PQ;
+    float2 *Xt = reinterpret_cast<float2 *>(p.v[0]);
+    float *part = p.v[0] + L * batch * MD, *part0 = part + int64_t(L) * batch * N * kPart;
+    // the layers' packed weights, each then the place of its packed gradient
+    float2 *Rp = pack_room(part0 + batch * N * kPart0, p.v[0] + (L + 1) * batch * V, L);
+    const int64_t xu = batch * NR2, planes = batch * N, qoff = 2 * SW + L * SLAYER, rows = batch * SW;
+    const dim3 blk(256), pg = dim3(unsigned(planes)), xg(unsigned((xu + 3) / 4));
+    if (Rp) pack<true>(theta + 2 * SW, L, Rp, st);
+    hipLaunchKernelGGL(k_fnt_modes, dim3(unsigned((rows + 63) / 64), SM3 / 64, L), blk, 0, st, p.X[0], Xt, rows);
+    hipLaunchKernelGGL((k_fnt_top<N, A>), pg, blk, 0, st, gout, theta + qoff, reinterpret_cast<const A *>(p.z[L - 1]), U,
+                       part0);
     for (int l = L - 1; l >= 0; --l) {
         const int64_t lo = 2 * SW + l * SLAYER;
-        const float2 *R = reinterpret_cast<const float2 *>(theta + lo);
-        float2 *gR = reinterpret_cast<float2 *>(grad + lo);
-        hipLaunchKernelGGL((k_sur_pw_bwd<N, A>), dim3(nblk(pts)), dim3(256), 0, st, gv,
-                           reinterpret_cast<const A *>(p.z[l]), theta + lo + SR, int(l < L - 1), gvin, pts);
-        hipLaunchKernelGGL((k_sur_wgrad<N, SW, SW, A>), wg, dim3(256), 0, st, gv, reinterpret_cast<const A *>(p.v[l]),
-                           grad + lo + SR, grad + lo + SR + SW * SW);
-        launch_dft<N, float>(gv, 1.0f, gY, slices, st);
-        hipLaunchKernelGGL(k_sur_mix_grad, dim3(nblk(int64_t(SW) * SW * SM3)), dim3(256), 0, st, p.X[l], gY, gR,
-                           batch);
-        hipLaunchKernelGGL(k_sur_mix_lds<1>, dim3(SM3 / 8, unsigned((batch + 31) / 32)), dim3(256), 0, st, gY, R,
-                           gX, batch);
-        launch_idft<N, float>(gX, 1.0f / SG<N>::N3, 1, gvin, slices, st);
-        float *tmp = gv;
-        gv = gvin;
-        gvin = tmp;
+        float2 *Rl = Rp ? Rp + int64_t(l) * kPack : nullptr;
+        hipLaunchKernelGGL((k_fno_x<N, true>), xg, blk, 0, st, U, gQ, 1.0f, xu);
+        mix<true>(gQ, theta + lo, Rl, gP, batch, st);
+        hipLaunchKernelGGL((Rl ? k_fnt_mix_grad<true> : k_fnt_mix_grad<false>), dim3(125, 2), dim3(512), 0, st,
+                           Xt + l * rows * SM3, gQ, Rl ? Rl : reinterpret_cast<float2 *>(grad + lo), int(batch));
+        hipLaunchKernelGGL((k_fno_x<N, false>), xg, blk, 0, st, gP, T, 1.0f / SG<N>::N3, xu);
+        const bool top = l == L - 1;
+        auto *k = l == 0 ? (top ? k_fnt_back<N, A, true, true> : k_fnt_back<N, A, false, true>)
+                         : (top ? k_fnt_back<N, A, true, false> : k_fnt_back<N, A, false, false>);
+        hipLaunchKernelGGL(k, pg, blk, 0, st, T, g, gout, theta, theta + lo + SR, theta + qoff,
+                           reinterpret_cast<const A *>(p.z[l ? l - 1 : 0]), gz, U, part + l * planes * kPart);
     }
-    hipLaunchKernelGGL((k_sur_wgrad<N, SW, 1, float>), wg, dim3(256), 0, st, gv, g, grad, grad + SW);
+    hipLaunchKernelGGL(k_fnt_sum, dim3((SW * SW + SW + 63) / 64, unsigned((planes + 63) / 64), L + 2), blk, 0, st, part,
+                       part0, L, planes, grad);
+    if (Rp) hipLaunchKernelGGL(k_fnt_unpack, dim3(16, 8, L), blk, 0, st, Rp, SLAYER, grad + 2 * SW);
 }
 
 // Dispatch on the activation storage type.
@@ -1688,7 +2014,7 @@ int fq_sur_loss(int64_t count, const float *out, const float *target, float *gou
     if (count < 0 || !out || !target || !gout || !sums)
         return fq_internal_fail(FQ_ERR_INVALID, "fq_sur_loss: invalid arguments");
     if (count == 0) return FQ_SUCCESS;
-    hipLaunchKernelGGL(k_sur_loss, dim3(nblk(count)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), out,
+    hipLaunchKernelGGL(k_sur_loss, dim3(count > 65536 ? 256 : nblk(count)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), out,
                        target, gout, sums, count);
     return hip_status("fq_sur_loss");
 }

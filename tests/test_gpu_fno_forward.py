@@ -16,7 +16,7 @@ W, M = 32, 8
 FWD_TOL = 1e-5
 
 
-def _net(backend, N, L, seed=11):
+def _dev_net(backend, N, L, seed=11):
     from frfs_amd.surrogate import FourierSurrogate, init_params
     th = init_params(L, seed)
     off = osur.layout(W, M, L)
@@ -38,7 +38,7 @@ def _g(B, N, seed):
 @pytest.mark.parametrize('N,L,B', [(16, 2, 1), (16, 3, 15), (16, 4, 17), (32, 2, 3), (32, 3, 1), (32, 4, 2)])
 def test_layers(backend, N, L, B):
     import torch
-    net, th = _net(backend, N, L)
+    net, th = _dev_net(backend, N, L)
     g = _g(B, N, 5)
     print(f'[fno forward N={N} L={L} B={B}]', flush=True)
     out = net.predict(torch.tensor(g, device='cuda')).cpu().numpy()
@@ -51,7 +51,7 @@ def test_batch_tiles(backend, B):
     """First, last and tile-edge DOFs against the oracle; the bits of each DOF
     alone and in the batch."""
     import torch
-    net, th = _net(backend, 16, 3)
+    net, th = _dev_net(backend, 16, 3)
     g = _g(B, 16, 6)
     print(f'[fno batch B={B}]', flush=True)
     out = net.predict(torch.tensor(g, device='cuda')).cpu().numpy()
@@ -66,7 +66,7 @@ def test_batch_tiles(backend, B):
 def test_special_values(backend):
     """A DOF with a NaN or an infinity does not reach its neighbours."""
     import torch
-    net, _ = _net(backend, 16, 4)
+    net, _ = _dev_net(backend, 16, 4)
     g = _g(18, 16, 7)
     clean = net.predict(torch.tensor(g, device='cuda')).cpu().numpy()
     bad = g.copy()
