@@ -929,6 +929,216 @@ __global__ __launch_bounds__(ProdGeo<N>::THREADS, (sizeof(T) == 4 ? 4 : 2)) void
 }
 
 // ---------------------------------------------------------------------------
+// k_pack: the FP64 product stage on 24^3 for conjugate pairs.  A workgroup
+// (slot, group, G) holds the twelve planes vz = G + 2k in LDS, a wave per plane,
+// and runs every pair of the group as one packed transform (see k_prod1).  With
+// K = a + 12 b and the pair's real weights w(K) the pruned z-DFT is
+//   Z(G + 2k) = FFT_12[ w_N^{aG} (w F(a) + (-1)^G w F(a + 12)) ](k)
+// on waves 0..8, one lane per pencil; the last three bring the pair's Nyquist
+// corrections from NY to LDS and the next pair's z phases.  The z stage needs
+// LDS only for its results, so a wave that is done with a pair starts on the
+// next one's spectrum before the others are.
+// REAL: only the real part of the group sum is kept (VHS and nodal weights are
+// real and even, so no more reaches Q).
+// TWIN (nodal): pairs 2m and 2m + 1 are E_f(+-theta) and E_g(+-theta), and the sum
+// of the products E_f(theta) E_g(-theta) + E_f(-theta) E_g(theta) is taken from
+// the two; packing each product instead would load both spectra twice.
+// Bound by its own chain: a pair takes a workgroup about 9 us, alone on the chip
+// or on every CU, of which the VALU of the busiest SIMD (three waves) issues for
+// two thirds.  Two workgroups of six planes per CU (four passes over the
+// spectrum) took 2.6 times as long.  Against k_prod's six planes on six waves
+// (one pass per item for general pairs): VHS, Nrho = 8, M = 6, 500 DOFs
+// 3.28 -> 1.66 ms, VSS, Nrho = 8, M = 12 4.10 -> 2.97, bilinear 7.59 -> 4.36;
+// 99 DOFs bilinear 1.71 -> 1.03 ms.  One DOF alone takes as long as before.
+// ---------------------------------------------------------------------------
+template <int N> struct PackGeo {
+    static constexpr int S = N / 2, LPP = ProdGeo<N>::LPP, THREADS = S * LPP;
+    static constexpr int FREE = THREADS - N * N;               // lanes without a pencil in the z stage
+    static constexpr int PLANES = S * ProdGeo<N>::PLANE, NYL = N * N + 2 * S * N;
+    static_assert(LPP == 64 && THREADS <= 1024 && FREE % 64 == 0 && FREE >= N, "a wave per plane, whole waves free in the z stage");
+};
+template <int N, bool REAL, bool TWIN>
+__global__ __launch_bounds__(PackGeo<N>::THREADS) void k_pack(
+    const cpx<double> *__restrict__ FT, cpx<double> *__restrict__ P, const cpx<double> *__restrict__ ph,
+    const cpx<double> *__restrict__ tw, const DevProd *__restrict__ prods, const int *__restrict__ g_p0,
+    const int *__restrict__ g_np, const int *__restrict__ item_src, int ngroups, int nsrc,
+    const cpx<double> *__restrict__ NY, int nprods) {
+    using HG = PackGeo<N>;
+    using PG = ProdGeo<N>;
+    using G3 = Geo<N>;
+    static_assert(REAL || !TWIN, "the twin sum keeps the real part");
+    constexpr int S = HG::S, E = PG::E;
+    constexpr uint32_t PB = uint32_t(N * N * sizeof(cpx<double>));
+    __shared__ cpx<double> lds[HG::PLANES + (TWIN ? 2 : 1) * HG::NYL + 2 * N + S];
+    // XCD-contiguous order when the grid allows it: the workgroups of a DOF
+    // then share one L2 for its spectrum and corrections
+    const int64_t unit = (gridDim.x & 7) == 0 ? xcd_block() : int64_t(blockIdx.x);
+    const int G = int(unit % 2);
+    const int g = int((unit / 2) % ngroups);
+    const int slot = int(unit / (2 * int64_t(ngroups)));
+    const int tid = int(threadIdx.x);
+    const int k = __builtin_amdgcn_readfirstlane(tid / 64);
+    // lane (c, half) of the plane: a pencil on two lanes.  Lanes past the plane
+    // run on column 0 and write nothing, so that no access needs a branch
+    const int lt = tid % 64, half = lt & 1;
+    const bool act = lt < 2 * N;
+    const int vz = G + 2 * k;
+    int c = act ? lt >> 1 : 0;
+    cpx<double> *L1 = lds + k * PG::PLANE;
+    // Nyquist corrections: K piece [vy][vx], J piece [k][vx], I piece [k][vy], vz = G + 2k
+    cpx<double> *nyb = lds + HG::PLANES;
+    cpx<double> *zp = nyb + (TWIN ? 2 : 1) * HG::NYL, *twl = zp + 2 * N;     // z phases of two pairs, w_N^{aG}
+    using A = typename std::conditional<REAL, double, cpx<double>>::type;
+    A acc[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) acc[e] = A{};
+    cpx<double> ev[E], ef[E];                                  // ef: TWIN's first pair
+    const int p0 = g_p0[g], pe = p0 + g_np[g];
+    const cpx<double> *Fs = FT + int64_t(slot) * nsrc * G3::VOL;
+    int it = prods[p0].i1, src = item_src[it];
+    double cf = prods[p0].coef;
+    if (tid < N) zp[(p0 & 1) * N + tid] = ph[int64_t(it) * 3 * N + 2 * N + tid];
+    if (tid < S) twl[tid] = tw[G * S + tid];
+    __syncthreads();
+    for (int pi = p0; pi < pe; ++pi) {
+        const int pn = pi + 1 < pe ? pi + 1 : pi;              // the next pair's, loaded early
+        const int itn = prods[pn].i1, srcn = item_src[itn];
+        const double cfn = prods[pn].coef;
+        cpx<double> *nyk = nyb + (TWIN ? (pi & 1) * HG::NYL : 0);
+        if (tid < N * N) {
+            const int I = tid / N, J = tid % N;
+            const uint32_t vo = uint32_t(tid) * uint32_t(sizeof(cpx<double>));
+            const BufView sv(Fs + int64_t(src) * G3::VOL, uint32_t(N) * PB);
+            const cpx<double> *ph1 = ph + int64_t(it) * 3 * N;
+            const cpx<double> q1 = fq::cmul(ph1[I], ph1[N + J]), *z = zp + (pi & 1) * N;
+            // (1 + i) Re((1 - i) gamma) F, gamma = q1 phi_z(K); the (1 + i) is applied after the transforms
+            const double A0 = q1.x + q1.y, B0 = q1.x - q1.y, A1 = G ? -A0 : A0, B1 = G ? -B0 : B0;
+            cpx<double> u[S];
+#pragma unroll
+            for (int a = 0; a < S; ++a) {
+                const cpx<double> x0 = sv.ld<double>(vo, a * PB), x1 = sv.ld<double>(vo, (a + S) * PB);
+                const cpx<double> z0 = z[a], z1 = z[a + S];
+                const double w0 = fq::fmadd(z0.x, A0, z0.y * B0), w1 = fq::fmadd(z1.x, A1, z1.y * B1);
+                const cpx<double> t = {fq::fmadd(x1.x, w1, x0.x * w0), fq::fmadd(x1.y, w1, x0.y * w0)};
+                u[a] = a ? fq::cmul(t, twl[a]) : t;
+            }
+            fq::LFFT<S, 1>::run(u);
+            __syncthreads();                                   // the planes are free
+            cpx<double> *dd = lds + I * PG::ROW + J;
+#pragma unroll
+            for (int j = 0; j < S; ++j) dd[j * PG::PLANE] = u[j];
+        } else {
+            const nt_d2 *ny = reinterpret_cast<const nt_d2 *>(NY + (int64_t(slot) * nprods + pi) * 3 * G3::N2);
+            nt_d2 *K = reinterpret_cast<nt_d2 *>(nyk), *J = K + N * N, *I = J + S * N;
+            constexpr int FREE = HG::FREE;
+            static_assert(N * N == 3 * FREE && S * N > FREE && S * N <= 2 * FREE, "three and two rounds");
+            int i = tid - N * N;
+            asm volatile("" : "+v"(i));
+            const int j = i + FREE < S * N ? i + FREE : i;     // second round of the short pieces
+            auto at = [&](int e) { return (e % N) * N + G + 2 * (e / N); };                  // X_I [vy][vz]
+            const nt_d2 k0 = ny[i], k1 = ny[i + FREE], k2 = ny[i + 2 * FREE];
+            const nt_d2 j0 = ny[G3::N2 + (G + 2 * (i / N)) * N + i % N];
+            const nt_d2 j1 = ny[G3::N2 + (G + 2 * (j / N)) * N + j % N];
+            const nt_d2 x0 = ny[2 * G3::N2 + at(i)], x1 = ny[2 * G3::N2 + at(j)];
+            const nt_d2 ft = reinterpret_cast<const nt_d2 *>(ph)[int64_t(itn) * 3 * N + 2 * N + (i < N ? i : 0)];
+            __syncthreads();                                   // the corrections' place is free
+            K[i] = k0;
+            K[i + FREE] = k1;
+            K[i + 2 * FREE] = k2;
+            J[i] = j0;
+            I[i] = x0;
+            J[j] = j1;
+            I[j] = x1;
+            if (i < N) reinterpret_cast<nt_d2 *>(zp)[(~pi & 1) * N + i] = ft;
+        }
+        __syncthreads();
+        asm volatile("" : "+v"(c));        // keeps the LDS addresses from being hoisted out of the loop (and spilled)
+        const cpx<double> *blk = L1 + half * (E * PG::ROW) + c, *row = L1 + c * PG::ROW + half * E;
+        cpx<double> *cyc = L1 + half * PG::ROW + c;
+        // x: lane (J = c, half), I in blocks -> vx cyclic, in place
+#pragma unroll
+        for (int e = 0; e < E; ++e) ev[e] = blk[e * PG::ROW];
+        fq::fft2_dif<N, 1>(ev, half);
+        plane_sync<N>();
+        if (act) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) cyc[2 * e * PG::ROW] = ev[e];
+        }
+        plane_sync<N>();
+        // y: lane (vx = c, half), J in blocks -> vy = half + 2e
+#pragma unroll
+        for (int e = 0; e < E; ++e) ev[e] = row[e];
+        fq::fft2_dif<N, 1>(ev, half);
+#pragma unroll
+        for (int e = 0; e < E; ++e) ev[e] = {ev[e].x - ev[e].y, ev[e].x + ev[e].y};
+        // (1 + i) E = (rx, ry) + U, U the corrections' sum (see k_prod1), at vy = half + 2e
+        const double sz = (vz & 1) ? -1.0 : 1.0, sc = (c & 1) ? -1.0 : 1.0, sy = half ? -1.0 : 1.0;
+        auto corr = [&](const cpx<double> *n, int e) {
+            const cpx<double> xk = n[(half + 2 * e) * N + c], xj = n[N * N + k * N + c], xi = n[N * N + S * N + k * N + half + 2 * e];
+            return cpx<double>{fq::fmadd(sc, xi.x, fq::fmadd(sz, xk.x, sy * xj.x)),
+                               fq::fmadd(sc, xi.y, fq::fmadd(sz, xk.y, sy * xj.y))};
+        };
+        if constexpr (TWIN) {
+            if ((pi - p0) & 1) {
+                // items of a pair: (rx, uy) at theta and (ry, -ux) at -theta
+                const cpx<double> *nyf = nyb + (~pi & 1) * HG::NYL;
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    const cpx<double> u = corr(nyf, e), w = corr(nyk, e);
+                    const double rx = ef[e].x - u.x, ry = ef[e].y - u.y, gx = ev[e].x - w.x, gy = ev[e].y - w.y;
+                    const double px = fq::fmadd(rx, gy, fq::fmadd(u.y, w.x, fq::fmadd(ry, gx, u.x * w.y)));
+                    acc[e] = fq::fmadd(cf, px, acc[e]);
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < E; ++e) ef[e] = ev[e];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const cpx<double> u = corr(nyk, e);
+                const double rx = ev[e].x - u.x, ry = ev[e].y - u.y;
+                // (rx + i uy)(ry - i ux)
+                const double px = fq::fmadd(rx, ry, u.y * u.x);
+                if constexpr (REAL) acc[e] = fq::fmadd(cf, px, acc[e]);
+                else {
+                    const double py = fq::fmadd(u.y, ry, -(rx * u.x));
+                    acc[e] = {fq::fmadd(cf, px, acc[e].x), fq::fmadd(cf, py, acc[e].y)};
+                }
+            }
+        }
+        it = itn;
+        src = srcn;
+        cf = cfn;
+    }
+    cpx<double> v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        if constexpr (REAL) v[e] = {acc[e], 0.0};
+        else v[e] = acc[e];
+    }
+    // forward transforms of the group sum: row vx = c, cyclic over vy (the
+    // plane's wave alone touches its rows from here on)
+    plane_sync<N>();
+    fq::fft2_dit<N, -1>(v, half);                          // -> J' = half*E + e
+    if (act) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) L1[c * PG::ROW + half * E + e] = v[e];
+    }
+    plane_sync<N>();
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = L1[(half + 2 * e) * PG::ROW + c];
+    fq::fft2_dit<N, -1>(v, half);                          // -> I' = half*E + e
+    cpx<double> *dst = P + (int64_t(slot) * ngroups + g) * G3::VOL + int64_t(vz) * G3::N2;
+    if (act) {
+        // non-temporal: the volumes are read once, by the accumulation kernel
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            __builtin_nontemporal_store(nt_d2{v[e].x, v[e].y}, reinterpret_cast<nt_d2 *>(dst + (half * E + e) * N + c));
+    }
+}
+
+// ---------------------------------------------------------------------------
 // k_prod1: the product stage with one lane per pencil (FP32, N = 24, 32).
 // The workgroup (slot, group, G) is the same as k_prod's, with the same
 // pruned z stage, but each half-wave (32 lanes) holds one plane, one pencil
@@ -1210,7 +1420,7 @@ __global__ __launch_bounds__(Prod1Geo<N>::THREADS, 2) void k_prod1(
 
 // ---------------------------------------------------------------------------
 // k_nyq: the Nyquist-plane corrections of the pair-packed product kernels
-// (k_prod1 in FP32; the two-lane k_prod for conjugate pairs in FP64).
+// (k_prod1 in FP32; k_prod and k_pack for conjugate pairs in FP64).
 // One workgroup per (slot, product), one 32-lane group per plane piece:
 //   piece 0 (K = N/2):                 rows a = I, lanes = J   -> NY0[vy][vx]
 //   piece 1 (J = N/2, K != N/2):       rows a = I, lanes = K   -> NY1[vz][vx]
@@ -3096,6 +3306,7 @@ struct fq_handle {
     void *FJ = nullptr;          // [chunk][sources][N^2] cpx<T> spectrum slice J = N/2 for k_nyq
     void *nyv = nullptr;         // [products][2][3][N][N] cpx<T> k_nyq weights
     bool pack_conj = false;      // every product: one source, conjugate phases (zstage_conj)
+    bool twin = false;           // k_pack: the products of a nodal plan as pairs of one source each
     int *pconj = nullptr;        // general FP32 plans: per product, 1 = conjugate pair (zstage_conj)
     void *zq = nullptr;          // [products][4][3 + 2 N/4] cpx<T> zstage_conj coefficients
     cpx<float> *F32 = nullptr;   // FP32 copy of F (mixed, fused)
@@ -3152,6 +3363,25 @@ bool conj_product(const fq::Plan &P, const fq::PProd &pr) {
     bool c = P.items[pr.i1].src == P.items[pr.i2].src;
     for (int d = 0; d < 3; ++d) c = c && P.items[pr.i2].th[d] == -P.items[pr.i1].th[d];
     return c;
+}
+
+// Whether the products of every group come in twos (f+, g-), (f-, g+) of equal
+// coefficients, + and - the conjugate items of one source each (nodal plans).
+bool twin_products(const fq::Plan &P) {
+    auto conj = [&](int i, int j) {
+        bool c = P.items[i].src == P.items[j].src;
+        for (int d = 0; d < 3; ++d) c = c && P.items[j].th[d] == -P.items[i].th[d];
+        return c;
+    };
+    if (P.model != FQ_MODEL_VHS_NODAL) return false;
+    for (int g = 0; g < P.ngroups; ++g) {
+        if (P.group_np[g] % 2 || P.group_p0[g] % 2) return false;
+        for (int p = P.group_p0[g]; p < P.group_p0[g] + P.group_np[g]; p += 2) {
+            const fq::PProd &a = P.prods[p], &b = P.prods[p + 1];
+            if (a.coef != b.coef || !conj(a.i1, b.i1) || !conj(b.i2, a.i2)) return false;
+        }
+    }
+    return true;
 }
 
 // The plan's segments for k_cube (false: it has no form for this plan): runs
@@ -3245,8 +3475,9 @@ template <typename T> int upload_nyq(fq_handle *h) {
         conj = conj && c;
         anyconj = anyconj || c;
     }
+    conj = conj || h->twin;
     h->pack_conj = conj;
-    // the FP64 (two-lane) product kernel packs conjugate pairs only
+    // the FP64 product kernels pack conjugate pairs only
     if (sizeof(T) == 8 && !conj) {
         h->pack = false;
         return FQ_SUCCESS;
@@ -3282,6 +3513,18 @@ template <typename T> int upload_nyq(fq_handle *h) {
     cpx<T> *dv = nullptr;
     rc = upload(&dv, v);
     h->nyv = dv;
+    }
+    if (sizeof(T) == 8 && N == 24) {
+        // k_pack: the twiddles w_N^{aG}, G = 0, 1, a < N / 2
+        std::vector<cpx<T>> tw(N);
+        for (int a = 0; a < N; ++a) {
+            const double ang = a < H ? 0.0 : 2 * M_PI * double(a - H) / N;
+            tw[a] = {T(std::cos(ang)), T(std::sin(ang))};
+        }
+        cpx<T> *d = nullptr;
+        rc = upload(&d, tw);
+        h->zq = d;
+        return rc;
     }
     if (rc != FQ_SUCCESS || !anyconj) return rc;
     if (!conj) {
@@ -3611,7 +3854,25 @@ template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, cons
             const cpx<T> *zq = reinterpret_cast<const cpx<T> *>(h->zq);
             using KP = decltype(&k_prod<N, T, true, false>);
             KP kern = m2 ? k_prod<N, T, true, false> : k_prod<N, T, false, false>;
-            if constexpr ((N == 24 || N == 32) && sizeof(T) == 8) {
+            bool done = false;
+            if constexpr (N == 24 && sizeof(T) == 8) {
+                if (h->pack) {
+                    pre();
+                    hipLaunchKernelGGL((k_nyq<N, T, true>), dim3(unsigned(int64_t(D) * nprods)), dim3(96), 0, st, FT,
+                                       reinterpret_cast<const cpx<T> *>(sc.FJ), NY, nullptr, ph, h->prods,
+                                       h->item_src, nprods, nsrc);
+                    post(8);
+                    auto kh = h->twin ? k_pack<N, true, true>
+                                      : (P.model != FQ_MODEL_VSS ? k_pack<N, true, false> : k_pack<N, false, false>);
+                    pre();
+                    hipLaunchKernelGGL(kh, dim3(unsigned(int64_t(D) * ngroups * 2)), dim3(PackGeo<N>::THREADS), 0, st,
+                                       FT, Pg, ph, zq, h->prods, h->g_p0, h->g_np, h->item_src, ngroups, nsrc, NY,
+                                       nprods);
+                    post(7);
+                    done = true;
+                }
+            }
+            if constexpr (N == 32 && sizeof(T) == 8) {
                 if (h->pack) {
                     pre();
                     hipLaunchKernelGGL((k_nyq<N, T, true>), dim3(unsigned(int64_t(D) * nprods)), dim3(96), 0, st, FT,
@@ -3623,10 +3884,12 @@ template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, cons
                     kern = multi ? k_prod<N, T, true, true> : k_prod<N, T, false, true>;
                 }
             }
-            pre();
-            hipLaunchKernelGGL(kern, grid, dim3(ProdGeo<N>::THREADS), 0, st, FT, Pg, ph, zc, h->prods, h->g_p0,
-                               h->g_np, h->item_src, ngroups, nsrc, NY, nprods, zq);
-            post(7);
+            if (!done) {
+                pre();
+                hipLaunchKernelGGL(kern, grid, dim3(ProdGeo<N>::THREADS), 0, st, FT, Pg, ph, zc, h->prods, h->g_p0,
+                                   h->g_np, h->item_src, ngroups, nsrc, NY, nprods, zq);
+                post(7);
+            }
         }
     } else {
     u = int64_t(D) * nitems * N;
@@ -4193,6 +4456,15 @@ int fq_create(const fq_params *prm, fq_handle **out) {
     for (auto &it : P.items) isrc.push_back(it.src);
     std::vector<DevProd> dp;
     for (auto &pr : P.prods) dp.push_back({pr.i1, pr.i2, pr.coef});
+    if (h->pack && h->precision == FQ_PREC_FP64 && N == 24 && twin_products(P)) {
+        // (f+, g-), (f-, g+) -> (f+, f-), (g+, g-)
+        h->twin = true;
+        for (size_t p = 0; p + 1 < dp.size(); p += 2) {
+            const DevProd a = dp[p], b = dp[p + 1];
+            dp[p] = {a.i1, b.i1, a.coef};
+            dp[p + 1] = {b.i2, a.i2, b.coef};
+        }
+    }
     std::vector<int> cg, tc0(P.ntgt, 0), tcn(P.ntgt, 0), ls, tl0(P.ntgt, 0), tln(P.ntgt, 0);
     for (auto &c : P.contribs) { cg.push_back(c.group); tcn[c.tgt]++; }
     for (int t = 1; t < P.ntgt; ++t) tc0[t] = tc0[t - 1] + tcn[t - 1];
