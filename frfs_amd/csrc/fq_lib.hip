@@ -232,8 +232,9 @@ __global__ __launch_bounds__(256) void k_fwd_z(AosoaPtrs ptr, Dof dof, cpx<doubl
     const int64_t ds = unit / N;
     const int s = int(ds % nsrc);
     const int slot = int(ds / nsrc);
-    const int J = lt >> 1, half = lt & 1;
-    const bool act = J < N;
+    const int half = lt & 1;
+    const bool act = lt < 2 * N;
+    const int J = act ? lt >> 1 : 0;              // lanes past the row load column 0: no branch per element
     const double *f = ptr.f[s];
     const int64_t b = dof.base(slot);
     cpx<double> v[E];
@@ -241,7 +242,7 @@ __global__ __launch_bounds__(256) void k_fwd_z(AosoaPtrs ptr, Dof dof, cpx<doubl
     for (int e = 0; e < E; ++e) {
         const int K = half * E + e;
         const int64_t vv = (int64_t(I) * N + J) * N + K;
-        v[e] = {act ? f[b + vv * dof.soasz] : 0.0, 0.0};
+        v[e] = {f[b + vv * dof.soasz], 0.0};
     }
     fq::fft2_dif<N, -1>(v, half);
     cpx<double> *dst = T0 + (int64_t(slot) * nsrc + s) * G::VOL + int64_t(I) * N + J;
@@ -314,18 +315,15 @@ __global__ __launch_bounds__(kPlaneThreads) void k_fwd_xy(const cpx<double> *T0,
     const int lt = threadIdx.x % G::LPP;
     const int64_t unit = int64_t(blockIdx.x) * UPB + u;
     const bool valid = unit < nunits;
-    const int c = lt >> 1, half = lt & 1;
-    const bool act = valid && c < N;
-    const cpx<double> *src = T0 + unit * G::N2;
+    const int half = lt & 1;
+    const bool act = valid && lt < 2 * N;
+    const int c = lt < 2 * N ? lt >> 1 : 0;      // lanes past the plane load column 0: no branch per element
+    const cpx<double> *src = T0 + (valid ? unit : 0) * G::N2;
     cpx<double> v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {                // T0 is read once: non-temporal
-        cpx<double> t = {0, 0};
-        if (act) {
-            const nt_d2 x = __builtin_nontemporal_load(reinterpret_cast<const nt_d2 *>(src + (half * E + e) * N + c));
-            t = {x.x, x.y};
-        }
-        v[e] = t;
+        const nt_d2 x = __builtin_nontemporal_load(reinterpret_cast<const nt_d2 *>(src + (half * E + e) * N + c));
+        v[e] = {x.x, x.y};
     }
     fq::fft2_dif<N, -1>(v, half);                       // over I -> I' cyclic
     cpx<double> *L = lds[u];
@@ -335,7 +333,7 @@ __global__ __launch_bounds__(kPlaneThreads) void k_fwd_xy(const cpx<double> *T0,
     }
     __syncthreads();
 #pragma unroll
-    for (int e = 0; e < E; ++e) v[e] = act ? L[c * G::LDSROW + half * E + e] : cpx<double>{0, 0};
+    for (int e = 0; e < E; ++e) v[e] = L[c * G::LDSROW + half * E + e];
     fq::fft2_dif<N, -1>(v, half);                       // over J -> J' cyclic, row I' = c
     const double nn = double(G::VOL);
 #pragma unroll
@@ -1566,8 +1564,9 @@ __global__ __launch_bounds__(256, accum_waves(N, sizeof(T))) void k_accum(const 
     const int64_t ti = unit / D;
     const int t = int(ti % ntgt);
     const int I = int(ti / ntgt);
-    const int J = lt >> 1, half = lt & 1;
-    const bool act = J < N;
+    const int half = lt & 1;
+    const bool act = lt < 2 * N;
+    const int J = act ? lt >> 1 : 0;              // lanes past the row load column 0: no branch per element
     const int64_t off = int64_t(I) * N + J;
     cpx<double> H[E];
 #pragma unroll
@@ -1582,47 +1581,37 @@ __global__ __launch_bounds__(256, accum_waves(N, sizeof(T))) void k_accum(const 
             const BufView pv(P + (int64_t(slot) * ngroups + c_group[ci]) * G::VOL, uint32_t(G::VOL * sizeof(cpx<T>)));
 #pragma unroll
             for (int e = 0; e < E; ++e)
-                dst[e] = act ? pv.ld<T>(voP, uint32_t(2 * e * G::N2 * sizeof(cpx<T>))) : cpx<T>{0, 0};
+                dst[e] = pv.ld<T>(voP, uint32_t(2 * e * G::N2 * sizeof(cpx<T>)));
         } else {
             const cpx<T> *src = pbase + int64_t(c_group[ci]) * G::VOL;
 #pragma unroll
-            for (int e = 0; e < E; ++e) dst[e] = act ? src[int64_t(half + 2 * e) * G::N2] : cpx<T>{0, 0};
+            for (int e = 0; e < E; ++e) dst[e] = src[int64_t(half + 2 * e) * G::N2];
         }
     };
-    // FP32 pencils: software pipeline, the pencil of contribution ci+1 is in
-    // flight while contribution ci is transformed and accumulated.  FP64
-    // pencils are loaded in place (the register budget has no room for both).
-    constexpr bool PF = sizeof(T) == 4;
-    cpx<T> nxt[PF ? E : 1];
-    if constexpr (PF) {
-        if (cn > 0) load_pencil(c0, nxt);
-    }
+    // software pipeline: the pencil of contribution ci + 1 and the weights of ci
+    // are in flight while the pencil of ci is transformed (the scheduling
+    // barrier keeps the loads from sinking to their uses, one latency each)
+    cpx<T> nxt[E];
+    if (cn > 0) load_pencil(c0, nxt);
     for (int ci = c0; ci < c0 + cn; ++ci) {
         cpx<T> v[E];
-        if constexpr (PF) {
+        cpx<double> we[E];
 #pragma unroll
-            for (int e = 0; e < E; ++e) v[e] = nxt[e];
-            if (ci + 1 < c0 + cn) load_pencil(ci + 1, nxt);
-        } else {
-            load_pencil(ci, v);
-        }
-        fq::fft2_dit<N, -1>(v, half);             // -> K' = half*E + e
+        for (int e = 0; e < E; ++e) v[e] = nxt[e];
         if constexpr (UNI) {
             const BufView wv(W + int64_t(ci) * G::VOL, uint32_t(G::VOL * sizeof(cpx<double>)));
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const cpx<double> we =
-                    act ? wv.ld<double>(voW, uint32_t(e * G::N2 * sizeof(cpx<double>))) : cpx<double>{0, 0};
-                fq::cmac(H[e], we, cvt<double>(v[e]));
-            }
+            for (int e = 0; e < E; ++e) we[e] = wv.ld<double>(voW, uint32_t(e * G::N2 * sizeof(cpx<double>)));
         } else {
             const cpx<double> *w = W + int64_t(ci) * G::VOL + off;
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const cpx<double> we = act ? w[int64_t(half * E + e) * G::N2] : cpx<double>{0, 0};
-                fq::cmac(H[e], we, cvt<double>(v[e]));
-            }
+            for (int e = 0; e < E; ++e) we[e] = w[int64_t(half * E + e) * G::N2];
         }
+        load_pencil(ci + 1 < c0 + cn ? ci + 1 : ci, nxt);
+        __builtin_amdgcn_sched_barrier(0);
+        fq::fft2_dit<N, -1>(v, half);             // -> K' = half*E + e
+#pragma unroll
+        for (int e = 0; e < E; ++e) fq::cmac(H[e], we[e], cvt<double>(v[e]));
     }
     fq::fft2_dif<N, 1>(H, half);                  // -> vz = half + 2e
     cpx<double> *yg = Y + ((int64_t(slot) * ntgt + t) * 2 + 0) * G::VOL + off;
@@ -1640,7 +1629,7 @@ __global__ __launch_bounds__(256, accum_waves(N, sizeof(T))) void k_accum(const 
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const int64_t k = int64_t(half * E + e) * G::N2;
-            if (act) H[e] = H[e] + fq::cmul(w[k], fs[k]);
+            H[e] = H[e] + fq::cmul(w[k], fs[k]);
         }
     }
     fq::fft2_dif<N, 1>(H, half);
@@ -2365,7 +2354,7 @@ __device__ __forceinline__ void plane_inv64(const cpx<double> *src, cpx<double> 
     using G = Geo<N>;
     constexpr int E = G::E;
 #pragma unroll
-    for (int e = 0; e < E; ++e) v[e] = act ? src[(half * E + e) * N + c] : cpx<double>{0, 0};
+    for (int e = 0; e < E; ++e) v[e] = src[(half * E + e) * N + c];
     fq::fft2_dif<N, 1>(v, half);
     __syncthreads();
     if (act) {
@@ -2374,7 +2363,7 @@ __device__ __forceinline__ void plane_inv64(const cpx<double> *src, cpx<double> 
     }
     __syncthreads();
 #pragma unroll
-    for (int e = 0; e < E; ++e) v[e] = act ? L[c * G::LDSROW + half * E + e] : cpx<double>{0, 0};
+    for (int e = 0; e < E; ++e) v[e] = L[c * G::LDSROW + half * E + e];
     fq::fft2_dif<N, 1>(v, half);
 }
 
@@ -2387,14 +2376,16 @@ __global__ __launch_bounds__(kPlaneThreads, 2) void k_out(const cpx<double> *Y, 
     __shared__ cpx<double> lds[UPB][N * G::LDSROW];
     const int u = threadIdx.x / G::LPP;
     const int lt = threadIdx.x % G::LPP;
-    const int64_t unit = int64_t(blockIdx.x) * UPB + u;
+    int64_t unit = int64_t(blockIdx.x) * UPB + u;
     const bool valid = unit < nunits;
+    if (!valid) unit = 0;                          // loads a plane that is there, stores nothing
     const int vz = int(unit % N);
     const int64_t dt = unit / N;
     const int t = int(dt % ntgt);
     const int slot = int(dt / ntgt);
-    const int c = lt >> 1, half = lt & 1;
-    const bool act = valid && c < N;
+    const int half = lt & 1;
+    const bool act = valid && lt < 2 * N;
+    const int c = lt < 2 * N ? lt >> 1 : 0;        // lanes past the plane load column 0: no branch per element
     cpx<double> *L = lds[u];
     const cpx<double> *yg = Y + ((int64_t(slot) * ntgt + t) * 2 + 0) * G::VOL + int64_t(vz) * G::N2;
     // only the real parts of the gain and loss transforms are used
@@ -2405,19 +2396,18 @@ __global__ __launch_bounds__(kPlaneThreads, 2) void k_out(const cpx<double> *Y, 
 #pragma unroll
         for (int e = 0; e < E; ++e) gr[e] = gv[e].x;
     }
+    // f is loaded before the loss transform and before the first store (q may be f)
+    const double *f = ptr.f[t] + dof.base(slot);
+    const int64_t v0 = (int64_t(c) * N + half) * N + vz;
+    double fv[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) fv[e] = f[(v0 + 2 * e * N) * dof.soasz];
     cpx<double> lv[E];
     plane_inv64<N>(yg + G::VOL, L, lv, c, half, act);
     if (act) {
-        const double *f = ptr.f[t];
-        double *q = ptr.q[t];
-        const int64_t b = dof.base(slot);
+        double *q = ptr.q[t] + dof.base(slot);
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-            const int vy = half + 2 * e;
-            const int64_t vv = (int64_t(c) * N + vy) * N + vz;
-            const int64_t a = b + vv * dof.soasz;
-            q[a] = gr[e] - f[a] * lv[e].x;
-        }
+        for (int e = 0; e < E; ++e) q[(v0 + 2 * e * N) * dof.soasz] = gr[e] - fv[e] * lv[e].x;
     }
 }
 
