@@ -252,7 +252,7 @@ __global__ __launch_bounds__(256) void k_fwd_z(AosoaPtrs ptr, Dof dof, cpx<doubl
     }
 }
 
-// k_fwd_z4 (N = 32): the same for four consecutive batch slots per workgroup
+// k_fwd_z4 (N = 24, 32): the same for four consecutive batch slots per workgroup
 // (one wave each, same source and row I).  The workgroup first reads the
 // row's 1024 values of the four slots with the slots on adjacent lanes, so
 // consecutive elements of one solution point meet in one AoSoA row segment,
@@ -283,12 +283,13 @@ __global__ __launch_bounds__(256) void k_fwd_z4(AosoaPtrs ptr, Dof dof, cpx<doub
     const int u = tid / 64, lt = tid % 64;
     const int slot = sg * U + u;
     if (slot >= D) return;                           // no barrier follows
-    const int J = lt >> 1, half = lt & 1;
+    const int J = lt < 2 * N ? lt >> 1 : 0, half = lt & 1;
     cpx<double> v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = {st[J * JS + half * HS + e * U + u], 0.0};
     fq::fft2_dif<N, -1>(v, half);
     cpx<double> *dst = T0 + (int64_t(slot) * nsrc + s) * G::VOL + int64_t(I) * N + J;
+    if (lt >= 2 * N) return;
 #pragma unroll
     for (int e = 0; e < E; ++e)        // non-temporal: read once, by k_fwd_xy
         __builtin_nontemporal_store(nt_d2{v[e].x, v[e].y}, reinterpret_cast<nt_d2 *>(dst + int64_t(half + 2 * e) * G::N2));
@@ -2367,6 +2368,12 @@ __device__ __forceinline__ void plane_inv64(const cpx<double> *src, cpx<double> 
     fq::fft2_dif<N, 1>(v, half);
 }
 
+__device__ __forceinline__ double wave_sum(double x) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+    return x;
+}
+
 template <int N>
 __global__ __launch_bounds__(kPlaneThreads, 2) void k_out(const cpx<double> *Y, AosoaPtrs ptr, Dof dof, int ntgt,
                                                 int64_t nunits) {
@@ -2412,22 +2419,17 @@ __global__ __launch_bounds__(kPlaneThreads, 2) void k_out(const cpx<double> *Y, 
 }
 
 // ---------------------------------------------------------------------------
-// k_out1: the output stage of the group-pair path.  Y = Yg + i Yl with the
-// gain and loss spectra Hermitian, so DFT+_{x,y}(Y) = gain + i loss with
-// both real: one complex transform per plane, Q = Re - f Im.  A workgroup
+// k_out1: the output stage on 24^3 and 32^3.  Group pairs (PAIR): Y = Yg + i Yl
+// with the gain and loss spectra Hermitian, so DFT+_{x,y}(Y) = gain + i loss
+// with both real: one complex transform per plane, Q = Re - f Im.  Otherwise
+// gain and loss are the real parts of the transforms of two volumes.  A workgroup
 // transforms one plane of four consecutive batch slots (one wave each), stages
 // the results in LDS as [point][slot], and reads f and writes Q with the four
 // slots on adjacent lanes, so that consecutive elements of one solution point
 // meet in one AoSoA row segment.  With MOM it also writes each slot's plane
 // sums of Q {1, c, |c|^2} (FP64) to mom[slot][t][vz][5] for k_project_b.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double wave_sum(double x) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-    return x;
-}
-
-template <int N, bool MOM>
+template <int N, bool MOM, bool PAIR>
 __global__ __launch_bounds__(4 * Geo<N>::LPP, 2) void k_out1(const cpx<double> *Y, AosoaPtrs ptr, Dof dof, int ntgt,
                                                    int D, double *mom, double L) {
     using G = Geo<N>;
@@ -2442,11 +2444,20 @@ __global__ __launch_bounds__(4 * Geo<N>::LPP, 2) void k_out1(const cpx<double> *
     const int b = int(blockIdx.x);
     const int vz = b % N, t = (b / N) % ntgt, sg = b / (N * ntgt);
     const int slot = sg * U + u;
-    const int c = lt >> 1, half = lt & 1;
-    const bool act = slot < D && c < N;
+    const int half = lt & 1;
+    const bool act = slot < D && lt < 2 * N;
+    const int c = lt < 2 * N ? lt >> 1 : 0;
     cpx<double> v[E];
-    plane_inv64<N>(Y + (int64_t(slot < D ? slot : 0) * ntgt + t) * G::VOL + int64_t(vz) * G::N2, lds[u], v, c,
-                   half, act);
+    const cpx<double> *y = Y + (int64_t(slot < D ? slot : 0) * ntgt + t) * (PAIR ? 1 : 2) * G::VOL + int64_t(vz) * G::N2;
+    plane_inv64<N>(y, lds[u], v, c, half, act);
+    if constexpr (!PAIR) {
+        double gr[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) gr[e] = v[e].x;
+        plane_inv64<N>(y + G::VOL, lds[u], v, c, half, act);
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = {gr[e], v[e].x};
+    }
     // stage (gain, loss) as [point][slot], point = vx * N + vy
     __syncthreads();
     cpx<double> *st = &lds[0][0];
@@ -3268,7 +3279,7 @@ struct Scratch {
     void *FJ = nullptr;
     float *NB = nullptr;          // group pairs: Nyquist sums of Im G_g (k_prod1 -> k_nyqb)
     cpx<double> *C = nullptr;     // group pairs: Nyquist corrections (k_nyqb -> k_accum_h)
-    double *MOM = nullptr;        // group pairs with projection: per-plane sums of Q (k_out1 -> k_project_b)
+    double *MOM = nullptr;        // 24^3 and 32^3 with projection: per-plane sums of Q (k_out1 -> k_project_b)
     int64_t cap = 0;              // DOF slots the regions hold
 };
 
@@ -3763,7 +3774,7 @@ template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, cons
     int64_t u;
     u = int64_t(D) * nsrc * N;
     pre();
-    if constexpr (N == 32)
+    if constexpr (N == 24 || N == 32)
         hipLaunchKernelGGL(k_fwd_z4<N>, dim3(unsigned((D + 3) / 4 * int64_t(nsrc) * N)), bt, 0, st, ptr, dof, T0,
                            nsrc, D);
     else
@@ -3942,34 +3953,35 @@ template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, cons
     }
     post(4);
     pre();
-    bool out1 = false;
-    if constexpr (N == 32) {
-        // group pairs: gain + i loss in one volume, one transform per plane
-        if (h->hpair) {
-            const dim3 g1(unsigned((D + 3) / 4 * int64_t(ntgt) * N)), b1(4 * Geo<N>::LPP);
-            if (h->flags & FQ_FLAG_PROJECT)
-                hipLaunchKernelGGL((k_out1<N, true>), g1, b1, 0, st, Y, ptr, dof, ntgt, D, sc.MOM, P.L);
-            else
-                hipLaunchKernelGGL((k_out1<N, false>), g1, b1, 0, st, Y, ptr, dof, ntgt, D, nullptr, P.L);
-            out1 = true;
-        }
+    // the grids with a plane per wave take four slots per workgroup (whole AoSoA
+    // row segments; 24^3, 9216 DOFs: 3.40 ms a plane at a time, 2.75 now;
+    // the first stage alike 1.99 -> 0.87)
+    constexpr bool wide = N == 24 || N == 32;
+    if constexpr (wide) {
+        const dim3 g1(unsigned((D + 3) / 4 * int64_t(ntgt) * N)), b1(4 * Geo<N>::LPP);
+        const bool mom = h->flags & FQ_FLAG_PROJECT;
+        auto kout = mom ? k_out1<N, true, false> : k_out1<N, false, false>;
+        if constexpr (N == 32)
+            if (h->hpair) kout = mom ? k_out1<N, true, true> : k_out1<N, false, true>;
+        hipLaunchKernelGGL(kout, g1, b1, 0, st, Y, ptr, dof, ntgt, D, mom ? sc.MOM : nullptr, P.L);
+    } else {
+        hipLaunchKernelGGL(k_out<N>, dim3(pblocks(u)), pt, 0, st, Y, ptr, dof, ntgt, u);
     }
-    if (!out1) hipLaunchKernelGGL(k_out<N>, dim3(pblocks(u)), pt, 0, st, Y, ptr, dof, ntgt, u);
     post(5);
     if (h->flags & FQ_FLAG_PROJECT) {
         // per batch, right after k_out: the batch's Q is still in L2
         pre();
-        if (h->hpair)
-{
-            // 1024 points per workgroup, fewer until there are four workgroups per CU
-            int pc = 1024;
+        if (wide) {
+            // up to 1024 (24^3: 512) points per workgroup, fewer until there are four workgroups per CU
+            int pc = N == 24 ? 512 : 1024;
+            static_assert(!wide || G::VOL % (N == 24 ? 512 : 1024) == 0, "whole chunks");
             while (pc > 64 && (D + 31) / 32 * (G::VOL / pc) < 4 * h->cus) pc /= 2;
             hipLaunchKernelGGL(k_project_b, dim3(unsigned((D + 31) / 32 * (G::VOL / pc))), dim3(256), 0, st, ptr,
                                dof, ntgt, N, P.L, h->ginv, h->pmass, sc.MOM, int(D), pc);
+        } else {
+            hipLaunchKernelGGL(k_project, dim3(unsigned(8 * ((D + 7) / 8))), dim3(256), 0, st, ptr, dof, ntgt, N, P.L,
+                               h->ginv, h->pmass, int(D));
         }
-        else
-        hipLaunchKernelGGL(k_project, dim3(unsigned(8 * ((D + 7) / 8))), dim3(256), 0, st, ptr, dof, ntgt, N, P.L,
-                           h->ginv, h->pmass, int(D));
         post(6);
     }
     hipError_t e = hipGetLastError();
@@ -4494,7 +4506,7 @@ int fq_create(const fq_params *prm, fq_handle **out) {
     // group pairs: the Nyquist sums of Im G_g and the per-target corrections
     const size_t per_dof_NB = h->hp_nyq ? size_t(P.ngroups) * kNbPer32 * sizeof(float) : 0;
     const size_t per_dof_C = h->hp_nyq ? size_t(P.ntgt) * kCPer32 * sizeof(cpx<double>) : 0;
-    const size_t per_dof_M = h->hpair && (h->flags & FQ_FLAG_PROJECT) ? size_t(P.ntgt) * N * 5 * sizeof(double) : 0;
+    const size_t per_dof_M = !generic && (N == 24 || N == 32) && (h->flags & FQ_FLAG_PROJECT) ? size_t(P.ntgt) * N * 5 * sizeof(double) : 0;
     const size_t per_dof = per_dof_F + per_dof_Z + per_dof_P + per_dof_F32 + per_dof_NY + per_dof_FJ +
                            per_dof_NB + per_dof_C + per_dof_M;
     h->per_dof_F = per_dof_F; h->per_dof_Z = per_dof_Z; h->per_dof_P = per_dof_P;

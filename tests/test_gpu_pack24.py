@@ -68,3 +68,20 @@ def test_same_bits_in_any_batch(backend):
     for chunk in (1, 7):
         assert np.array_equal(_run_nodal(backend, vhs_cfg(N, 2, 6, 5.0, model='vhs-gll-nodal', max_chunk=chunk), f, g,
                                          2, 10), Q)
+
+
+@pytest.mark.parametrize('prec', ['double', 'mixed'])
+def test_row_groups_with_projection(backend, prec):
+    """Five DOFs (one past a group of four slots) in batches of 1, 3 and 5: the
+    same bits, and collision invariants at rounding level of sum |Q phi|."""
+    from oracle import fastspectral as fsp
+    cfg = vhs_cfg(N, 2, 6, 5.0, precision=prec, project=1)
+    cv = oracle_vhs(cfg)[0]['cv']
+    f = fsp.two_maxwellian_batch(cv, 5, seed=47)
+    print(f'[rows24 {prec}]', flush=True)
+    Q, _ = _run_vhs(backend, cfg, f, 1, 5)
+    phi = np.stack([np.ones(N ** 3), *cv, (cv ** 2).sum(0)])
+    assert (np.abs(Q @ phi.T) <= 1e-12 * (np.abs(Q) @ np.abs(phi).T)).all()
+    for chunk in (1, 3):
+        q, _ = _run_vhs(backend, vhs_cfg(N, 2, 6, 5.0, precision=prec, project=1, max_chunk=chunk), f, 1, 5)
+        assert np.array_equal(q, Q)
