@@ -684,7 +684,7 @@ __device__ __forceinline__ void conj_pencil(const cpx<T> (&x)[4][S], cpx<T> pxy,
     fq::LFFT<S, 1>::run(u);
 }
 
-template <int N, typename T, int THREADS, bool ODD>
+template <int N, typename T, int THREADS, bool ODD, bool SYNC = false>
 __device__ __forceinline__ void zstage_conj(const cpx<T> *__restrict__ src, const cpx<T> *__restrict__ zq,
                                             const cpx<T> *__restrict__ ph1, cpx<T> *dst) {
     using PG = ProdGeo<N>;
@@ -743,6 +743,7 @@ __device__ __forceinline__ void zstage_conj(const cpx<T> *__restrict__ src, cons
                 for (int a = 0; a < S; ++a) x[b][a] = sv.ld<T>(vo, uint32_t(a + S * b) * PB);
             }
             conj_pencil<S, T, ODD>(x, fq::cmul(ph1[I], ph1[N + J]), pq, am, cw, u);
+            if (SYNC && it == 0) __syncthreads();          // LDS free; the first round needs it for its results only
             cpx<T> *dd = dst + I * PG::ROW + J;
 #pragma unroll
             for (int k = 0; k < S; ++k) dd[k * PG::PLANE] = u[k];
@@ -792,7 +793,7 @@ __global__ __launch_bounds__(ProdGeo<N>::THREADS, (sizeof(T) == 4 ? 4 : 2)) void
                                                               const int *__restrict__ g_p0, const int *__restrict__ g_np,
                                                               const int *__restrict__ item_src, int ngroups, int nsrc,
                                                               const cpx<T> *__restrict__ NY, int nprods,
-                                                              const cpx<T> *__restrict__ zq) {
+                                                              const cpx<T> *__restrict__ zq, int gpw) {
     using PG = ProdGeo<N>;
     using G3 = Geo<N>;
     constexpr int E = PG::E;
@@ -804,15 +805,25 @@ __global__ __launch_bounds__(ProdGeo<N>::THREADS, (sizeof(T) == 4 ? 4 : 2)) void
     // XCD-contiguous order when the grid allows it: the 4 * ngroups
     // workgroups of a DOF then share one L2 for its spectrum and corrections
     const int64_t unit = (gridDim.x & 7) == 0 ? xcd_block() : int64_t(blockIdx.x);
+    // PACK, single products: gpw groups per workgroup, one after the other (the
+    // CU has room for one workgroup, so the loads of the next product start
+    // under the transforms of this one instead of after its end)
+    constexpr bool LOOP = PACK && !MULTI;
+    const int ng = LOOP ? (ngroups + gpw - 1) / gpw : ngroups;
     const int G = int(unit % 4);
-    const int g = int((unit / 4) % ngroups);
-    const int slot = int(unit / (4 * int64_t(ngroups)));
+    const int g0 = int((unit / 4) % ng) * (LOOP ? gpw : 1);
+    const int slot = int(unit / (4 * int64_t(ng)));
     const int k = threadIdx.x / PG::LPP;
     const int lt = threadIdx.x % PG::LPP;
-    const int c = lt >> 1, half = lt & 1;
+    int c = lt >> 1;
+    const int half = lt & 1;
     const bool act = c < N;
     const int vz = G + 4 * k;
     cpx<T> *L1 = lds + k * PG::PLANE;
+    const int g1 = LOOP ? (g0 + gpw < ngroups ? g0 + gpw : ngroups) : g0 + 1;
+#pragma unroll 1
+    for (int g = g0; g < g1; ++g) {
+    if constexpr (LOOP) asm volatile("" : "+v"(c));        // no addresses hoisted out of the loop
     cpx<T> acc[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) acc[e] = {0, 0};
@@ -825,19 +836,20 @@ __global__ __launch_bounds__(ProdGeo<N>::THREADS, (sizeof(T) == 4 ? 4 : 2)) void
         if constexpr (PACK) {
             static_assert(PG::LPP == 64, "one plane per wave");
             cpx<T> ev[E];
-            __syncthreads();                                   // LDS free
-            const cpx<T> *zqp = zq + (int64_t(pi) * 4 + G) * (3 + 2 * PG::S);
-            if (G & 1) zstage_conj<N, T, PG::THREADS, true>(src1, zqp, ph1, lds);
-            else zstage_conj<N, T, PG::THREADS, false>(src1, zqp, ph1, lds);
-            __syncthreads();
+            if constexpr (!LOOP) __syncthreads();              // LDS free (LOOP: inside the z stage)
             constexpr int KPT = (N * N + PG::THREADS - 1) / PG::THREADS;
             constexpr int SN = PG::S * N;
             static_assert(SN <= PG::THREADS, "one J and one I element per thread");
             const cpx<T> *ny = NY + (int64_t(slot) * nprods + pi) * 3 * G3::N2;
             const int tid = int(threadIdx.x);
             cpx<T> *nyk = lds + PG::S * PG::PLANE, *nyj = nyk + N * N, *nyi = nyj + SN;
+            const cpx<T> *zqp = zq + (int64_t(pi) * 4 + G) * (3 + 2 * PG::S);
+            if (G & 1) zstage_conj<N, T, PG::THREADS, true, LOOP>(src1, zqp, ph1, lds);
+            else zstage_conj<N, T, PG::THREADS, false, LOOP>(src1, zqp, ph1, lds);
             // the corrections go to their own LDS area before the x,y
             // transforms: held in registers across them they would spill
+            // (LOOP: before the barrier, free since the one in the z stage)
+            if constexpr (!LOOP) __syncthreads();
 #pragma unroll
             for (int r = 0; r < KPT; ++r) {
                 const int idx = tid + r * PG::THREADS;
@@ -848,8 +860,9 @@ __global__ __launch_bounds__(ProdGeo<N>::THREADS, (sizeof(T) == 4 ? 4 : 2)) void
                 nyj[tid] = ny[G3::N2 + z * N + w];
                 nyi[tid] = ny[2 * G3::N2 + w * N + z];
             }
+            if constexpr (LOOP) __syncthreads();
             plane_inv_lds<N, T>(L1, ev, c, half, act);        // lane (c, half): vx = c, vy = half + 2e
-            __syncthreads();
+            if constexpr (!LOOP) __syncthreads();
             const T sz = (vz & 1) ? T(-1) : T(1);
             const T sc = (c & 1) ? T(-1) : T(1);
             cpx<T> xj = act ? nyj[k * N + c] : cpx<T>{0, 0};
@@ -924,6 +937,7 @@ __global__ __launch_bounds__(ProdGeo<N>::THREADS, (sizeof(T) == 4 ? 4 : 2)) void
             else
                 dst[(half * E + e) * N + c] = acc[e];
         }
+    }
     }
 }
 
@@ -3886,9 +3900,15 @@ template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, cons
                 }
             }
             if (!done) {
+                // FP64 32^3, single-product groups: up to 16 groups per workgroup
+                // while four workgroups per CU remain (512 DOFs, 96 groups:
+                // 18.9 ms with one, 17.2 with 16; the bits are the same)
+                int gpw = N == 32 && sizeof(T) == 8 && h->pack && !multi ? 16 : 1;
+                while (gpw > 1 && int64_t(D) * 4 * ((ngroups + gpw - 1) / gpw) < 4 * h->cus) gpw /= 2;
+                const dim3 kgrid(unsigned(int64_t(D) * 4 * ((ngroups + gpw - 1) / gpw)));
                 pre();
-                hipLaunchKernelGGL(kern, grid, dim3(ProdGeo<N>::THREADS), 0, st, FT, Pg, ph, zc, h->prods, h->g_p0,
-                                   h->g_np, h->item_src, ngroups, nsrc, NY, nprods, zq);
+                hipLaunchKernelGGL(kern, kgrid, dim3(ProdGeo<N>::THREADS), 0, st, FT, Pg, ph, zc, h->prods, h->g_p0,
+                                   h->g_np, h->item_src, ngroups, nsrc, NY, nprods, zq, gpw);
                 post(7);
             }
         }
