@@ -875,7 +875,7 @@ __global__ __launch_bounds__(256) void k_sur_fuse(const float *__restrict__ th, 
 // What bounds it: the plane kernel's two streams of v (8.4 MB per DOF and
 // layer on the 32^3 grid, 1 MB on 16^3) and, nearly as long, its 30 matrix
 // instructions and 8 gelu per lane for every 16 points.  Measured for L = 4:
-// 4096 DOFs on 16^3 20.5 ms with one VALU pass over v per stage, 11.6 ms now;
+// 8192 DOFs on 16^3 20.5 ms with one VALU pass over v per stage, 11.6 ms now;
 // 700 DOFs on 32^3 10.99 -> 4.64 ms, of it the plane kernels 4.13 ms (first
 // layer 1.10, writing 2.9 GB; middle 1.60, reading and writing them; last
 // 1.43, reading), the mode product 0.16 and the x stages 0.38.  Error against
@@ -1230,7 +1230,7 @@ __global__ __launch_bounds__(256) void k_fnt_unpack(const float2 *__restrict__ g
 // theta.  ADJ: conj(R)^T in place of R, the backward product (P = gQ, Q = gP).
 // Bound by the matrix instructions of the classes with 8 modes, 32 of 32 cycles
 // per mode, wave and tile: 64 DOFs 24 us with both halves in one workgroup (125
-// of them), 14 us now; 4096 DOFs 773 -> 645.
+// of them), 14 us now; 8192 DOFs 773 -> 645.
 template <bool ADJ, bool PACKED>
 __global__ __launch_bounds__(256) void k_fno_mix(const float *__restrict__ P, const float2 *__restrict__ R,
                                                  float *__restrict__ Q, int batch) {
