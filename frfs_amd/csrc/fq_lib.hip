@@ -21,6 +21,9 @@
 // FP64 plans with one target on grids up to 20^3 run k_cube_fwd, k_cube and
 // k_cube_out instead, batches of few DOFs of the 32^3 group-pair path k_nyqt,
 // k_nyqc, k_hz and k_hsum in the place of k_nyqb and k_accum_h.
+// FP64 on 24^3 with pair packing runs k_pack as the product stage; 24^3 and 32^3
+// take four batch slots per workgroup at both ends (k_fwd_z4, k_out1) and project
+// from plane sums (k_project_b).
 // T = double (FQ_PREC_FP64) or float (FQ_PREC_MIXED).
 //
 // Lane mapping: a "unit" (one plane or one row of N pencils) is LPP = 2*NP
