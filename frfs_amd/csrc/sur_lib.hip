@@ -1015,8 +1015,7 @@ __global__ __launch_bounds__(256) void k_fno_plane(const float *__restrict__ T, 
             f32x4 d0, d1;
             if constexpr (FIRST) {
                 const float *gp = g + (plane * N + J) * N + 16 * k + 4 * q;
-                const float2 ga = reinterpret_cast<const float2 *>(gp)[0], gb = reinterpret_cast<const float2 *>(gp)[1];
-                const float gv[4] = {ga.x, ga.y, gb.x, gb.y};
+                const float gv[4] = {gp[0], gp[1], gp[2], gp[3]};       // the caller's g: no alignment beyond a float's
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     d0[i] = w0[0] * gv[i] + b0[0];

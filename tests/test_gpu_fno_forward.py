@@ -76,3 +76,17 @@ def test_special_values(backend):
     keep = [b for b in range(18) if b not in (3, 16)]
     assert np.array_equal(out[keep], clean[keep])
     assert np.isnan(out[3]).all() and not np.isfinite(out[16]).any()
+
+
+def test_unaligned_rows(backend):
+    """g and out one float past an aligned address: the same bits as aligned."""
+    import torch
+    net, _ = _dev_net(backend, 16, 3)
+    g = torch.tensor(_g(5, 16, 8), device='cuda')
+    want = net.predict(g).cpu().numpy()
+    n = g.numel()
+    gu, ou = (torch.zeros(n + 1, device='cuda')[1:].view(5, -1) for _ in range(2))
+    gu.copy_(g)
+    print('[fno unaligned]', flush=True)
+    net.forward(gu, ou)
+    assert np.array_equal(ou.cpu().numpy(), want)
