@@ -20,6 +20,7 @@
 // (R (i,o,k) complex interleaved, Wm (o,i), b), Qw, q0.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <string>
 #include <type_traits>
@@ -1068,14 +1069,14 @@ __global__ __launch_bounds__(256) void k_fno_plane(const float *__restrict__ T, 
     plane_y_out<N>(Fz, U + plane * (NR2 * SW), wave, col, q);
 }
 
-// x stages, one wave per (b, yr, zr) and 32 channels.
+// x stages, one wave per (b, yr, zr) and 32 channels, block blk of four.
 // FWD: P[b][xr][yz][c] = scale sum_I beta_xr(I) U[b][I][yz][c];
 // else T[b][I][yz][c] = scale sum_xr beta_xr(I) Q[b][xr][yz][c].
 template <int N, bool FWD>
-__global__ __launch_bounds__(256) void k_fno_x(const float *__restrict__ in, float *__restrict__ out, float scale,
-                                               int64_t units) {
+__device__ __forceinline__ void x_stage(int64_t blk, const float *__restrict__ in, float *__restrict__ out, float scale,
+                                        int64_t units) {
     const int lane = threadIdx.x & 63, col = lane & 15, q = lane >> 4;
-    const int64_t u = int64_t(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t u = blk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (u >= units) return;
     const int64_t b = u / NR2;
     const int yz = int(u % NR2);
@@ -1118,6 +1119,12 @@ __global__ __launch_bounds__(256) void k_fno_x(const float *__restrict__ in, flo
                 *reinterpret_cast<float2 *>(o + (16 * k + 4 * q + i) * NR2 * SW) = make_float2(scale * d0[i], scale * d1[i]);
         }
     }
+}
+
+template <int N, bool FWD>
+__global__ __launch_bounds__(256) void k_fno_x(const float *__restrict__ in, float *__restrict__ out, float scale,
+                                               int64_t units) {
+    x_stage<N, FWD>(blockIdx.x, in, out, scale, units);
 }
 
 // Class (q_x, q_y, q_z), q in 0..4, of the modes: class index cls = (q_x*5 + q_y)*5 + q_z.
@@ -1178,15 +1185,12 @@ __device__ __forceinline__ int stage_at(int i, int o) {
     return o / 16 * kHalf + rho * 16 + o % 16;
 }
 
-// Rp = packed R of the layers blockIdx.z (R: the first layer's, layers stride
-// complex values apart); ADJ: of conj(R)^T.  64 (i, o) x 64 modes through LDS.
+// dst = packed R of a layer (ADJ: of conj(R)^T), rows row and row + 1 of the
+// packed matrices (32 columns) of 64 modes through LDS.
 template <bool ADJ>
-__global__ __launch_bounds__(256) void k_fno_pack(const float *__restrict__ R, int64_t stride, float2 *__restrict__ Rp) {
-    __shared__ float2 tile[64][65];
-    const int t = threadIdx.x, k0 = blockIdx.y * 64;
-    const float2 *src = reinterpret_cast<const float2 *>(R + blockIdx.z * stride);
-    float2 *dst = Rp + int64_t(blockIdx.z) * kPack;
-    const int row = 2 * blockIdx.x;                          // two rows of the packed matrix, 32 columns
+__device__ __forceinline__ void pack_tile(const float2 *__restrict__ src, float2 *__restrict__ dst, int row, int k0,
+                                          float2 (*tile)[65]) {
+    const int t = threadIdx.x;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
         const int e = (t >> 6) + 4 * j, i = ADJ ? e % SW : row + e / SW, o = ADJ ? row + e / SW : e % SW;
@@ -1201,12 +1205,15 @@ __global__ __launch_bounds__(256) void k_fno_pack(const float *__restrict__ R, i
     }
 }
 
-// gR += the modes-first gradient g[k][i * 32 + o] of the layers blockIdx.z.
-__global__ __launch_bounds__(256) void k_fnt_unpack(const float2 *__restrict__ g, int64_t stride, float *__restrict__ gR) {
+__global__ __launch_bounds__(256) void k_fno_pack(const float2 *__restrict__ R, float2 *__restrict__ Rp) {
     __shared__ float2 tile[64][65];
-    const int t = threadIdx.x, k0 = blockIdx.y * 64, e0 = blockIdx.x * 64;
-    const float2 *src = g + int64_t(blockIdx.z) * kPack;
-    float2 *dst = reinterpret_cast<float2 *>(gR + blockIdx.z * stride);
+    pack_tile<false>(R, Rp, 2 * blockIdx.x, blockIdx.y * 64, tile);
+}
+
+// dst += the modes-first gradient src[k][i * 32 + o] of a layer, for 64 modes and 64 (i, o).
+__device__ __forceinline__ void unpack_tile(const float2 *__restrict__ src, float2 *__restrict__ dst, int e0, int k0,
+                                            float2 (*tile)[65]) {
+    const int t = threadIdx.x;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
         const int k = (t >> 6) + 4 * j;
@@ -1384,16 +1391,19 @@ __global__ __launch_bounds__(256) void k_fno_add(const float *__restrict__ s1, f
 //   k_fnt_top    coefficients of gz_{L-1} = Qw gout, and dQw
 //   k_fnt_back   from gz_l and T: dWm, db, gv_l, then gz_{l-1} and its U, or
 //                the lift's gradients; gz_{l-1} takes the place of gz_l
-//   k_fnt_sum    adds the planes' weight gradients
+//   k_fnt_pre    the packed weights, the transposed X, the sums over the planes of
+//                the layer above and the x stage of gQ, in one launch
+//   k_fnt_post   the x stage of T and the packed gR added to the gradient
+//   k_fnt_sum    the last sums over the planes
 // gz is [b][x][c]; z and X are the forward pass's, [b][c][x] and [b][c][k].
 // A layer reads gz_l and z_{l-1} and writes gz_{l-1}, three streams of the
 // activations (15 with a kernel per product and transform), and its matrix
 // instructions, 46 for 16 points, and 8 gelu and gelu' per lane take about as
 // long.  A plane's weight gradients stay in registers, and the sums over planes
 // are taken from one partial per plane, not with an atomic per plane and weight.
-// 64 rows on 16^3, 4 layers: forward and backward 1467 us, 732 us now; the
-// backward kernels of one layer 226 -> 74 us (k_fnt_back 33, k_fno_mix 14,
-// k_fnt_mix_grad 15, k_fno_x 12).  Error of the gradient against 64 bits 2.5e-7
+// 64 rows on 16^3, 4 layers: forward and backward 1467 us, 714 us now; the
+// backward kernels of one layer 226 -> 82 us (k_fnt_back 33, k_fno_mix 14,
+// k_fnt_mix_grad 14, k_fnt_pre 12, k_fnt_post 9).  Error of the gradient against 64 bits 2.5e-7
 // -> 1.3e-7.  The forward pass in training keeps its kernels and their rounding.
 // ---------------------------------------------------------------------------
 constexpr int kPart = SW * SW + 3 * SW;      // partials of a plane: dWm, db, dP, dp0
@@ -1619,53 +1629,88 @@ __global__ __launch_bounds__(256) void k_fnt_back(const float *__restrict__ T, c
         part[plane * kPart + j] = (Fz[j] + Fz[kPart + j]) + (Fz[2 * kPart + j] + Fz[3 * kPart + j]);
 }
 
-// grad[to + j] += sum over the planes of part[plane][j], for each of the L + 2
-// blocks blockIdx.z: the layers' dWm and db, the lift's and the projection's
-// gradients.  64 columns and 64 planes per workgroup; one launch for all.
-__global__ __launch_bounds__(256) void k_fnt_sum(const float *__restrict__ part, const float *__restrict__ part0, int L,
-                                                 int64_t planes, float *__restrict__ grad) {
-    __shared__ float red[256];
-    const int t = threadIdx.x, j = blockIdx.x * 64 + (t & 63), z = blockIdx.z;
-    const float *from = part + int64_t(z < L ? z : 0) * planes * kPart + (z == L ? SW * SW + SW : 0);
-    int stride = kPart, cols = z < L ? SW * SW + SW : 2 * SW;
-    float *to = z < L ? grad + 2 * SW + z * SLAYER + SR : grad;
-    if (z == L + 1) {
-        from = part0;
-        stride = kPart0;
-        cols = SW + 1;
-        to = grad + 2 * SW + L * SLAYER;
-    }
-    const int64_t r0 = int64_t(blockIdx.y) * 64 + (t >> 6);
-    if (int(blockIdx.x) * 64 >= cols) return;                // uniform
+// to[j] += sum over planes of from[plane][j], j < cols: 64 columns and 64 planes per workgroup.
+struct Sum { const float *from; float *to; int stride, cols; };
+__device__ __forceinline__ void sum_block(const Sum &sm, int cb, int64_t pb, int64_t planes, float *red) {
+    const int t = threadIdx.x, j = cb * 64 + (t & 63);
+    const int64_t r0 = pb * 64 + (t >> 6);
     float s = 0.f;
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
         const int64_t r = r0 + 4 * k;
-        if (j < cols && r < planes) s += from[r * stride + j];
+        if (j < sm.cols && r < planes) s += sm.from[r * sm.stride + j];
     }
     red[t] = s;
     __syncthreads();
-    if (t < 64 && j < cols) atomicAdd(&to[j], (red[t] + red[t + 64]) + (red[t + 128] + red[t + 192]));
+    if (t < 64 && j < sm.cols) atomicAdd(&sm.to[j], (red[t] + red[t + 64]) + (red[t + 128] + red[t + 192]));
 }
 
-// Xt[k][r] = X[r][k] of the layers blockIdx.z (rows r = (b, c), cols a multiple
-// of 64), 64 x 64 through LDS.
-__global__ __launch_bounds__(256) void k_fnt_modes(const float2 *__restrict__ X, float2 *__restrict__ Xt, int64_t rows) {
-    __shared__ float2 tile[64][65];
-    const int t = threadIdx.x, k0 = blockIdx.y * 64;
-    const int64_t r0 = int64_t(blockIdx.x) * 64, base = int64_t(blockIdx.z) * rows * SM3;
+// Xt[k][r] = X[r][k] (rows r = (b, c)) for 64 rows and 64 modes.
+__device__ __forceinline__ void modes_tile(const float2 *__restrict__ X, float2 *__restrict__ Xt, int64_t rows, int64_t r0,
+                                           int k0, float2 (*tile)[65]) {
+    const int t = threadIdx.x;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
         const int64_t r = r0 + (t >> 6) + 4 * j;
-        if (r < rows) tile[(t >> 6) + 4 * j][t & 63] = X[base + r * SM3 + k0 + (t & 63)];
+        tile[(t >> 6) + 4 * j][t & 63] = X[(r < rows ? r : rows - 1) * SM3 + k0 + (t & 63)];
     }
     __syncthreads();
     if (r0 + (t & 63) >= rows) return;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
         const int k = (t >> 6) + 4 * j;
-        Xt[base + (k0 + k) * rows + r0 + (t & 63)] = tile[t & 63][k];
+        Xt[(k0 + k) * rows + r0 + (t & 63)] = tile[t & 63][k];
     }
+}
+
+// The start of a layer, its parts side by side on the blocks of one launch (each
+// alone is too short to fill the chip; 64 DOFs on 16^3, 4 layers: a gradient takes
+// 714 us, and 758 with a launch for each here and in k_fnt_post):
+//   pk blocks    conj(R)^T packed into Rp (64 modes, two rows)
+//   tr blocks    Xt from X (64 modes, 64 rows)
+//   sm blocks    the sum sm over the planes, of what the kernel before left
+//   then         gQ = x stage of U
+struct Pre {
+    const float2 *R, *X;
+    float2 *Rp, *Xt;
+    int64_t rows;
+    Sum sm;
+    int64_t planes;
+    const float *U;
+    float *gQ;
+    int64_t units;
+    int pk, tr, smb;
+};
+template <int N> __global__ __launch_bounds__(256) void k_fnt_pre(Pre a) {
+    __shared__ float2 tile[64][65];
+    int64_t b = blockIdx.x;                                  // every branch is uniform
+    if (b < a.pk) return pack_tile<true>(a.R, a.Rp, 2 * int(b / 8), int(b % 8) * 64, tile);
+    b -= a.pk;
+    if (b < a.tr) return modes_tile(a.X, a.Xt, a.rows, b / 8 * 64, int(b % 8) * 64, tile);
+    b -= a.tr;
+    if (b < a.smb) {
+        const int cb = (a.sm.cols + 63) / 64;
+        return sum_block(a.sm, int(b % cb), b / cb, a.planes, &tile[0][0].x);
+    }
+    x_stage<N, true>(b - a.smb, a.U, a.gQ, 1.0f, a.units);
+}
+
+// The end of a layer's mode products: the packed gradient into the gradient (up
+// blocks), T = x stage of gP / n.
+template <int N>
+__global__ __launch_bounds__(256) void k_fnt_post(const float2 *__restrict__ g, float2 *__restrict__ gR, int up,
+                                                  const float *__restrict__ gP, float *__restrict__ T, int64_t units) {
+    __shared__ float2 tile[64][65];
+    const int b = int(blockIdx.x);
+    if (b < up) return unpack_tile(g, gR, b / 8 * 64, b % 8 * 64, tile);
+    x_stage<N, false>(b - up, gP, T, 1.0f / SG<N>::N3, units);
+}
+
+// The last sums of a pass: dWm and db of layer 0 (a) and the lift's gradients (b).
+__global__ __launch_bounds__(256) void k_fnt_sum(Sum a, Sum b, int64_t planes) {
+    __shared__ float red[256];
+    const Sum &s = blockIdx.z ? b : a;
+    if (int(blockIdx.x) * 64 < s.cols) sum_block(s, blockIdx.x, blockIdx.y, planes, red);
 }
 
 // gR(i,o,k) = sum_b conj X(b,i,k) gY(b,o,k) for the modes of class blockIdx.x,
@@ -1798,15 +1843,12 @@ ActPtrs act_ptrs(int N3, float *acts, int L, int64_t B, bool training) {
     return p;
 }
 
-// Room for n layers' packed weights between `from` and `end` (floats), 16-byte
-// aligned as the arrays before them are, or null: few DOFs (16^3: fewer than 9
-// in training, 6 in inference) leave none, and read theta in place.
-inline float2 *pack_room(float *from, float *end, int n) {
+// Room for a layer's packed weights between `from` and `end` (floats), 16-byte
+// aligned as the arrays before them are, or null: few DOFs leave none and the
+// weights are read from theta in place.
+inline float2 *pack_room(float *from, float *end) {
     float *at = from + (-(reinterpret_cast<uintptr_t>(from) / sizeof(float)) & 3);
-    return end - at >= 2LL * n * kPack ? reinterpret_cast<float2 *>(at) : nullptr;
-}
-template <bool ADJ> void pack(const float *R, int layers, float2 *Rp, hipStream_t st) {
-    hipLaunchKernelGGL(k_fno_pack<ADJ>, dim3(16, 8, layers), dim3(256), 0, st, R, SLAYER, Rp);
+    return end - at >= 2LL * kPack ? reinterpret_cast<float2 *>(at) : nullptr;
 }
 template <bool ADJ> void mix(const float *P, const float *R, const float2 *Rp, float *Q, int64_t batch, hipStream_t st) {
     hipLaunchKernelGGL((Rp ? k_fno_mix<ADJ, true> : k_fno_mix<ADJ, false>), mix_grid(batch), dim3(256), 0, st, P,
@@ -1828,7 +1870,7 @@ void forward_fused(int L, const float *theta, const float *fused, const float *g
     float *s1 = Q + pq + 2 * batch * SM3;
     static_assert(int64_t(SW) * N3 + 2 * N * NR2 * SW + 2 * NR3 * SW + 2 * SM3 + N3 <=
                   3LL * SW * N3 + 4 * SW * SM3, "fits the inference activation space");
-    float2 *Rp = pack_room(s1 + batch * N3, acts + act_floats(N3, L, batch, false), 1);
+    float2 *Rp = pack_room(s1 + batch * N3, acts + act_floats(N3, L, batch, false));
     const int64_t pts = batch * N3, xu = batch * NR2;
     const dim3 blk(256), pg(unsigned(batch * N)), xg(unsigned((xu + 3) / 4));
     // first layer from the one-channel transform of g
@@ -1840,7 +1882,8 @@ void forward_fused(int L, const float *theta, const float *fused, const float *g
     for (int l = 1; l < L - 1; ++l) {
         const float *lay = theta + 2 * SW + l * SLAYER;
         hipLaunchKernelGGL((k_fno_x<N, true>), xg, blk, 0, st, U, P, 1.0f / N3, xu);
-        if (Rp) pack<false>(lay, 1, Rp, st);
+        if (Rp)
+            hipLaunchKernelGGL(k_fno_pack, dim3(16, 8), blk, 0, st, reinterpret_cast<const float2 *>(lay), Rp);
         mix<false>(P, lay, Rp, Q, batch, st);
         hipLaunchKernelGGL((k_fno_x<N, false>), xg, blk, 0, st, Q, T, 1.0f, xu);
         hipLaunchKernelGGL((l == L - 2 ? k_fno_plane<N, A, false, true> : k_fno_plane<N, A, false, false>), pg, blk, 0,
@@ -1879,44 +1922,56 @@ void forward_impl(int L, const float *theta, const float *g, int64_t batch, bool
 }
 
 // Gradients from the activations of a training forward_impl<A>; the
-// gradients themselves (gz, the coefficient arrays) stay FP32.  work: gz, then
-// T, U, gQ and gP.  The backward pass does not read the v_l; their place takes
-// the planes' partial sums, the transposed X_l and the packed weights.
+// gradients themselves (gz, the coefficient arrays) stay FP32.  Everything is
+// kept in work, so that calls with work arrays of their own can share one acts:
+//   gz, gQ, gP; T, U; free space; the planes' partial sums of the start and of a layer.
+// From a layer's gQ to its T the T array holds nothing: the transposed X_l stands
+// there.  The packed weights, afterwards the packed gradient, take the free space
+// (16^3: from 22 DOFs on), or U and the free space once gQ is made (from 12); fewer
+// DOFs read the weights in place.  The bottom layer writes no U: its partial sums
+// take that place.
 template <int N, typename A>
 void backward_impl(int L, const float *theta, const float *g, int64_t batch, float *acts, const float *gout,
                    float *grad, float *work, hipStream_t st) {
     constexpr int64_t V = int64_t(SW) * SG<N>::N3, TP = int64_t(N) * NR2 * SW, PQ = int64_t(NR3) * SW, MD = 2LL * SW * SM3;
-    static_assert(2 * TP + 2 * PQ <= V + 2 * MD, "fits the work size");
-    static_assert(N * kPart0 <= V && MD + N * kPart <= V, "the partial sums and X fit in place of v");
-    const ActPtrs p = act_ptrs(SG<N>::N3, acts, L, batch, true);
-    float *gz = work, *T = gz + batch * V, *U = T + batch * TP, *gQ = U + batch * TP, *gP = gQ + batch * PQ;
-    float2 *Xt = reinterpret_cast<float2 *>(p.v[0]);
-    float *part = p.v[0] + L * batch * MD, *part0 = part + int64_t(L) * batch * N * kPart;
-    // the layers' packed weights, each then the place of its packed gradient
-    float2 *Rp = pack_room(part0 + batch * N * kPart0, p.v[0] + (L + 1) * batch * V, L);
+    constexpr int64_t PP = int64_t(N) * kPart, P0 = int64_t(N) * kPart0;
+    static_assert(V + 2 * PQ + 2 * TP + PP + P0 <= 2 * V + 2 * MD, "fits the work size");
+    static_assert(MD <= TP && PP <= TP, "X in place of T, the bottom layer's partial sums in place of U");
+    const ActPtrs p = act_ptrs(SG<N>::N3, acts, L, batch, true);     // read only
+    float *gz = work, *gQ = gz + batch * V, *gP = gQ + batch * PQ, *T = gP + batch * PQ, *U = T + batch * TP;
+    float *part0 = work + batch * (2 * V + 2 * MD - P0), *part = part0 - batch * PP;
+    float2 *Xt = reinterpret_cast<float2 *>(T);
+    float2 *Rp = pack_room(U + batch * TP, part);
+    const bool apart = Rp != nullptr;                                // beside U
+    if (!Rp) Rp = pack_room(U, part);
     const int64_t xu = batch * NR2, planes = batch * N, qoff = 2 * SW + L * SLAYER, rows = batch * SW;
-    const dim3 blk(256), pg = dim3(unsigned(planes)), xg(unsigned((xu + 3) / 4));
-    if (Rp) pack<true>(theta + 2 * SW, L, Rp, st);
-    hipLaunchKernelGGL(k_fnt_modes, dim3(unsigned((rows + 63) / 64), SM3 / 64, L), blk, 0, st, p.X[0], Xt, rows);
+    const int64_t xb = (xu + 3) / 4, pb = (planes + 63) / 64;
+    const dim3 blk(256), pg = dim3(unsigned(planes));
+    auto wsum = [&](const float *from, int l) { return Sum{from, grad + 2 * SW + l * SLAYER + SR, kPart, SW * SW + SW}; };
     hipLaunchKernelGGL((k_fnt_top<N, A>), pg, blk, 0, st, gout, theta + qoff, reinterpret_cast<const A *>(p.z[L - 1]), U,
                        part0);
     for (int l = L - 1; l >= 0; --l) {
         const int64_t lo = 2 * SW + l * SLAYER;
-        float2 *Rl = Rp ? Rp + int64_t(l) * kPack : nullptr;
-        hipLaunchKernelGGL((k_fno_x<N, true>), xg, blk, 0, st, U, gQ, 1.0f, xu);
-        mix<true>(gQ, theta + lo, Rl, gP, batch, st);
-        hipLaunchKernelGGL((Rl ? k_fnt_mix_grad<true> : k_fnt_mix_grad<false>), dim3(125, 2), dim3(512), 0, st,
-                           Xt + l * rows * SM3, gQ, Rl ? Rl : reinterpret_cast<float2 *>(grad + lo), int(batch));
-        hipLaunchKernelGGL((k_fno_x<N, false>), xg, blk, 0, st, gP, T, 1.0f / SG<N>::N3, xu);
+        float2 *gR = reinterpret_cast<float2 *>(grad + lo);
         const bool top = l == L - 1;
+        Pre pre{reinterpret_cast<const float2 *>(theta + lo), p.X[l], Rp, Xt, rows,
+                top ? Sum{part0, grad + qoff, kPart0, SW + 1} : wsum(part, l + 1), planes, U, gQ, xu, 0, 0, 0};
+        if (Rp && !apart) hipLaunchKernelGGL(k_fnt_pre<N>, dim3(unsigned(xb)), blk, 0, st, pre);
+        pre.pk = Rp ? 16 * 8 : 0;
+        pre.tr = int((rows + 63) / 64 * 8);
+        pre.smb = int(pb * ((pre.sm.cols + 63) / 64));
+        hipLaunchKernelGGL(k_fnt_pre<N>, dim3(unsigned(pre.pk + pre.tr + pre.smb + (Rp && !apart ? 0 : xb))), blk, 0, st, pre);
+        mix<true>(gQ, theta + lo, Rp, gP, batch, st);
+        hipLaunchKernelGGL((Rp ? k_fnt_mix_grad<true> : k_fnt_mix_grad<false>), dim3(125, 2), dim3(512), 0, st, Xt, gQ,
+                           Rp ? Rp : gR, int(batch));
+        hipLaunchKernelGGL(k_fnt_post<N>, dim3(unsigned(pre.pk + xb)), blk, 0, st, Rp, gR, pre.pk, gP, T, xu);
         auto *k = l == 0 ? (top ? k_fnt_back<N, A, true, true> : k_fnt_back<N, A, false, true>)
                          : (top ? k_fnt_back<N, A, true, false> : k_fnt_back<N, A, false, false>);
         hipLaunchKernelGGL(k, pg, blk, 0, st, T, g, gout, theta, theta + lo + SR, theta + qoff,
-                           reinterpret_cast<const A *>(p.z[l ? l - 1 : 0]), gz, U, part + l * planes * kPart);
+                           reinterpret_cast<const A *>(p.z[l ? l - 1 : 0]), gz, U, l ? part : U);
     }
-    hipLaunchKernelGGL(k_fnt_sum, dim3((SW * SW + SW + 63) / 64, unsigned((planes + 63) / 64), L + 2), blk, 0, st, part,
-                       part0, L, planes, grad);
-    if (Rp) hipLaunchKernelGGL(k_fnt_unpack, dim3(16, 8, L), blk, 0, st, Rp, SLAYER, grad + 2 * SW);
+    hipLaunchKernelGGL(k_fnt_sum, dim3((SW * SW + SW + 63) / 64, unsigned(pb), 2), blk, 0, st, wsum(U, 0),
+                       Sum{U + SW * SW + SW, grad, kPart, 2 * SW}, planes);
 }
 
 // Dispatch on the activation storage type.

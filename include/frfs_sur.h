@@ -81,8 +81,8 @@ int fq_sur_forward_fused(const fq_sur_shape *shape, const float *theta, const fl
                          int64_t batch, int32_t acts_type, float *acts, float *out, void *stream);
 
 /* grad += d(sum gout*out)/d theta, from the activations of a training
- * forward call on the same theta and g (grad is caller-zeroed; of acts only
- * what no backward call reads is overwritten, so it can be used again). */
+ * forward call on the same theta and g (grad is caller-zeroed; acts is only
+ * read, so calls with work arrays of their own can share it). */
 int fq_sur_backward(const fq_sur_shape *shape, const float *theta, const float *g, int64_t batch,
                     int32_t acts_type, float *acts, const float *gout, float *grad, float *work, void *stream);
 
