@@ -275,6 +275,8 @@ __global__ __launch_bounds__(256) void k_sur_idft16(const float2 *__restrict__ Y
 // row t into its 8 modes (A, 76 KB).  The y and x stages then work from LDS
 // as on the 16^3 grid (Bs reuses vin).  143 KB of LDS: one workgroup per CU.
 constexpr int kDft32Threads = 512;
+// four floats at a float's alignment (the caller's g has no more), one 16-byte load
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 // LDS index of the 8 modes of grid row r = I*32 + J in the 32^3 transforms:
 // rows padded to 9 and the 32 rows of one I to 296 float2 values, so that
 // both the per-row accesses (z stage) and the per-(I, pz) accesses (y stage)
@@ -298,7 +300,7 @@ __global__ __launch_bounds__(kDft32Threads) void k_sur_dft32(const TA *__restric
 #pragma unroll
             for (int w = 0; w < T * N / 4 / T; ++w) {
                 const int e4 = t + T * w;                 // float4 index in the pass
-                const float4 x = reinterpret_cast<const float4 *>(rows)[e4];
+                const f32x4_u x = reinterpret_cast<const f32x4_u *>(rows)[e4];
                 float *d = vin + (e4 >> 3) * RS + (e4 & 7) * 4;
                 d[0] = x.x; d[1] = x.y; d[2] = x.z; d[3] = x.w;
             }
