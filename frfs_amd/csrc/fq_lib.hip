@@ -3296,7 +3296,6 @@ struct Scratch {
     void *FJ = nullptr;
     float *NB = nullptr;          // group pairs: Nyquist sums of Im G_g (k_prod1 -> k_nyqb)
     cpx<double> *C = nullptr;     // group pairs: Nyquist corrections (k_nyqb -> k_accum_h)
-    double *MOM = nullptr;        // 24^3 and 32^3 with projection: per-plane sums of Q (k_out1 -> k_project_b)
     int64_t cap = 0;              // DOF slots the regions hold
 };
 
@@ -3339,7 +3338,6 @@ struct fq_handle {
     int *e_vol = nullptr, *t_e0 = nullptr, *t_en = nullptr;
     float *NB = nullptr;         // scratch [chunk][groups][kNbPer32]
     cpx<double> *Cn = nullptr;   // scratch [chunk][targets][kCPer32]
-    double *MOM = nullptr;       // scratch [chunk][targets][N][5]
     // cube kernels (FP64, one target, even N up to 20): segments of the plan
     bool cube = false;
     CubeSeg *segs = nullptr;
@@ -3363,7 +3361,7 @@ struct fq_handle {
     // per-DOF bytes of each scratch region (for carving the static array of
     // fq_eval_noalloc) and that array's device address on this handle's device
     size_t per_dof_F = 0, per_dof_Z = 0, per_dof_P = 0, per_dof_F32 = 0, per_dof_NY = 0, per_dof_FJ = 0;
-    size_t per_dof_NB = 0, per_dof_C = 0, per_dof_M = 0;
+    size_t per_dof_NB = 0, per_dof_C = 0;
     unsigned char *noalloc = nullptr;
     int cus = 256;               // compute units of the device
     // optional per-kernel HIP-event timing
@@ -3980,13 +3978,17 @@ template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, cons
     // row segments; 24^3, 9216 DOFs: 3.40 ms a plane at a time, 2.75 now;
     // the first stage alike 1.99 -> 0.87)
     constexpr bool wide = N == 24 || N == 32;
+    // the plane sums of Q, [slot][target][plane][5], for k_project_b take the
+    // place of the group volumes, which the accumulation has read
+    double *const mom_sums = static_cast<double *>(sc.Pg);
+    static_assert(!wide || 4 * N * 5 * sizeof(double) <= G::VOL * sizeof(cpx<float>), "four targets' sums in one volume");
     if constexpr (wide) {
         const dim3 g1(unsigned((D + 3) / 4 * int64_t(ntgt) * N)), b1(4 * Geo<N>::LPP);
         const bool mom = h->flags & FQ_FLAG_PROJECT;
         auto kout = mom ? k_out1<N, true, false> : k_out1<N, false, false>;
         if constexpr (N == 32)
             if (h->hpair) kout = mom ? k_out1<N, true, true> : k_out1<N, false, true>;
-        hipLaunchKernelGGL(kout, g1, b1, 0, st, Y, ptr, dof, ntgt, D, mom ? sc.MOM : nullptr, P.L);
+        hipLaunchKernelGGL(kout, g1, b1, 0, st, Y, ptr, dof, ntgt, D, mom ? mom_sums : nullptr, P.L);
     } else {
         hipLaunchKernelGGL(k_out<N>, dim3(pblocks(u)), pt, 0, st, Y, ptr, dof, ntgt, u);
     }
@@ -4000,7 +4002,7 @@ template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, cons
             static_assert(!wide || G::VOL % (N == 24 ? 512 : 1024) == 0, "whole chunks");
             while (pc > 64 && (D + 31) / 32 * (G::VOL / pc) < 4 * h->cus) pc /= 2;
             hipLaunchKernelGGL(k_project_b, dim3(unsigned((D + 31) / 32 * (G::VOL / pc))), dim3(256), 0, st, ptr,
-                               dof, ntgt, N, P.L, h->ginv, h->pmass, sc.MOM, int(D), pc);
+                               dof, ntgt, N, P.L, h->ginv, h->pmass, mom_sums, int(D), pc);
         } else {
             hipLaunchKernelGGL(k_project, dim3(unsigned(8 * ((D + 7) / 8))), dim3(256), 0, st, ptr, dof, ntgt, N, P.L,
                                h->ginv, h->pmass, int(D));
@@ -4304,7 +4306,6 @@ int eval_own(fq_handle *h, const AosoaPtrs &ptr, int32_t nupts, int64_t ldim, in
         sc[k].FJ = at(h->FJ, h->per_dof_FJ);
         sc[k].NB = static_cast<float *>(at(h->NB, h->per_dof_NB));
         sc[k].C = static_cast<cpx<double> *>(at(h->Cn, h->per_dof_C));
-        sc[k].MOM = static_cast<double *>(at(h->MOM, h->per_dof_M));
         sc[k].cap = h->chunk;
     }
     return eval_impl(h, sc, h->nsets, h->chunk, h->prof, ptr, nupts, ldim, neles, first_dof, ndof, stream);
@@ -4335,7 +4336,7 @@ size_t noalloc_bytes(const fq_handle *h, int64_t c) {
     const size_t cc = size_t(c);
     return align256(h->per_dof_F * cc) + align256(h->per_dof_Z * cc) + align256(h->per_dof_P * cc) +
            align256(h->per_dof_F32 * cc) + align256(h->per_dof_NY * cc) + align256(h->per_dof_FJ * cc) +
-           align256(h->per_dof_NB * cc) + align256(h->per_dof_C * cc) + align256(h->per_dof_M * cc);
+           align256(h->per_dof_NB * cc) + align256(h->per_dof_C * cc);
 }
 
 // Carves the regions of a batch of c DOFs out of the static scratch at base.
@@ -4357,7 +4358,6 @@ Scratch noalloc_carve(const fq_handle *h, unsigned char *base, int64_t c) {
     sc.FJ = take(h->per_dof_FJ);
     sc.NB = static_cast<float *>(take(h->per_dof_NB));
     sc.C = static_cast<cpx<double> *>(take(h->per_dof_C));
-    sc.MOM = static_cast<double *>(take(h->per_dof_M));
     sc.cap = c;
     return sc;
 }
@@ -4529,12 +4529,11 @@ int fq_create(const fq_params *prm, fq_handle **out) {
     // group pairs: the Nyquist sums of Im G_g and the per-target corrections
     const size_t per_dof_NB = h->hp_nyq ? size_t(P.ngroups) * kNbPer32 * sizeof(float) : 0;
     const size_t per_dof_C = h->hp_nyq ? size_t(P.ntgt) * kCPer32 * sizeof(cpx<double>) : 0;
-    const size_t per_dof_M = !generic && (N == 24 || N == 32) && (h->flags & FQ_FLAG_PROJECT) ? size_t(P.ntgt) * N * 5 * sizeof(double) : 0;
     const size_t per_dof = per_dof_F + per_dof_Z + per_dof_P + per_dof_F32 + per_dof_NY + per_dof_FJ +
-                           per_dof_NB + per_dof_C + per_dof_M;
+                           per_dof_NB + per_dof_C;
     h->per_dof_F = per_dof_F; h->per_dof_Z = per_dof_Z; h->per_dof_P = per_dof_P;
     h->per_dof_F32 = per_dof_F32; h->per_dof_NY = per_dof_NY; h->per_dof_FJ = per_dof_FJ;
-    h->per_dof_NB = per_dof_NB; h->per_dof_C = per_dof_C; h->per_dof_M = per_dof_M;
+    h->per_dof_NB = per_dof_NB; h->per_dof_C = per_dof_C;
     // the static scratch of fq_eval_noalloc, resolved with this device current
     h->noalloc = noalloc_resolve(h->device);
     if (rc == FQ_SUCCESS && (h->flags & FQ_FLAG_NO_SCRATCH) && !h->noalloc)
@@ -4569,7 +4568,6 @@ int fq_create(const fq_params *prm, fq_handle **out) {
             e5 = hipMalloc(&h->NB, per_dof_NB * cs);
             if (e5 == hipSuccess) e5 = hipMalloc(&h->Cn, per_dof_C * cs);
         }
-        if (e5 == hipSuccess && per_dof_M) e5 = hipMalloc(&h->MOM, per_dof_M * cs);
         if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess || e4 != hipSuccess || e5 != hipSuccess)
             rc = fail(FQ_ERR_ALLOC, "hipMalloc scratch failed (reduce max_chunk)");
         h->scratch = per_dof * cs;
@@ -4659,7 +4657,7 @@ int fq_destroy(fq_handle *h) {
                     (void *)h->t_ln, (void *)h->W, (void *)h->ginv, (void *)h->pmass, (void *)h->F, h->Z,
                     h->Pg, h->zc, (void *)h->F32, h->NY, h->FJ, (void *)h->nyv, (void *)h->zq,
                     (void *)h->pconj, (void *)h->X, (void *)h->VN, (void *)h->e_vol, (void *)h->t_e0,
-                    (void *)h->t_en, (void *)h->NB, (void *)h->Cn, (void *)h->MOM, (void *)h->segs})
+                    (void *)h->t_en, (void *)h->NB, (void *)h->Cn, (void *)h->segs})
         if (p) (void)hipFree(p);
     (void)hipThreadExchangeStreamCaptureMode(&mode);
     delete h;
