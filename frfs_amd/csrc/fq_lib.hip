@@ -2698,7 +2698,8 @@ __global__ __launch_bounds__(256) void k_project_b(AosoaPtrs ptr, Dof dof, int n
 //   k_cube_fwd  f -> F, R_loss         per (slot, source): gather, DFT-, / n; Re DFT+(Lt . F)
 //   k_cube      F -> R (real)          per (slot, segment): see below
 //   k_cube_out  R, f -> Q              Q = sum_seg R_seg - f R_loss
-// A segment is up to kSegProds products of one group, or several groups of one
+// A segment is up to kSegProds products (where the no-alloc scratch would not hold
+// a DOF, more: fq_create) of one group, or several groups of one
 // product each.  Its workgroup keeps one volume in LDS and one pencil per lane
 // in registers: per product the packed volume T_1 + i T_2 (k_prod1's pair
 // packing) is transformed along z, x and y with two LDS transposes, multiplied
@@ -3401,10 +3402,10 @@ bool twin_products(const fq::Plan &P) {
 }
 
 // The plan's segments for k_cube (false: it has no form for this plan): runs
-// of at most kSegProds products, within one group (VHS) or of as many
+// of at most `most` products, within one group (VHS) or of as many
 // single-product groups (VSS, conjugate products).  The weights are indexed by
 // group, so contribution g has to be group g.
-bool cube_segments(const fq::Plan &P, std::vector<CubeSeg> &segs, bool &conj) {
+bool cube_segments(const fq::Plan &P, int most, std::vector<CubeSeg> &segs, bool &conj) {
     conj = true;
     for (auto &pr : P.prods) conj = conj && conj_product(P, pr);
     if (int(P.contribs.size()) != P.ngroups || P.loss.size() != 1) return false;
@@ -3415,7 +3416,7 @@ bool cube_segments(const fq::Plan &P, std::vector<CubeSeg> &segs, bool &conj) {
         for (int g = 0; g < P.ngroups; ++g)
             if (P.group_np[g] != 1 || P.group_p0[g] != g) return false;
         if (!conj) return false;
-        const int ns = (P.ngroups + kSegProds - 1) / kSegProds;
+        const int ns = (P.ngroups + most - 1) / most;
         for (int i = 0; i < ns; ++i) {
             const int b = int(int64_t(P.ngroups) * i / ns), e = int(int64_t(P.ngroups) * (i + 1) / ns);
             segs.push_back({b, b, e - b});
@@ -3423,7 +3424,7 @@ bool cube_segments(const fq::Plan &P, std::vector<CubeSeg> &segs, bool &conj) {
         return true;
     }
     for (int g = 0; g < P.ngroups; ++g) {
-        const int np = P.group_np[g], ns = (np + kSegProds - 1) / kSegProds;
+        const int np = P.group_np[g], ns = (np + most - 1) / most;
         for (int i = 0; i < ns; ++i) {
             const int b = np * i / ns, e = np * (i + 1) / ns;
             segs.push_back({g, P.group_p0[g] + b, e - b});
@@ -4455,7 +4456,20 @@ int fq_create(const fq_params *prm, fq_handle **out) {
     h->cube = prm->precision == FQ_PREC_FP64 && h->P.ntgt == 1 && (!n_supported(prm->Nv) || prm->Nv == 8 || prm->Nv == 16) &&
               prm->Nv <= kCubeMaxN && !(prm->flags & (FQ_FLAG_LIBRARY_FFT | FQ_FLAG_UNFUSED | FQ_FLAG_NO_PACK));
     std::vector<CubeSeg> segs;
-    if (h->cube) h->cube = cube_segments(h->P, segs, h->pack_conj);
+    // bytes per DOF of the kernels above on the cube path, and of the product
+    // volumes (native grids) or the library path's arrays in their place
+    size_t cube_plain = 0;
+    if (h->cube) {
+        const size_t vol = size_t(prm->Nv) * prm->Nv * prm->Nv * sizeof(cpx<double>);
+        cube_plain = vol * (h->P.nsrc + std::max(h->P.nsrc, 2) + (generic ? 3 : h->P.ngroups));
+        // longer segments, fewer volumes, where fq_eval_noalloc would refuse a
+        // plan that it serves with the product volumes
+        const size_t limit = std::max(cube_plain, size_t(FQ_NOALLOC_SCRATCH_BYTES));
+        for (int most = kSegProds; h->cube; most *= 2) {
+            h->cube = cube_segments(h->P, most, segs, h->pack_conj);
+            if (generic || vol * h->P.nsrc + vol / 2 * (segs.size() + 1) <= limit) break;
+        }
+    }
     h->nseg = int(segs.size());
     h->nvol = generic ? 3 : h->P.ngroups;         // library path: the items A, B and the group G
     if (h->pack && !h->two_lane && prm->Nv == 32 && h->precision == FQ_PREC_MIXED && !(prm->flags & FQ_FLAG_NO_HPAIR)) {
