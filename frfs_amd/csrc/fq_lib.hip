@@ -4556,12 +4556,21 @@ int fq_create(const fq_params *prm, fq_handle **out) {
     // (the library path's plans share one work area: one set, one stream)
     h->nsets = (h->flags & FQ_FLAG_OVERLAP) && !(h->flags & FQ_FLAG_NO_SCRATCH) && !generic ? 2 : 1;
     const size_t ns = size_t(h->nsets);
+    // max_chunk also stands for memory: the cube kernels and the twin packing of
+    // bilinear plans may take more per DOF than the product volumes or the library
+    // path's arrays would (20^3, Nrho = 32: 2.9 times, 24^3 bilinear, M = 6: twice),
+    // and then take fewer slots instead, within the bytes that max_chunk slots
+    // (by default on grids of the library path 512) of those would hold
+    const size_t plain = h->cube ? cube_plain : (h->twin ? per_dof - per_dof_NY - per_dof_FJ : per_dof);
+    auto within = [&](int64_t slots) { return std::max<int64_t>(1, int64_t(double(slots) * (double(plain) / double(per_dof)))); };
     int64_t chunk = prm->max_chunk;
     if (chunk <= 0) {
         const size_t budget = size_t(8) << 30;    // 8 GiB default scratch budget (of 288 GB HBM)
         // the library path also holds an FFT work area of up to one Y per DOF
         chunk = std::max<int64_t>(1, int64_t(budget / ((per_dof + (generic ? per_dof_Z : 0)) * ns)));
-        chunk = std::min<int64_t>(chunk, generic && !h->cube ? 512 : 4096);
+        chunk = std::min(chunk, generic ? std::min<int64_t>(within(512), 4096) : 4096);
+    } else if (plain < per_dof) {
+        chunk = within(chunk);
     }
     h->chunk = chunk;
     if (rc == FQ_SUCCESS && (h->flags & FQ_FLAG_NO_SCRATCH)) {

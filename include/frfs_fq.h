@@ -119,7 +119,7 @@ typedef struct fq_params {
     int32_t nspcs;            /* species (1 for VHS) */
     int32_t Mpre;             /* VSS pre-integration design points */
     int32_t soasz;            /* AoSoA block size (32 in the reference) */
-    int64_t max_chunk;        /* DOFs per internal batch; 0 = library default */
+    int64_t max_chunk;        /* most DOFs per internal batch; 0 = library default */
     double L;                 /* velocity box half-width */
     double sw;                /* spherical weight: 2 pi/M (VHS) or 4 pi/M (VSS) */
     double cw;                /* velocity cell volume (2L/N)^3, for the projection */
