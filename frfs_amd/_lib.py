@@ -34,6 +34,7 @@ FLAG_OVERLAP = 128
 FLAG_LIBRARY_FFT = 256
 PATHS = ((1, 'fused'), (2, 'one_lane'), (4, 'pair_pack'), (8, 'group_pairs'), (16, 'overlap'),
          (32, 'library_fft'))
+PATH_LDS_VOLUME = 64
 NOALLOC_SCRATCH_BYTES = 256 << 20
 
 _dp = C.POINTER(C.c_double)
@@ -251,6 +252,13 @@ class Handle:
         b = C.c_int32()
         check(load().fq_get_paths(self._h, C.byref(b)))
         return [name for bit, name in PATHS if b.value & bit]
+
+    def lds_volume(self):
+        """Whether the kernels that keep a volume in LDS run in the place of
+        what paths() names (FQ_PATH_LDS_VOLUME)."""
+        b = C.c_int32()
+        check(load().fq_get_paths(self._h, C.byref(b)))
+        return bool(b.value & PATH_LDS_VOLUME)
 
     def profile(self, on=True):
         check(load().fq_profile_enable(self._h, 1 if on else 0))

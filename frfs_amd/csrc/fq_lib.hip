@@ -4657,6 +4657,7 @@ int fq_get_paths(const fq_handle *h, int32_t *paths) {
              (h->pack ? FQ_PATH_PAIR_PACK : 0) | (h->hpair ? FQ_PATH_GROUP_PAIRS : 0) |
              (h->nsets > 1 ? FQ_PATH_OVERLAP : 0);
     if (h->generic) *paths = FQ_PATH_LIBRARY_FFT;
+    if (h->cube) *paths |= FQ_PATH_LDS_VOLUME;
     return FQ_SUCCESS;
 }
 

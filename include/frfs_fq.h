@@ -218,7 +218,12 @@ int fq_eval_bilinear(fq_handle *h, const double *f, const double *g, double *q,
  * (frfs/solvers/dgfsbi/scattering.py:166-205). */
 int fq_profile_enable(fq_handle *h, int on);
 /* Wait for the recorded events; ms[k] / launches[k] = summed duration and
- * launch count of kernel k (k < FQ_NKERNELS) since the last read. */
+ * launch count of stage k (k < FQ_NKERNELS) since the last read.  A stage has
+ * the name of one kernel that serves it; another may have run: with
+ * FQ_PATH_LDS_VOLUME k_cube_fwd as k_fwd_xy, k_cube as k_prod and k_cube_out as
+ * k_out, on 24^3 and 32^3 k_pack or k_prod1 as k_prod, k_out1 as k_out and
+ * k_project_b as k_project, for few DOFs k_hz + k_hsum as k_accum, and with
+ * FQ_PATH_LIBRARY_FFT alone the library transforms with the stage they feed. */
 int fq_profile_read(fq_handle *h, double *ms, int64_t *launches);
 const char *fq_kernel_name(int k);
 /* DOFs per internal batch (kernel launch sequence). */
@@ -231,9 +236,12 @@ enum fq_path {
     FQ_PATH_PAIR_PACK = 4,    /* the two items of a product as one complex volume */
     FQ_PATH_GROUP_PAIRS = 8,  /* two groups' real parts as one product volume */
     FQ_PATH_OVERLAP = 16,     /* two scratch sets and two streams */
-    FQ_PATH_LIBRARY_FFT = 32  /* grid without a schedule of its own: hipFFT
-                                 transforms, or in FP64 with one target up to
-                                 20^3 the kernels that keep a volume in LDS */
+    FQ_PATH_LIBRARY_FFT = 32, /* grid without a schedule of its own, or
+                                 FQ_FLAG_LIBRARY_FFT: hipFFT transforms, unless
+                                 FQ_PATH_LDS_VOLUME is set as well */
+    FQ_PATH_LDS_VOLUME = 64   /* FP64, one target, up to 20^3: the kernels that
+                                 keep a volume in LDS run in the place of what
+                                 the other bits name (no library transform) */
 };
 int fq_get_paths(const fq_handle *h, int32_t *paths);
 
