@@ -46,3 +46,19 @@ def test_other_paths(backend, label, make):
     print(f'[not lds volume: {label}]', flush=True)
     lds, ran = _stages(backend, make(), False)
     assert not lds and 'k_accum' in ran and 'k_fwd_z' in ran
+
+
+@pytest.mark.parametrize('N,project', [(8, 0), (16, 1), (18, 0)])
+def test_in_place(backend, N, project):
+    """Q written over f, in several batches, has the bits of Q beside f."""
+    import numpy as np
+    from frfs_amd import _lib
+    vm, sm = _model(backend, vhs_cfg(N, 2, 6, 5.0, project=project, max_chunk=5), False)
+    assert sm._h.lds_volume()
+    fin = _inputs(backend, vm, 37, seed=72)
+    q = backend.matrix(fin.ioshape)
+    print(f'[lds volume in place N={N}]', flush=True)
+    _lib.check(_call(sm._h._h, _lib.load().fq_eval, fin, q, 37))
+    want = q.get()
+    _lib.check(_call(sm._h._h, _lib.load().fq_eval, fin, fin, 37))
+    assert np.array_equal(fin.get(), want)
