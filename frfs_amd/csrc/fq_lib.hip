@@ -4556,21 +4556,24 @@ int fq_create(const fq_params *prm, fq_handle **out) {
     // (the library path's plans share one work area: one set, one stream)
     h->nsets = (h->flags & FQ_FLAG_OVERLAP) && !(h->flags & FQ_FLAG_NO_SCRATCH) && !generic ? 2 : 1;
     const size_t ns = size_t(h->nsets);
-    // max_chunk also stands for memory: the cube kernels and the twin packing of
-    // bilinear plans may take more per DOF than the product volumes or the library
-    // path's arrays would (20^3, Nrho = 32: 2.9 times, 24^3 bilinear, M = 6: twice),
-    // and then take fewer slots instead, within the bytes that max_chunk slots
-    // (by default on grids of the library path 512) of those would hold
-    const size_t plain = h->cube ? cube_plain : (h->twin ? per_dof - per_dof_NY - per_dof_FJ : per_dof);
-    auto within = [&](int64_t slots) { return std::max<int64_t>(1, int64_t(double(slots) * (double(plain) / double(per_dof)))); };
+    const size_t budget = size_t(8) << 30;        // 8 GiB default scratch budget (of 288 GB HBM)
     int64_t chunk = prm->max_chunk;
     if (chunk <= 0) {
-        const size_t budget = size_t(8) << 30;    // 8 GiB default scratch budget (of 288 GB HBM)
         // the library path also holds an FFT work area of up to one Y per DOF
         chunk = std::max<int64_t>(1, int64_t(budget / ((per_dof + (generic ? per_dof_Z : 0)) * ns)));
-        chunk = std::min(chunk, generic ? std::min<int64_t>(within(512), 4096) : 4096);
-    } else if (plain < per_dof) {
-        chunk = within(chunk);
+        chunk = std::min<int64_t>(chunk, generic && !h->cube ? 512 : 4096);
+    } else {
+        // The cube kernels and the twin packing of bilinear plans may take more per
+        // DOF than the library path's arrays or the product volumes would (20^3,
+        // Nrho = 32: 2.9 times, 24^3 bilinear, M = 6: twice).  Beyond the default
+        // budget they take fewer slots than max_chunk instead, within the bytes of
+        // max_chunk slots of those.  (Fewer slots always: 24^3 bilinear, 300 DOFs,
+        // max_chunk = 32 3455 -> 4075 us, and by default 512 library slots' bytes:
+        // 10^3, Nrho = 10, 1440 DOFs 427 -> 518 us.)
+        const size_t plain = h->cube ? cube_plain : (h->twin ? per_dof - per_dof_NY - per_dof_FJ : per_dof);
+        const int64_t fit = int64_t(budget / (per_dof * ns));
+        if (plain < per_dof && chunk > fit)
+            chunk = std::max({int64_t(1), fit, int64_t(double(chunk) * (double(plain) / double(per_dof)))});
     }
     h->chunk = chunk;
     if (rc == FQ_SUCCESS && (h->flags & FQ_FLAG_NO_SCRATCH)) {

@@ -1,13 +1,12 @@
 """Scratch of the FP64 plans whose kernels take more per DOF than the product
 volumes (or the library path's arrays) would: for the same max_chunk they hold
-no more bytes, with the same results; plans that fq_eval_noalloc serves with the
-product volumes are served; the projection's plane sums take no scratch of
-their own."""
+no more bytes, or no more than the default budget; plans that fq_eval_noalloc
+serves with the product volumes are served; the projection's plane sums take no
+scratch of their own."""
 import numpy as np
 import pytest
 
-from tests.cases import oracle_vhs, vhs_cfg, vss_cfg
-from tests.test_gpu_parity import _io, _run_vhs
+from tests.cases import vhs_cfg
 from tests.test_zz_no_alloc import _call, _inputs, _model
 
 pytestmark = pytest.mark.gpu
@@ -19,19 +18,25 @@ def _vhs_model(backend, **kw):
     return _model(backend, vhs_cfg(**kw), False)[1]
 
 
-def test_cube_within_the_library_paths_bytes(backend):
-    """20^3: the spectrum, gain and loss, and three work volumes per slot."""
-    from oracle import fastspectral as fsp
+BUDGET = 8 << 30                           # the default scratch
+
+
+@pytest.mark.parametrize('Nrho,max_chunk', [(32, 8192), (60, 12000)])
+def test_cube_within_the_library_paths_bytes(backend, Nrho, max_chunk):
+    """20^3: the spectrum, gain and loss, and three work volumes per slot, or the
+    default budget where that is more."""
     slot = 6 * VOL * 20 ** 3
-    f = fsp.two_maxwellian_batch(oracle_vhs(vhs_cfg(20, 16, 6, 5.0))[0]['cv'], 9, seed=3)
-    print('[scratch cube]', flush=True)
-    Q, sm = _run_vhs(backend, vhs_cfg(20, 16, 6, 5.0), f, 1, 9)
-    assert sm._h.scratch_bytes() <= 512 * slot
-    q, sm = _run_vhs(backend, vhs_cfg(20, 16, 6, 5.0, max_chunk=8), f, 1, 9)
-    assert sm._h.scratch_bytes() <= 8 * slot and 1 <= sm._h.chunk_dofs() < 8
-    assert np.array_equal(q, Q)
-    _, sm = _run_vhs(backend, vhs_cfg(20, 2, 6, 5.0, max_chunk=8), f, 1, 9)
-    assert sm._h.chunk_dofs() == 8
+    sm = _vhs_model(backend, Nv=20, Nrho=Nrho, M=6, max_chunk=max_chunk)
+    print('[scratch cube]', sm._h.scratch_bytes(), sm._h.chunk_dofs(), flush=True)
+    assert sm._h.lds_volume() and sm._h.chunk_dofs() < max_chunk
+    assert 0.99 * max(BUDGET, max_chunk * slot) <= sm._h.scratch_bytes() <= max(BUDGET, max_chunk * slot)
+
+
+def test_cube_takes_max_chunk_within_the_budget(backend):
+    for kw in (dict(Nrho=32, max_chunk=100), dict(Nrho=2, max_chunk=8192)):
+        sm = _vhs_model(backend, Nv=20, M=6, **kw)
+        assert sm._h.chunk_dofs() == kw['max_chunk']
+    assert _vhs_model(backend, Nv=20, Nrho=32, M=6)._h.scratch_bytes() <= BUDGET
 
 
 def test_twin_packing_within_the_unpacked_bytes(backend):
@@ -39,10 +44,10 @@ def test_twin_packing_within_the_unpacked_bytes(backend):
     from frfs_amd.velocitymesh import DGFSVelocityMesh
     got = {}
     for pack in (1, 0):
-        cfg = vhs_cfg(24, 4, 16, 5.0, model='vhs-gll-nodal', max_chunk=40, pack=pack)
+        cfg = vhs_cfg(24, 4, 16, 5.0, model='vhs-gll-nodal', max_chunk=6000, pack=pack)
         got[pack] = DGFSVHSGLLNodalScatteringModel(backend, cfg, DGFSVelocityMesh(backend, cfg))._h.scratch_bytes()
     print('[scratch twin]', got, flush=True)
-    assert got[1] <= got[0]
+    assert BUDGET < got[1] <= got[0]
 
 
 @pytest.mark.parametrize('N,prec', [(24, 'double'), (24, 'mixed'), (32, 'double'), (32, 'mixed')])
