@@ -221,12 +221,13 @@ __global__ void k_tables(cpx<double> *tabs, const DevTerm *terms, const int *tbe
 }
 
 // ---------------------------------------------------------------------------
-// k_fwd_z: AoSoA gather + DFT- along z.  unit = (slot, src, I).
+// k_fwd_z (N = 8, 16): AoSoA gather + DFT- along z.  unit = (slot, src, I).
 // ---------------------------------------------------------------------------
 template <int N>
 __global__ __launch_bounds__(256) void k_fwd_z(AosoaPtrs ptr, Dof dof, cpx<double> *T0, int nsrc,
                                                int64_t nunits) {
     using G = Geo<N>;
+    static_assert(G::LPP == 2 * N, "every lane of a unit has a column");
     constexpr int E = G::E;
     const int lt = threadIdx.x % G::LPP;
     const int64_t unit = int64_t(blockIdx.x) * (blockDim.x / G::LPP) + threadIdx.x / G::LPP;
@@ -235,9 +236,7 @@ __global__ __launch_bounds__(256) void k_fwd_z(AosoaPtrs ptr, Dof dof, cpx<doubl
     const int64_t ds = unit / N;
     const int s = int(ds % nsrc);
     const int slot = int(ds / nsrc);
-    const int half = lt & 1;
-    const bool act = lt < 2 * N;
-    const int J = act ? lt >> 1 : 0;              // lanes past the row load column 0: no branch per element
+    const int J = lt >> 1, half = lt & 1;
     const double *f = ptr.f[s];
     const int64_t b = dof.base(slot);
     cpx<double> v[E];
@@ -249,18 +248,16 @@ __global__ __launch_bounds__(256) void k_fwd_z(AosoaPtrs ptr, Dof dof, cpx<doubl
     }
     fq::fft2_dif<N, -1>(v, half);
     cpx<double> *dst = T0 + (int64_t(slot) * nsrc + s) * G::VOL + int64_t(I) * N + J;
-    if (act) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) dst[int64_t(half + 2 * e) * G::N2] = v[e];
-    }
+    for (int e = 0; e < E; ++e) dst[int64_t(half + 2 * e) * G::N2] = v[e];
 }
 
 // k_fwd_z4 (N = 24, 32): the same for four consecutive batch slots per workgroup
 // (one wave each, same source and row I).  The workgroup first reads the
-// row's 1024 values of the four slots with the slots on adjacent lanes, so
+// row's N^2 values of the four slots with the slots on adjacent lanes, so
 // consecutive elements of one solution point meet in one AoSoA row segment,
-// and stages them in LDS as [J][half][e][slot] (half-rows of 65 and rows of
-// 130 doubles: lanes J and J + 16 share a bank pair, no other conflicts).
+// and stages them in LDS as [J][half][e][slot] (half-rows of 2 N + 1 and rows of
+// 4 N + 2 doubles, which spreads the lanes' columns over the banks).
 template <int N>
 __global__ __launch_bounds__(256) void k_fwd_z4(AosoaPtrs ptr, Dof dof, cpx<double> *T0, int nsrc, int D) {
     using G = Geo<N>;
@@ -960,12 +957,14 @@ __global__ __launch_bounds__(ProdGeo<N>::THREADS, (sizeof(T) == 4 ? 4 : 2)) void
 // of the products E_f(theta) E_g(-theta) + E_f(-theta) E_g(theta) is taken from
 // the two; packing each product instead would load both spectra twice.
 // Bound by its own chain: a pair takes a workgroup about 9 us, alone on the chip
-// or on every CU, of which the VALU of the busiest SIMD (three waves) issues for
-// two thirds.  Two workgroups of six planes per CU (four passes over the
-// spectrum) took 2.6 times as long.  Against k_prod's six planes on six waves
+// or on every CU (99 DOFs, bilinear, Nrho = 8: 6.2 rounds of one workgroup per CU,
+// VALU 36% of the cycles, LDS 25%, 61% of the waves' time in waits).  Two
+// workgroups of six planes per CU (four passes over the spectrum) took 2.6 times
+// as long.  Against k_prod's six planes on six waves
 // (one pass per item for general pairs): VHS, Nrho = 8, M = 6, 500 DOFs
 // 3.28 -> 1.66 ms, VSS, Nrho = 8, M = 12 4.10 -> 2.97, bilinear 7.59 -> 4.36;
-// 99 DOFs bilinear 1.71 -> 1.03 ms.  One DOF alone takes as long as before.
+// 99 DOFs bilinear 1.71 -> 1.03 ms.  A bilinear call of one to three DOFs takes
+// 1.5% longer (163.5 against 161 us; k_nyq is a launch of its own).
 // ---------------------------------------------------------------------------
 template <int N> struct PackGeo {
     static constexpr int S = N / 2, LPP = ProdGeo<N>::LPP, THREADS = S * LPP;
@@ -2716,10 +2715,12 @@ __global__ __launch_bounds__(256) void k_project_b(AosoaPtrs ptr, Dof dof, int n
 // Every sum runs in an order the plan fixes, so a DOF gets the same bits in any
 // batch.  Measured against the k_prod path (16^3, M = 6, Nrho = 8): 134 -> 77 us
 // for 64 DOFs, 12.5 -> 7.1 ms for 8192 with the projection; against the library
-// path (20^3, Nrho = 10, 153 DOFs): 13.4 ms -> 420 us.  k_cube issues FP64 VALU
-// in 45% of the cycles and keeps the LDS busy in 32%; its barriers and the one
-// wave with the Nyquist planes, at two waves per SIMD (LDS, registers), are the
-// rest.
+// path (20^3, Nrho = 10, 153 DOFs, of which that path transformed 512 slots):
+// 13.4 ms -> 420 us.  k_cube issues FP64 VALU in 47% of the cycles and keeps the
+// LDS busy in 34%; its barriers and the one wave with the Nyquist planes, at two
+// waves per SIMD (LDS, registers), are the rest.
+// kSegProds was chosen at M = 6; with 16, 24 and 60 products per group (two to
+// eight segments) 1 to 512 DOFs on 16^3 are 1.4 to 3.1 times as fast as k_prod.
 // ---------------------------------------------------------------------------
 constexpr int kCubeMaxN = 20;
 constexpr int kSegProds = 8;
@@ -3754,7 +3755,9 @@ int build_hpair(fq_handle *h) {
 // 255 us (M = 12, Nrho = 16) until they pass one per CU; the two kernels take
 // 56 us at one pair, 148 us at 128, and more than k_nyqb beyond 256.  k_accum_h
 // takes 160-211 us up to 60 pairs; k_hz + k_hsum 41 us at one, 74 us at 8,
-// 168 us at 16 and 252 us at 24 (their spectra then pass through HBM).
+// 168 us at 16 and 252 us at 24 (their spectra then pass through HBM).  The serial
+// length goes with Nrho on both sides: at Nrho = 2 and 6, and with two species, no
+// call of 1 to 300 DOFs is slower than with the one-kernel forms alone.
 constexpr int64_t kNyqFew = 256, kSumFew = 16;
 
 template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, const AosoaPtrs &ptr, const Dof &dof,
@@ -3904,7 +3907,7 @@ template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, cons
             if (!done) {
                 // FP64 32^3, single-product groups: up to 16 groups per workgroup
                 // while four workgroups per CU remain (512 DOFs, 96 groups:
-                // 18.9 ms with one, 17.2 with 16; the bits are the same)
+                // 18.8 ms with one, 17.3 with 16; the bits are the same)
                 int gpw = N == 32 && sizeof(T) == 8 && h->pack && !multi ? 16 : 1;
                 while (gpw > 1 && int64_t(D) * 4 * ((ngroups + gpw - 1) / gpw) < 4 * h->cus) gpw /= 2;
                 const dim3 kgrid(unsigned(int64_t(D) * 4 * ((ngroups + gpw - 1) / gpw)));

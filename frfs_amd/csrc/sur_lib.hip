@@ -876,13 +876,14 @@ __global__ __launch_bounds__(256) void k_sur_fuse(const float *__restrict__ th, 
 // [b][x][channel], so a lane's operands are contiguous.
 //
 // What bounds it: the plane kernel's two streams of v (8.4 MB per DOF and
-// layer on the 32^3 grid, 1 MB on 16^3) and, nearly as long, its 30 matrix
-// instructions and 8 gelu per lane for every 16 points.  Measured for L = 4:
-// 8192 DOFs on 16^3 20.5 ms with one VALU pass over v per stage, 11.6 ms now;
-// 700 DOFs on 32^3 10.99 -> 4.64 ms, of it the plane kernels 4.13 ms (first
-// layer 1.10, writing 2.9 GB; middle 1.60, reading and writing them; last
-// 1.43, reading), the mode product 0.16 and the x stages 0.38.  Error against
-// 64 bits 2.4e-7 -> 1.4e-7.
+// layer on the 32^3 grid, 1 MB on 16^3; the texture data units are busy in 92-98%
+// of the cycles) and, nearly as long, its 30 matrix instructions (34-52% of the
+// cycles) and 8 gelu per lane for every 16 points.  Measured for L = 4: 8192 DOFs
+// on 16^3 20.2 ms with one VALU pass over v per stage, 10.9 ms now; 700 DOFs on
+// 32^3 10.97 -> 4.51 ms, of it the plane kernels 4.00 ms (first layer 1.06,
+// writing 2.9 GB; middle 1.57, reading and writing them; last 1.36, reading), the
+// mode product 0.12 and the x stages 0.39.  Error against 64 bits 2.4e-7 ->
+// 1.8e-7 (other inputs: 1.4e-7 -> 5.3e-8).
 // Channels of a column tile t: o = 2 * (lane % 16) + t, so that the two tiles
 // of a lane are neighbours (8-byte accesses).
 // ---------------------------------------------------------------------------
@@ -1405,8 +1406,9 @@ __global__ __launch_bounds__(256) void k_fno_add(const float *__restrict__ s1, f
 // are taken from one partial per plane, not with an atomic per plane and weight.
 // 64 rows on 16^3, 4 layers: forward and backward 1467 us, 714 us now; the
 // backward kernels of one layer 226 -> 82 us (k_fnt_back 33, k_fno_mix 14,
-// k_fnt_mix_grad 14, k_fnt_pre 12, k_fnt_post 9).  Error of the gradient against 64 bits 2.5e-7
-// -> 1.3e-7.  The forward pass in training keeps its kernels and their rounding.
+// k_fnt_mix_grad 14, k_fnt_pre 12, k_fnt_post 9).  Error of the gradient against
+// 64 bits 1.7e-7..5.4e-7 -> 3.5e-8..1.3e-7 over inputs and orders of the sums.  The
+// forward pass in training keeps its kernels and their rounding.
 // ---------------------------------------------------------------------------
 constexpr int kPart = SW * SW + 3 * SW;      // partials of a plane: dWm, db, dP, dp0
 constexpr int kPart0 = 2 * SW;               // and of the start: dQw, dq0 (the rest unused)
