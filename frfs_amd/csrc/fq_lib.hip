@@ -2390,9 +2390,9 @@ __device__ __forceinline__ double wave_sum(double x) {
     return x;
 }
 
-// k_out (N = 8, 16).  f is read where it is used (1024 DOFs on 16^3: 64.7 us, and
-// 75.0 loaded ahead of the loss transform, though both leave three waves per SIMD).
-template <int N>
+// k_out (N = 8, 16).  AHEAD: f is loaded ahead of the loss transform, for batches
+// of few DOFs (launch rule in run_chunk); otherwise where it is used.
+template <int N, bool AHEAD>
 __global__ __launch_bounds__(kPlaneThreads, 2) void k_out(const cpx<double> *Y, AosoaPtrs ptr, Dof dof, int ntgt,
                                                 int64_t nunits) {
     using G = Geo<N>;
@@ -2420,16 +2420,21 @@ __global__ __launch_bounds__(kPlaneThreads, 2) void k_out(const cpx<double> *Y, 
 #pragma unroll
         for (int e = 0; e < E; ++e) gr[e] = gv[e].x;
     }
+    const double *f = ptr.f[t] + dof.base(slot);
+    const int64_t v0 = (int64_t(c) * N + half) * N + vz;
+    double fv[E];
+    if constexpr (AHEAD) {                         // before the first store too (q may be f)
+#pragma unroll
+        for (int e = 0; e < E; ++e) fv[e] = f[(v0 + 2 * e * N) * dof.soasz];
+    }
     cpx<double> lv[E];
     plane_inv64<N>(yg + G::VOL, L, lv, c, half, act);
     if (act) {
-        const double *f = ptr.f[t];
-        double *q = ptr.q[t];
-        const int64_t b = dof.base(slot);
+        double *q = ptr.q[t] + dof.base(slot);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const int64_t a = b + ((int64_t(c) * N + half + 2 * e) * N + vz) * dof.soasz;
-            q[a] = gr[e] - f[a] * lv[e].x;
+            const int64_t a = (v0 + 2 * e * N) * dof.soasz;
+            q[a] = gr[e] - (AHEAD ? fv[e] : f[a]) * lv[e].x;
         }
     }
 }
@@ -3994,7 +3999,11 @@ template <int N, typename T> int run_chunk(fq_handle *h, const Scratch &sc, cons
             if (h->hpair) kout = mom ? k_out1<N, true, true> : k_out1<N, false, true>;
         hipLaunchKernelGGL(kout, g1, b1, 0, st, Y, ptr, dof, ntgt, D, mom ? mom_sums : nullptr, P.L);
     } else {
-        hipLaunchKernelGGL(k_out<N>, dim3(pblocks(u)), pt, 0, st, Y, ptr, dof, ntgt, u);
+        // f ahead of the loss transform while at most eight workgroups per CU hide
+        // its latency (a call on 16^3, mixed, Nrho = 2: 9 DOFs 47.6 -> 47.1 us, 512
+        // DOFs 204 -> 202); with sixteen it only holds registers (1024 DOFs 421 -> 434)
+        auto kout = int64_t(pblocks(u)) <= 8 * int64_t(h->cus) ? k_out<N, true> : k_out<N, false>;
+        hipLaunchKernelGGL(kout, dim3(pblocks(u)), pt, 0, st, Y, ptr, dof, ntgt, u);
     }
     post(5);
     if (h->flags & FQ_FLAG_PROJECT) {
