@@ -1213,25 +1213,6 @@ __global__ __launch_bounds__(256) void k_fno_pack(const float2 *__restrict__ R, 
     pack_tile<false>(R, Rp, 2 * blockIdx.x, blockIdx.y * 64, tile);
 }
 
-// dst += the modes-first gradient src[k][i * 32 + o] of a layer, for 64 modes and 64 (i, o).
-__device__ __forceinline__ void unpack_tile(const float2 *__restrict__ src, float2 *__restrict__ dst, int e0, int k0,
-                                            float2 (*tile)[65]) {
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const int k = (t >> 6) + 4 * j;
-        tile[k][t & 63] = src[int64_t(k0 + k) * (SW * SW) + e0 + (t & 63)];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const int e = (t >> 6) + 4 * j;
-        const int64_t at = int64_t(e0 + e) * SM3 + k0 + (t & 63);
-        const float2 r = tile[t & 63][e], w = dst[at];
-        dst[at] = make_float2(w.x + r.x, w.y + r.y);
-    }
-}
-
 // Q = fold(X R) for the modes of class blockIdx.x, the output channels o = 16
 // blockIdx.z + col and 64 DOFs at a time (blockIdx.y, then by gridDim.y), sixteen
 // per wave.  The class's weights (up to 8 modes, 32 KB) are staged in LDS, from
@@ -1394,9 +1375,8 @@ __global__ __launch_bounds__(256) void k_fno_add(const float *__restrict__ s1, f
 //   k_fnt_top    coefficients of gz_{L-1} = Qw gout, and dQw
 //   k_fnt_back   from gz_l and T: dWm, db, gv_l, then gz_{l-1} and its U, or
 //                the lift's gradients; gz_{l-1} takes the place of gz_l
-//   k_fnt_pre    the packed weights, the transposed X, the sums over the planes of
-//                the layer above and the x stage of gQ, in one launch
-//   k_fnt_post   the x stage of T and the packed gR added to the gradient
+//   k_fnt_pre    the packed weights, the sums over the planes of the layer above
+//                and the x stage of gQ, in one launch
 //   k_fnt_sum    the last sums over the planes
 // gz is [b][x][c]; z and X are the forward pass's, [b][c][x] and [b][c][k].
 // A layer reads gz_l and z_{l-1} and writes gz_{l-1}, three streams of the
@@ -1404,9 +1384,9 @@ __global__ __launch_bounds__(256) void k_fno_add(const float *__restrict__ s1, f
 // instructions, 46 for 16 points, and 8 gelu and gelu' per lane take about as
 // long.  A plane's weight gradients stay in registers, and the sums over planes
 // are taken from one partial per plane, not with an atomic per plane and weight.
-// 64 rows on 16^3, 4 layers: forward and backward 1467 us, 714 us now; the
-// backward kernels of one layer 226 -> 82 us (k_fnt_back 33, k_fno_mix 14,
-// k_fnt_mix_grad 14, k_fnt_pre 12, k_fnt_post 9).  Error of the gradient against
+// 64 rows on 16^3, 4 layers: forward and backward 1467 us, 720 us now; the
+// backward kernels of one layer 226 -> 84 us (k_fnt_back 33, k_fnt_mix_grad 21,
+// k_fno_mix 14, k_fnt_pre 10, k_fno_x 6).  Error of the gradient against
 // 64 bits 1.7e-7..5.4e-7 -> 3.5e-8..1.3e-7 over inputs and orders of the sums.  The
 // forward pass in training keeps its kernels and their rounding.
 // ---------------------------------------------------------------------------
@@ -1649,65 +1629,31 @@ __device__ __forceinline__ void sum_block(const Sum &sm, int cb, int64_t pb, int
     if (t < 64 && j < sm.cols) atomicAdd(&sm.to[j], (red[t] + red[t + 64]) + (red[t + 128] + red[t + 192]));
 }
 
-// Xt[k][r] = X[r][k] (rows r = (b, c)) for 64 rows and 64 modes.
-__device__ __forceinline__ void modes_tile(const float2 *__restrict__ X, float2 *__restrict__ Xt, int64_t rows, int64_t r0,
-                                           int k0, float2 (*tile)[65]) {
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const int64_t r = r0 + (t >> 6) + 4 * j;
-        tile[(t >> 6) + 4 * j][t & 63] = X[(r < rows ? r : rows - 1) * SM3 + k0 + (t & 63)];
-    }
-    __syncthreads();
-    if (r0 + (t & 63) >= rows) return;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const int k = (t >> 6) + 4 * j;
-        Xt[(k0 + k) * rows + r0 + (t & 63)] = tile[t & 63][k];
-    }
-}
-
 // The start of a layer, its parts side by side on the blocks of one launch (each
-// alone is too short to fill the chip; 64 DOFs on 16^3, 4 layers: a gradient takes
-// 714 us, and 758 with a launch for each here and in k_fnt_post):
+// alone is too short to fill the chip):
 //   pk blocks    conj(R)^T packed into Rp (64 modes, two rows)
-//   tr blocks    Xt from X (64 modes, 64 rows)
 //   sm blocks    the sum sm over the planes, of what the kernel before left
 //   then         gQ = x stage of U
 struct Pre {
-    const float2 *R, *X;
-    float2 *Rp, *Xt;
-    int64_t rows;
+    const float2 *R;
+    float2 *Rp;
     Sum sm;
     int64_t planes;
     const float *U;
     float *gQ;
     int64_t units;
-    int pk, tr, smb;
+    int pk, smb;
 };
 template <int N> __global__ __launch_bounds__(256) void k_fnt_pre(Pre a) {
     __shared__ float2 tile[64][65];
     int64_t b = blockIdx.x;                                  // every branch is uniform
     if (b < a.pk) return pack_tile<true>(a.R, a.Rp, 2 * int(b / 8), int(b % 8) * 64, tile);
     b -= a.pk;
-    if (b < a.tr) return modes_tile(a.X, a.Xt, a.rows, b / 8 * 64, int(b % 8) * 64, tile);
-    b -= a.tr;
     if (b < a.smb) {
         const int cb = (a.sm.cols + 63) / 64;
         return sum_block(a.sm, int(b % cb), b / cb, a.planes, &tile[0][0].x);
     }
     x_stage<N, true>(b - a.smb, a.U, a.gQ, 1.0f, a.units);
-}
-
-// The end of a layer's mode products: the packed gradient into the gradient (up
-// blocks), T = x stage of gP / n.
-template <int N>
-__global__ __launch_bounds__(256) void k_fnt_post(const float2 *__restrict__ g, float2 *__restrict__ gR, int up,
-                                                  const float *__restrict__ gP, float *__restrict__ T, int64_t units) {
-    __shared__ float2 tile[64][65];
-    const int b = int(blockIdx.x);
-    if (b < up) return unpack_tile(g, gR, b / 8 * 64, b % 8 * 64, tile);
-    x_stage<N, false>(b - up, gP, T, 1.0f / SG<N>::N3, units);
 }
 
 // The last sums of a pass: dWm and db of layer 0 (a) and the lift's gradients (b).
@@ -1717,17 +1663,31 @@ __global__ __launch_bounds__(256) void k_fnt_sum(Sum a, Sum b, int64_t planes) {
     if (int(blockIdx.x) * 64 < s.cols) sum_block(s, blockIdx.x, blockIdx.y, planes, red);
 }
 
-// gR(i,o,k) = sum_b conj X(b,i,k) gY(b,o,k) for the modes of class blockIdx.x,
-// one mode per wave, and the input channels i = 16 blockIdx.y + col, from Xt[k][b][i] and the coefficients gQ of gz.  The DOFs
-// are the inner dimension of the product.  Stored modes first (PACKED:
-// gR[k][i * 32 + o]), or added into the gradient.
-template <bool PACKED>
-__global__ __launch_bounds__(512) void k_fnt_mix_grad(const float2 *__restrict__ Xt, const float *__restrict__ gQ,
+// gR(i,o,k) += sum_b conj X(b,i,k) gY(b,o,k), gY from the coefficients gQ of gz.
+// A workgroup takes the eight modes (px, py) = blockIdx.x, a wave each, and the
+// input channels i = 16 blockIdx.y + col; the DOFs are the inner dimension of the
+// product.  The eight modes are 64 contiguous bytes of X and of the gradient, both
+// taken through LDS.  Bound by latency (128 workgroups, a batch of loads per 16
+// DOFs): 64 DOFs on 16^3 21 us; 22 with X read by each wave for itself, 37 with
+// the output channels on two workgroups besides.  A class of modes per workgroup
+// took 14, but 12 more to transpose X and to bring the result into place, in
+// arrays that few DOFs have no room for.
+__global__ __launch_bounds__(512) void k_fnt_mix_grad(const float2 *__restrict__ X, const float *__restrict__ gQ,
                                                       float2 *__restrict__ gR, int batch) {
-    const int cls = blockIdx.x, lane = threadIdx.x & 63, col = lane & 15, q = lane >> 4;
+    __shared__ float2 buf[16 * SW][SM + 1];                  // [i * 32 + o][pz]
+    __shared__ float2 xs[16][16][SM + 1];                    // X of 16 DOFs [b][i][pz]
+    const int lane = threadIdx.x & 63, col = lane & 15, q = lane >> 4;
+    const int pz = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // the mode's class and signs (cls_mode's inverse)
+    const int pd[3] = {int(blockIdx.x) / SM, int(blockIdx.x) % SM, pz};
+    int cls = 0;
     float sg[3];
-    const int k = cls_mode(cls, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), sg);
-    if (k < 0) return;                                       // no barrier in this kernel
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const bool neg = pd[d] >= SM / 2;
+        cls = cls * 5 + (neg ? SM - pd[d] : pd[d]);
+        sg[d] = pd[d] == 0 ? 0.f : (neg ? -1.f : 1.f);
+    }
     int at[8];
     float has[8];                                            // 0 where the class has no such coefficient
 #pragma unroll
@@ -1736,51 +1696,71 @@ __global__ __launch_bounds__(512) void k_fnt_mix_grad(const float2 *__restrict__
         at[e] = (c < 0 ? 0 : c) * SW + 2 * col;
         has[e] = c < 0 ? 0.f : 1.f;
     }
-    const float2 *xk = Xt + int64_t(k) * batch * SW + 16 * blockIdx.y + col;
+    // X of 16 DOFs at a time through LDS, eight lanes on a channel's eight modes:
+    // element threadIdx.x + 512 j is DOF (threadIdx.x / 128) + 4 j
+    const int xi = int(threadIdx.x) / SM % 16, xp = int(threadIdx.x) % SM, xb = int(threadIdx.x) / (16 * SM);
+    const float2 *xk = X + (16 * blockIdx.y + xi) * SM3 + blockIdx.x * SM + xp;
+    float2 nx[4];
+    auto load = [&](int b0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int b = b0 + xb + 4 * j;
+            nx[j] = xk[int64_t(b < batch ? b : batch - 1) * (SW * SM3)];
+        }
+    };
     f32x4 re[2][2], im[2][2];                                // [o parity][term]
 #pragma unroll
     for (int t = 0; t < 4; ++t) re[t >> 1][t & 1] = im[t >> 1][t & 1] = {0, 0, 0, 0};
-#pragma unroll 4
-    for (int b0 = 0; b0 < batch; b0 += 4) {
-        const int b = b0 + q, bl = b < batch ? b : batch - 1;
-        const bool live = b < batch;
-        float py[2][8];
-        float2 X = xk[int64_t(bl) * SW];
+    load(0);
+#pragma unroll 1
+    for (int s0 = 0; s0 < batch; s0 += 16) {
+        __syncthreads();                                         // xs is free
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float2 y = *reinterpret_cast<const float2 *>(gQ + int64_t(bl) * (NR3 * SW) + at[e]);
-            py[0][e] = has[e] != 0.f ? y.x : 0.f;
-            py[1][e] = has[e] != 0.f ? y.y : 0.f;
-        }
-        float2 Y[2] = {cls_x(py[0], sg), cls_x(py[1], sg)};
-        if (!live) X = Y[0] = Y[1] = make_float2(0.f, 0.f);
+        for (int j = 0; j < 4; ++j) xs[xb + 4 * j][xi][xp] = nx[j];
+        __syncthreads();
+        load(s0 + 16);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            re[u][0] = mfma4(X.x, Y[u].x, re[u][0]);
-            re[u][1] = mfma4(X.y, Y[u].y, re[u][1]);
-            im[u][0] = mfma4(X.x, Y[u].y, im[u][0]);
-            im[u][1] = mfma4(-X.y, Y[u].x, im[u][1]);
+        for (int it = 0; it < 4; ++it) {
+            const int b = s0 + 4 * it + q, bl = b < batch ? b : batch - 1;
+            const bool live = b < batch;
+            float py[2][8];
+            float2 x = xs[4 * it + q][col][pz];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float2 y = *reinterpret_cast<const float2 *>(gQ + int64_t(bl) * (NR3 * SW) + at[e]);
+                py[0][e] = has[e] != 0.f ? y.x : 0.f;
+                py[1][e] = has[e] != 0.f ? y.y : 0.f;
+            }
+            float2 Y[2] = {cls_x(py[0], sg), cls_x(py[1], sg)};
+            if (!live) x = Y[0] = Y[1] = make_float2(0.f, 0.f);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                re[u][0] = mfma4(x.x, Y[u].x, re[u][0]);
+                re[u][1] = mfma4(x.y, Y[u].y, re[u][1]);
+                im[u][0] = mfma4(x.x, Y[u].y, im[u][0]);
+                im[u][1] = mfma4(-x.y, Y[u].x, im[u][1]);
+            }
         }
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int i = 16 * blockIdx.y + 4 * q + r;
-        float w[4];
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            w[2 * u] = re[u][0][r] + re[u][1][r];
-            w[2 * u + 1] = im[u][0][r] + im[u][1][r];
-        }
-        if constexpr (PACKED) {
-            *reinterpret_cast<f32x4 *>(gR + int64_t(k) * (SW * SW) + i * SW + 2 * col) = f32x4{w[0], w[1], w[2], w[3]};
-        } else {
+        for (int u = 0; u < 2; ++u)
+            buf[(4 * q + r) * SW + 2 * col + u][pz] = make_float2(re[u][0][r] + re[u][1][r], im[u][0][r] + im[u][1][r]);
+    __syncthreads();
+    constexpr int E = 16 * SW * SM / 512;
+    float2 *g = gR + int64_t(16 * blockIdx.y) * SW * SM3 + blockIdx.x * SM;
+    float2 old[E];
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                float2 *p = gR + int64_t(i * SW + 2 * col + u) * SM3 + k;
-                const float2 old = *p;
-                *p = make_float2(old.x + w[2 * u], old.y + w[2 * u + 1]);
-            }
-        }
+    for (int j = 0; j < E; ++j) {
+        const int e = threadIdx.x + 512 * j;
+        old[j] = g[int64_t(e / SM) * SM3 + e % SM];
+    }
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        const int e = threadIdx.x + 512 * j;
+        const float2 w = buf[e / SM][e % SM];
+        g[int64_t(e / SM) * SM3 + e % SM] = make_float2(old[j].x + w.x, old[j].y + w.y);
     }
 }
 
@@ -1928,27 +1908,22 @@ void forward_impl(int L, const float *theta, const float *g, int64_t batch, bool
 // Gradients from the activations of a training forward_impl<A>; the
 // gradients themselves (gz, the coefficient arrays) stay FP32.  Everything is
 // kept in work, so that calls with work arrays of their own can share one acts:
-//   gz, gQ, gP; T, U; free space; the planes' partial sums of the start and of a layer.
-// From a layer's gQ to its T the T array holds nothing: the transposed X_l stands
-// there.  The packed weights, afterwards the packed gradient, take the free space
-// (16^3: from 22 DOFs on), or U and the free space once gQ is made (from 12); fewer
-// DOFs read the weights in place.  The bottom layer writes no U: its partial sums
-// take that place.
+//   gz, gQ, gP, U, T; free space; the planes' partial sums of a layer and of the start.
+// From a layer's gQ to its T the T array holds nothing: the packed weights stand
+// there and in the free space behind it (16^3: from 12 DOFs on; fewer read the
+// weights in place).  The bottom layer writes no U: its partial sums take that place.
 template <int N, typename A>
 void backward_impl(int L, const float *theta, const float *g, int64_t batch, float *acts, const float *gout,
                    float *grad, float *work, hipStream_t st) {
     constexpr int64_t V = int64_t(SW) * SG<N>::N3, TP = int64_t(N) * NR2 * SW, PQ = int64_t(NR3) * SW, MD = 2LL * SW * SM3;
     constexpr int64_t PP = int64_t(N) * kPart, P0 = int64_t(N) * kPart0;
     static_assert(V + 2 * PQ + 2 * TP + PP + P0 <= 2 * V + 2 * MD, "fits the work size");
-    static_assert(MD <= TP && PP <= TP, "X in place of T, the bottom layer's partial sums in place of U");
+    static_assert(PP <= TP, "the bottom layer's partial sums in place of U");
     const ActPtrs p = act_ptrs(SG<N>::N3, acts, L, batch, true);     // read only
-    float *gz = work, *gQ = gz + batch * V, *gP = gQ + batch * PQ, *T = gP + batch * PQ, *U = T + batch * TP;
+    float *gz = work, *gQ = gz + batch * V, *gP = gQ + batch * PQ, *U = gP + batch * PQ, *T = U + batch * TP;
     float *part0 = work + batch * (2 * V + 2 * MD - P0), *part = part0 - batch * PP;
-    float2 *Xt = reinterpret_cast<float2 *>(T);
-    float2 *Rp = pack_room(U + batch * TP, part);
-    const bool apart = Rp != nullptr;                                // beside U
-    if (!Rp) Rp = pack_room(U, part);
-    const int64_t xu = batch * NR2, planes = batch * N, qoff = 2 * SW + L * SLAYER, rows = batch * SW;
+    float2 *Rp = pack_room(T, part);
+    const int64_t xu = batch * NR2, planes = batch * N, qoff = 2 * SW + L * SLAYER;
     const int64_t xb = (xu + 3) / 4, pb = (planes + 63) / 64;
     const dim3 blk(256), pg = dim3(unsigned(planes));
     auto wsum = [&](const float *from, int l) { return Sum{from, grad + 2 * SW + l * SLAYER + SR, kPart, SW * SW + SW}; };
@@ -1956,19 +1931,15 @@ void backward_impl(int L, const float *theta, const float *g, int64_t batch, flo
                        part0);
     for (int l = L - 1; l >= 0; --l) {
         const int64_t lo = 2 * SW + l * SLAYER;
-        float2 *gR = reinterpret_cast<float2 *>(grad + lo);
         const bool top = l == L - 1;
-        Pre pre{reinterpret_cast<const float2 *>(theta + lo), p.X[l], Rp, Xt, rows,
-                top ? Sum{part0, grad + qoff, kPart0, SW + 1} : wsum(part, l + 1), planes, U, gQ, xu, 0, 0, 0};
-        if (Rp && !apart) hipLaunchKernelGGL(k_fnt_pre<N>, dim3(unsigned(xb)), blk, 0, st, pre);
-        pre.pk = Rp ? 16 * 8 : 0;
-        pre.tr = int((rows + 63) / 64 * 8);
+        Pre pre{reinterpret_cast<const float2 *>(theta + lo), Rp, top ? Sum{part0, grad + qoff, kPart0, SW + 1} : wsum(part, l + 1),
+                planes, U, gQ, xu, Rp ? 16 * 8 : 0, 0};
         pre.smb = int(pb * ((pre.sm.cols + 63) / 64));
-        hipLaunchKernelGGL(k_fnt_pre<N>, dim3(unsigned(pre.pk + pre.tr + pre.smb + (Rp && !apart ? 0 : xb))), blk, 0, st, pre);
+        hipLaunchKernelGGL(k_fnt_pre<N>, dim3(unsigned(pre.pk + pre.smb + xb)), blk, 0, st, pre);
         mix<true>(gQ, theta + lo, Rp, gP, batch, st);
-        hipLaunchKernelGGL((Rp ? k_fnt_mix_grad<true> : k_fnt_mix_grad<false>), dim3(125, 2), dim3(512), 0, st, Xt, gQ,
-                           Rp ? Rp : gR, int(batch));
-        hipLaunchKernelGGL(k_fnt_post<N>, dim3(unsigned(pre.pk + xb)), blk, 0, st, Rp, gR, pre.pk, gP, T, xu);
+        hipLaunchKernelGGL(k_fnt_mix_grad, dim3(SM * SM, 2), dim3(512), 0, st, p.X[l], gQ,
+                           reinterpret_cast<float2 *>(grad + lo), int(batch));
+        hipLaunchKernelGGL((k_fno_x<N, false>), dim3(unsigned(xb)), blk, 0, st, gP, T, 1.0f / SG<N>::N3, xu);
         auto *k = l == 0 ? (top ? k_fnt_back<N, A, true, true> : k_fnt_back<N, A, false, true>)
                          : (top ? k_fnt_back<N, A, true, false> : k_fnt_back<N, A, false, false>);
         hipLaunchKernelGGL(k, pg, blk, 0, st, T, g, gout, theta, theta + lo + SR, theta + qoff,
