@@ -4468,8 +4468,8 @@ int fq_create(const fq_params *prm, fq_handle **out) {
     h->cube = prm->precision == FQ_PREC_FP64 && h->P.ntgt == 1 && (!n_supported(prm->Nv) || prm->Nv == 8 || prm->Nv == 16) &&
               prm->Nv <= kCubeMaxN && !(prm->flags & (FQ_FLAG_LIBRARY_FFT | FQ_FLAG_UNFUSED | FQ_FLAG_NO_PACK));
     std::vector<CubeSeg> segs;
-    // bytes per DOF of the kernels above on the cube path, and of the product
-    // volumes (native grids) or the library path's arrays in their place
+    // bytes per DOF of what the cube kernels replace: the product volumes (native
+    // grids) or the library path's arrays, with the spectra before and after them
     size_t cube_plain = 0;
     if (h->cube) {
         const size_t vol = size_t(prm->Nv) * prm->Nv * prm->Nv * sizeof(cpx<double>);
