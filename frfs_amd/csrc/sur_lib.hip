@@ -967,12 +967,12 @@ template <int N> __device__ __forceinline__ void plane_y_out(const float *Fz, fl
 // One plane I of DOF b per workgroup; FIRST: v_1 from g (lw: the folded first
 // layer's A, a0), else v_{l+1} from v_l in place (lw: the layer's Wm, b).
 // LAST: v_{L-1} is not stored; its part of the projection, QW . v + qb, goes
-// to out (qw: QW, qb) and its modes to U.
+// to out (qw: QW, qb) and its modes to U.  out may be g: a wave reads its 16 points
+// of g before it writes them.
 template <int N, typename TA, bool FIRST, bool LAST>
-__global__ __launch_bounds__(256) void k_fno_plane(const float *__restrict__ T, const float *__restrict__ g,
+__global__ __launch_bounds__(256) void k_fno_plane(const float *__restrict__ T, const float *g,
                                                    const float *__restrict__ lw, TA *__restrict__ v,
-                                                   float *__restrict__ U, const float *__restrict__ qw,
-                                                   float *__restrict__ out) {
+                                                   float *__restrict__ U, const float *__restrict__ qw, float *out) {
     constexpr int KT = N / 16;                               // 16-point tiles of a row, 16-row tiles of the plane
     __shared__ float Fz[N * NR * SW];                        // [J][zr][c]: the row's z coefficients, in then out
     const int tid = threadIdx.x, lane = tid & 63;
